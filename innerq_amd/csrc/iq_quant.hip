@@ -1,249 +1,15 @@
-// Quantize-on-append and dense dequantization kernels (gfx950).
+// A decode step's window append, dense dequantization and unpacking (gfx950).
 //
-// Quantization restates src/innerq/quant.py op by op: every fp16 op of the
-// reference (sub, division by the int level count, division by the scale) is
-// an fp32 op rounded to fp16 with round-to-nearest-even (exact for + - * /
-// because fp32 has more than 2*11+2 significand bits), the clamp keeps NaN,
-// the rounding is half-to-even (v_rndne_f32), and NaN becomes INT32_MIN in the
-// dense int32 output (0 in the packed field).  Division is IEEE (hipcc's
-// default correctly rounded fp32 divide; no fast-math anywhere in this build).
-//
-// One thread owns one quantization group: the group's min/max (or max |x|)
-// is a serial loop over G registers, which keeps the rounding order trivially
-// identical to the reference and needs no cross-lane traffic.  Appends are a
-// few hundred groups per decode step and prefill is a streaming pass, so this
-// kernel is latency- resp. HBM-bound either way.
+// The append quantizes a few hundred groups per step with the reference's own
+// per-value arithmetic (iq_qcodes.h); prompts go through iq_quantize_k.hip and
+// iq_quantize_v.h, whose results are the same bits.
 #include "iq_common.h"
 #include "iq_device.h"
+#include "iq_qcodes.h"
 
 using namespace iq;
 
 namespace {
-
-constexpr int32_t I32_MIN = (int32_t)0x80000000u;
-
-// groups of a K quantize call up to which it runs one lane per value
-// (quant_k_lane_kernel); past it, one thread per group (~2x fewer
-// instructions per value, and enough threads to fill the device)
-constexpr int64_t LANE_MAX_GROUPS = 65536;
-
-struct QuantOut {
-  uint32_t* codes;     // packed store codes (or null)
-  uint16_t* meta;      // packed store meta
-  int64_t cap_units;   // K: t_cap/64 blocks, V: t_cap/G groups
-  int64_t t_off;       // first token written in the store
-  int32_t* codes_i32;  // dense outputs (optional)
-  uint16_t* scale16;
-  uint16_t* zero16;
-  uint16_t* signs16;
-};
-
-__device__ __forceinline__ bool is_nan(float v) { return v != v; }
-
-// clamp(y, 0, L) keeping NaN, then half-to-even round.  Returns the dense
-// int32 code (INT32_MIN for NaN, as torch's float->int32 on x86).
-__device__ __forceinline__ int32_t code_of(float y, float L) {
-  if (is_nan(y)) return I32_MIN;
-  y = fminf(fmaxf(y, 0.0f), L);
-  return (int32_t)rintf(y);
-}
-
-// Group statistics and per-element codes of the two quantizers, one rounding
-// to the activation dtype (fp16, or bf16 with bf) per reference op (runtime
-// bit width; the templates below pass a constant).
-// asym (quant.py:66-71): scale of b-bit codes from the group's min and max
-__device__ __forceinline__ float asym_scale_b(float mn, float mx, int bits, bool bf = false) {
-  return round_act(round_act(mx - mn, bf) / float((1 << bits) - 1), bf);    // quant.py:68
-}
-__device__ __forceinline__ int32_t asym_code_b(float x, float mn, float s, int bits, bool bf = false) {
-  return code_of(round_act(round_act(x - mn, bf) / s, bf), float((1 << bits) - 1));  // quant.py:69-71
-}
-// sym (quant.py:104-109): scale of b-bit codes (one bit is the sign)
-__device__ __forceinline__ float sym_scale_b(float mx, int bits, bool bf = false) {
-  return round_act(mx / float((1 << (bits - 1)) - 1), bf);              // quant.py:107
-}
-__device__ __forceinline__ int32_t sym_code_b(float x, float s, int bits, bool bf = false) {
-  return code_of(round_act(fabsf(x) / s, bf), float((1 << (bits - 1)) - 1));  // quant.py:108-109
-}
-__device__ __forceinline__ float sign_of(float x) { return x > 0.f ? 1.f : (x < 0.f ? -1.f : 0.f); }  // torch.sign
-// stored fields: the asym code (0 for NaN); sym sign*magnitude + 2^(b-1)
-__device__ __forceinline__ uint32_t asym_field_b(int32_t c, int bits) {
-  return (c == I32_MIN) ? 0u : (uint32_t(c) & ((1u << bits) - 1u));
-}
-__device__ __forceinline__ uint32_t sym_field_b(int32_t c, float sg, int bits) {
-  const int32_t sc = (c == I32_MIN) ? 0 : (sg > 0.f ? c : (sg < 0.f ? -c : 0));
-  return uint32_t(sc + (1 << (bits - 1))) & ((1u << bits) - 1u);  // offset binary
-}
-
-template <int BITS, int G>
-__device__ __forceinline__ void asym_params(const float* v, float& s, float& mn) {
-  float mx = v[0];
-  bool nan = false;
-  mn = v[0];
-#pragma unroll
-  for (int i = 0; i < G; ++i) {
-    nan |= is_nan(v[i]);
-    mn = fminf(mn, v[i]);
-    mx = fmaxf(mx, v[i]);
-  }
-  if (nan) { mn = __builtin_nanf(""); mx = mn; }
-  s = asym_scale_b(mn, mx, BITS);
-}
-template <int BITS>
-__device__ __forceinline__ int32_t asym_code(float x, float mn, float s) { return asym_code_b(x, mn, s, BITS); }
-template <int BITS, int G>
-__device__ __forceinline__ float sym_scale(const float* v) {
-  float mx = 0.f;
-  bool nan = false;
-#pragma unroll
-  for (int i = 0; i < G; ++i) {
-    nan |= is_nan(v[i]);
-    mx = fmaxf(mx, fabsf(v[i]));
-  }
-  if (nan) mx = __builtin_nanf("");
-  return sym_scale_b(mx, BITS);
-}
-template <int BITS>
-__device__ __forceinline__ int32_t sym_code(float x, float s) { return sym_code_b(x, s, BITS); }
-template <int BITS>
-__device__ __forceinline__ uint32_t asym_field(int32_t c) { return asym_field_b(c, BITS); }
-template <int BITS>
-__device__ __forceinline__ uint32_t sym_field(int32_t c, float sg) { return sym_field_b(c, sg, BITS); }
-
-// x / s in fp32, rounded to nearest, for a finite x >= 0 and a finite s > 0
-// that are fp16 values, given r = RN32(1 / s): q0 = RN32(x r), then one
-// correction by the residual x - q0 s, which an fma gives exactly
-// (Markstein's division step), so the result is RN32(x / s) and its fp16
-// rounding is the reference's fp16 division.  One divide per group and three
-// operations per value instead of a divide per value; checked over every
-// such pair of fp16 operands (tests/test_quant_division.py).
-__device__ __forceinline__ float div_rcp(float x, float s, float r) {
-  const float q0 = __fmul_rn(x, r);
-  return __fmaf_rn(__fmaf_rn(-q0, s, x), r, q0);
-}
-
-// Quantize G values held as fp32 copies of fp16 numbers.  fields[] receives
-// the b-bit stored field, codes[] the dense reference code, sgn[] the sign.
-// A group whose scale is finite and positive (every group but the constant,
-// NaN and infinite ones, which divide per value) divides through its
-// reciprocal: its dividends x - min (asym) and |x| (sym) are finite and >= 0.
-template <int BITS, int G>
-__device__ __forceinline__ void quantize_group(const float* v, bool sym, uint32_t* fields, int32_t* codes,
-                                               float* sgn, float& s_out, float& z_out) {
-  if (!sym) {
-    float s, mn;
-    asym_params<BITS, G>(v, s, mn);
-    if (s > 0.f && s < INFINITY) {
-      constexpr float L = float((1 << BITS) - 1);
-      const float r = __fdiv_rn(1.0f, s);
-#pragma unroll
-      for (int i = 0; i < G; ++i) {
-        const int32_t c = code_of(round_f16(div_rcp(round_f16(v[i] - mn), s, r)), L);  // quant.py:69-71
-        codes[i] = c;
-        fields[i] = asym_field<BITS>(c);
-        sgn[i] = 0.f;
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < G; ++i) {
-        const int32_t c = asym_code<BITS>(v[i], mn, s);
-        codes[i] = c;
-        fields[i] = asym_field<BITS>(c);
-        sgn[i] = 0.f;
-      }
-    }
-    s_out = s;
-    z_out = mn;
-  } else {
-    const float s = sym_scale<BITS, G>(v);
-    if (s > 0.f && s < INFINITY) {
-      constexpr float L = float((1 << (BITS - 1)) - 1);
-      const float r = __fdiv_rn(1.0f, s);
-#pragma unroll
-      for (int i = 0; i < G; ++i) {
-        const int32_t c = code_of(round_f16(div_rcp(fabsf(v[i]), s, r)), L);  // quant.py:108-109
-        const float sg = sign_of(v[i]);
-        codes[i] = c;
-        fields[i] = sym_field<BITS>(c, sg);
-        sgn[i] = sg;
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < G; ++i) {
-        const int32_t c = sym_code<BITS>(v[i], s);
-        const float sg = sign_of(v[i]);
-        codes[i] = c;
-        fields[i] = sym_field<BITS>(c, sg);
-        sgn[i] = sg;
-      }
-    }
-    s_out = s;
-    z_out = 0.f;
-  }
-}
-
-// Hybrid (quant.py:133-151): the group quantized both ways, (b-1)-bit asym
-// and b-bit sym; their fp32 dequantizations as the reference computes them
-// (asym c*s + z, sym c*s*sign, a NaN code as INT32_MIN: quant.py:83-93,
-// 121-131); the sym codes are kept iff the asym L1 error is the larger.  The
-// error sums are accumulated in fp64 (as iq_hybrid_mask).  fields[] gets the
-// kept b-bit fields, mw the meta dword {scale | flag << 15, zero}.
-template <int BITS, int G>
-__device__ __forceinline__ void quantize_group_hybrid(const float* v, uint32_t* fields, uint32_t& mw) {
-  float sa, za;
-  asym_params<BITS - 1, G>(v, sa, za);
-  const float ss = sym_scale<BITS, G>(v);
-  double ea = 0.0, es = 0.0;
-#pragma unroll
-  for (int i = 0; i < G; ++i) {
-    const float da = __fadd_rn(__fmul_rn(float(asym_code<BITS - 1>(v[i], za, sa)), sa), za);
-    const float ds = __fmul_rn(__fmul_rn(float(sym_code<BITS>(v[i], ss)), ss), sign_of(v[i]));
-    ea += double(fabsf(__fsub_rn(da, v[i])));
-    es += double(fabsf(__fsub_rn(ds, v[i])));
-  }
-  const bool sym = ea > es;
-#pragma unroll
-  for (int i = 0; i < G; ++i)
-    fields[i] = sym ? sym_field<BITS>(sym_code<BITS>(v[i], ss), sign_of(v[i]))
-                    : asym_field<BITS>(asym_code<BITS - 1>(v[i], za, sa));
-  const uint32_t sh = __half_as_ushort(__float2half_rn(sym ? ss : sa));
-  mw = sym ? (sh | HYB_FLAG) : ((sh & 0x7fffu) | (uint32_t(__half_as_ushort(__float2half_rn(za))) << 16));
-}
-
-template <int BITS, int G>
-__device__ __forceinline__ void pack_fields(const uint32_t* f, uint32_t* w) {
-  constexpr int W = G * BITS / 32;
-#pragma unroll
-  for (int j = 0; j < W; ++j) w[j] = 0u;
-#pragma unroll
-  for (int i = 0; i < G; ++i) {
-    constexpr int dummy = 0;
-    (void)dummy;
-    const int bit = BITS * i;
-    const int wi = bit >> 5, o = bit & 31;
-    w[wi] |= f[i] << o;
-    if (o + BITS > 32) w[wi + 1] |= f[i] >> (32 - o);
-  }
-}
-
-// one group's fields and meta into the store: W code words at unit * W;
-// meta one fp16 scale (sym) or one {scale, zero} dword (asym, hybrid)
-template <int BITS, int G>
-__device__ __forceinline__ void store_group(const QuantOut& o, int64_t unit, const uint32_t* f, bool half_meta,
-                                            uint32_t mw) {
-  constexpr int W = G * BITS / 32;
-  uint32_t w[W];
-  pack_fields<BITS, G>(f, w);
-  uint32_t* cp = o.codes + unit * W;
-#pragma unroll
-  for (int j = 0; j < W; ++j) cp[j] = w[j];
-  if (half_meta) o.meta[unit] = uint16_t(mw);
-  else reinterpret_cast<uint32_t*>(o.meta)[unit] = mw;
-}
-
-__device__ __forceinline__ uint32_t meta_word(float s, float z, bool bf = false) {
-  return uint32_t(f2act(s, bf)) | (uint32_t(f2act(z, bf)) << 16);
-}
 
 template <int BITS, int G>
 __device__ __forceinline__ void unpack_fields(const uint32_t* w, bool sym, int32_t* c) {
@@ -261,85 +27,16 @@ __device__ __forceinline__ void unpack_fields(const uint32_t* w, bool sym, int32
   }
 }
 
-// ---- K: groups along head_dim, one thread per (b, h, t, g) ----------------
-// HYB: a hybrid store (store only, no dense outputs)
-template <int BITS, int G, bool DENSE, bool HYB = false>
-__global__ __launch_bounds__(256) void quant_k_kernel(const uint16_t* __restrict__ x, int64_t sxb, int64_t sxh,
-                                                      int64_t sxt, const uint16_t* __restrict__ norm, int B,
-                                                      int H, int n, int D, int sym, QuantOut o) {
-  const int ng = D / G;
-  const int64_t gid = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int64_t total = int64_t(B) * H * n * ng;
-  if (gid >= total) return;
-  const int g = int(gid % ng);
-  int64_t r = gid / ng;
-  const int t = int(r % n);
-  r /= n;
-  const int h = int(r % H);
-  const int b = int(r / H);
-
-  const uint16_t* xp = x + b * sxb + h * sxh + t * sxt + g * G;
-  float v[G];
-#pragma unroll
-  for (int i = 0; i < G; i += 8) {
-    const uint4 u = *reinterpret_cast<const uint4*>(xp + i);
-    const uint32_t uu[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      v[i + 2 * j] = h2f(uint16_t(uu[j] & 0xffffu));
-      v[i + 2 * j + 1] = h2f(uint16_t(uu[j] >> 16));
-    }
-  }
-  if (norm) {  // cache.py:125  key_states / key_normalization_factor (fp16)
-    const uint16_t* np_ = norm + (int64_t(b) * H + h) * D + g * G;
-#pragma unroll
-    for (int i = 0; i < G; ++i) v[i] = round_f16(v[i] / h2f(np_[i]));
-  }
-  const int64_t bh = int64_t(b) * H + h;
-  const int64_t tt = o.t_off + t;
-  const int64_t unit = ((bh * o.cap_units + tt / TOKEN_BLOCK) * ng + g) * TOKEN_BLOCK + tt % TOKEN_BLOCK;
-  uint32_t f[G];
-  if constexpr (HYB) {
-    if constexpr (BITS >= 2) {
-      uint32_t mw;
-      quantize_group_hybrid<BITS, G>(v, f, mw);
-      store_group<BITS, G>(o, unit, f, false, mw);
-    }
-    return;
-  }
-  int32_t c[G];
-  float sg[G];
-  float s, z;
-  quantize_group<BITS, G>(v, sym != 0, f, c, sg, s, z);
-  if (o.codes) store_group<BITS, G>(o, unit, f, sym != 0, meta_word(s, z));
-  if constexpr (DENSE) {  // the reference-format outputs (quant.py API)
-    const int64_t row_el = (bh * n + t) * D + g * G;
-    if (o.codes_i32) {
-#pragma unroll
-      for (int i = 0; i < G; ++i) o.codes_i32[row_el + i] = c[i];
-    }
-    if (o.signs16) {
-#pragma unroll
-      for (int i = 0; i < G; ++i) o.signs16[row_el + i] = __half_as_ushort(__float2half_rn(sg[i]));
-    }
-    const int64_t red = (bh * n + t) * ng + g;
-    if (o.scale16) o.scale16[red] = __half_as_ushort(__float2half_rn(s));
-    if (o.zero16) o.zero16[red] = __half_as_ushort(__float2half_rn(z));
-  }
-}
-
-// ---- one group across G lanes (small appends) ------------------------------
-// The one-thread-per-group kernels run each group as one thread's chain of
-// ~G * 25 dependent instructions: fine for a prompt (many groups), but a
-// decode step's append is a few hundred groups, i.e. one or two workgroups
-// and ~8 us of latency (a one-token K append at B=16: measured).  Here the
-// G <= 64 lanes of an aligned segment of one wave hold one group, lane i its
-// element i; the extremes, the NaN test and the packed words are reduced
-// across the segment.  The per-value arithmetic is quantize_group's /
-// quant_group_rt's, the extremes are exact and the words are ORs of disjoint
-// bit fields, so the fields and meta are the same bit for bit.  Hybrid's two
-// error sums are added in element order (seg_sum_ordered), as the
-// one-thread path adds them.
+// ---- one group across G lanes (a decode step's append) ---------------------
+// One thread per group is a chain of ~G * 25 dependent instructions, and an
+// append is a few hundred groups: one or two workgroups and ~8 us of latency
+// (a one-token K append at B=16: measured).  Here the G <= 64 lanes of an
+// aligned segment of one wave hold one group, lane i its element i; the
+// extremes, the NaN test and the packed words are reduced across the segment.
+// The per-value arithmetic is quant_group_rt's, the extremes are exact and
+// the words are ORs of disjoint bit fields, so the fields and meta are the
+// same bit for bit.  Hybrid's two error sums are added in element order
+// (seg_sum_ordered), as the one-thread path adds them.
 template <int G>
 __device__ __forceinline__ uint64_t seg_mask() {
   if constexpr (G == 64) {
@@ -468,84 +165,12 @@ __device__ __forceinline__ int32_t quant_group_lanes(float v, int i, int bits, i
   return c;
 }
 
-// ---- one lane per value (quant_group_lanes), either axis -------------------
-// G <= 64, asym or sym, fp16 or bf16 activations; the same stores and
-// reference-format outputs as quant_k_kernel (axis 0, groups along D) and
-// quant_v_kernel (axis 1, groups along tokens).  Serves small K calls (a
-// decode step's tokens, where one thread per group would idle the device)
-// and every bf16 quantization of those formats.
-struct LaneArgs {
-  const uint16_t* x;
-  int64_t sxb, sxh, sxt;
-  const uint16_t* norm;  // axis 0 only
-  int B, H, n, D, bits, mode, bf, axis;
-};
-template <int G>
-__global__ __launch_bounds__(256) void quant_lane_kernel(LaneArgs a, QuantOut o) {
-  const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int64_t gid = e / G;
-  const int i = int(e % G);
-  const bool bf = a.bf != 0;
-  int64_t bh, unit, xoff, el, red, row_el = 0;
-  int dcol;
-  if (a.axis == 0) {
-    const int ng = a.D / G;
-    if (gid >= int64_t(a.B) * a.H * a.n * ng) return;  // whole G-lane segments
-    const int g = int(gid % ng);
-    const int64_t row = gid / ng;  // bh * n + t
-    const int t = int(row % a.n);
-    bh = row / a.n;
-    dcol = g * G + i;
-    xoff = (bh / a.H) * a.sxb + (bh % a.H) * a.sxh + t * a.sxt + dcol;
-    const int64_t tt = o.t_off + t;
-    unit = ((bh * o.cap_units + tt / TOKEN_BLOCK) * ng + g) * TOKEN_BLOCK + tt % TOKEN_BLOCK;
-    row_el = row * a.D + g * G;
-    el = row_el + i;
-    red = row * ng + g;
-  } else {
-    const int ngn = a.n / G;
-    if (gid >= int64_t(a.B) * a.H * ngn * a.D) return;
-    const int d = int(gid % a.D);
-    const int64_t r = gid / a.D;  // bh * ngn + gi
-    const int gi = int(r % ngn);
-    bh = r / ngn;
-    dcol = d;
-    const int t = gi * G + i;
-    xoff = (bh / a.H) * a.sxb + (bh % a.H) * a.sxh + int64_t(t) * a.sxt + d;
-    unit = (bh * o.cap_units + o.t_off / G + gi) * a.D + d;
-    el = (bh * a.n + t) * a.D + d;
-    red = r * a.D + d;
-  }
-  float v = act2f(a.x[xoff], bf);
-  if (a.norm) v = round_act(v / act2f(a.norm[bh * a.D + dcol], bf), bf);  // cache.py:125
-  float sg, sc, zp;
-  const int32_t c = quant_group_lanes<G>(v, i, a.bits, a.mode, bf, o.codes != nullptr,
-                                         o.codes ? o.codes + unit * ((G * a.bits) >> 5) : nullptr, o.meta, unit, sg,
-                                         sc, zp);
-  if (o.codes_i32) o.codes_i32[el] = c;
-  if (o.signs16) o.signs16[el] = f2act(sg, bf);
-  if (i == 0) {
-    if (o.scale16) o.scale16[red] = f2act(sc, bf);
-    if (o.zero16) o.zero16[red] = f2act(zp, bf);
-  }
-}
-
-// One group, quantized as quantize_group / quantize_group_hybrid do, with
-// the bit width, mode and activation dtype known at run time: v[] holds the
+// One group by one thread (groups of 128), with the bit width, mode and activation dtype known at run time: v[] holds the
 // group's G inputs (registers; loaded together, one memory latency per group),
 // the fields are stored word by word as they fill, the meta word last.
-// Optional reference-format outputs (RtRef, asym or sym): element i's code and
-// sign at codes[el0 + i * el_step], signs[...], the scale and zero at red.
-struct RtRef {
-  int32_t* codes;
-  uint16_t* signs;
-  uint16_t* scale;
-  uint16_t* zero;
-  int64_t el0, el_step, red;
-};
 template <int G>
 __device__ __forceinline__ void quant_group_rt(const float* v, int bits, int mode, bool bf, uint32_t* out,
-                                               uint16_t* meta, int64_t unit, const RtRef* ref = nullptr) {
+                                               uint16_t* meta, int64_t unit) {
   const int abits = mode == IQ_MODE_HYBRID ? bits - 1 : bits;
   float mn = v[0], mx = v[0], amx = 0.f;
   bool nan = false;
@@ -559,7 +184,7 @@ __device__ __forceinline__ void quant_group_rt(const float* v, int bits, int mod
   if (nan) { mn = __builtin_nanf(""); mx = mn; amx = mn; }
   const float sa = asym_scale_b(mn, mx, abits, bf), ss = sym_scale_b(amx, bits, bf);
   bool sym = mode == IQ_MODE_SYM;
-  if (mode == IQ_MODE_HYBRID) {  // quantize_group_hybrid's choice
+  if (mode == IQ_MODE_HYBRID) {  // quant.py:144
     double ea = 0.0, es = 0.0;
 #pragma unroll
     for (int i = 0; i < G; ++i) {
@@ -576,24 +201,14 @@ __device__ __forceinline__ void quant_group_rt(const float* v, int bits, int mod
   for (int i = 0; i < G; ++i) {
     const int32_t c = sym ? sym_code_b(v[i], ss, bits, bf) : asym_code_b(v[i], mn, sa, abits, bf);
     const uint32_t fld = sym ? sym_field_b(c, sign_of(v[i]), bits) : asym_field_b(c, bits);
-    if (ref) {
-      if (ref->codes) ref->codes[ref->el0 + i * ref->el_step] = c;
-      if (ref->signs) ref->signs[ref->el0 + i * ref->el_step] = f2act(sign_of(v[i]), bf);
-    }
     acc |= uint64_t(fld) << pos;
     pos += bits;
     if (pos >= 32) {
-      if (out) out[wj] = uint32_t(acc);
-      ++wj;
+      out[wj++] = uint32_t(acc);
       acc >>= 32;
       pos -= 32;
     }
   }
-  if (ref) {
-    if (ref->scale) ref->scale[ref->red] = f2act(sym ? ss : sa, bf);
-    if (ref->zero) ref->zero[ref->red] = f2act(mn, bf);
-  }
-  if (!out) return;
   if (mode == IQ_MODE_SYM) {
     meta[unit] = f2act(ss, bf);
   } else if (mode == IQ_MODE_HYBRID) {
@@ -602,122 +217,6 @@ __device__ __forceinline__ void quant_group_rt(const float* v, int bits, int mod
         sym ? (sh | HYB_FLAG) : ((sh & 0x7fffu) | (uint32_t(f2act(mn, bf)) << 16));
   } else {
     reinterpret_cast<uint32_t*>(meta)[unit] = meta_word(sa, mn, bf);
-  }
-}
-
-// ---- one thread per group, bit width / mode / dtype at run time -----------
-// (quant_group_rt) The bf16 formats quant_lane_kernel does not take: groups
-// of 128 and hybrid stores; either axis, stores and reference outputs.
-template <int G>
-__global__ __launch_bounds__(256) void quant_rt_kernel(LaneArgs a, QuantOut o) {
-  const int64_t gid = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const bool bf = a.bf != 0;
-  float v[G];
-  int64_t bh, unit;
-  RtRef ref{o.codes_i32, o.signs16, o.scale16, o.zero16, 0, 0, 0};
-  if (a.axis == 0) {
-    const int ng = a.D / G;
-    if (gid >= int64_t(a.B) * a.H * a.n * ng) return;
-    const int g = int(gid % ng);
-    const int64_t row = gid / ng;  // bh * n + t
-    const int t = int(row % a.n);
-    bh = row / a.n;
-    const uint16_t* xp = a.x + (bh / a.H) * a.sxb + (bh % a.H) * a.sxh + t * a.sxt + g * G;
-#pragma unroll
-    for (int i = 0; i < G; ++i) v[i] = act2f(xp[i], bf);
-    if (a.norm) {  // cache.py:125
-#pragma unroll
-      for (int i = 0; i < G; ++i) v[i] = round_act(v[i] / act2f(a.norm[bh * a.D + g * G + i], bf), bf);
-    }
-    const int64_t tt = o.t_off + t;
-    unit = ((bh * o.cap_units + tt / TOKEN_BLOCK) * ng + g) * TOKEN_BLOCK + tt % TOKEN_BLOCK;
-    ref.el0 = row * a.D + g * G;
-    ref.el_step = 1;
-    ref.red = row * ng + g;
-  } else {
-    const int ngn = a.n / G;
-    if (gid >= int64_t(a.B) * a.H * ngn * a.D) return;
-    const int d = int(gid % a.D);
-    const int64_t r = gid / a.D;  // bh * ngn + gi
-    const int gi = int(r % ngn);
-    bh = r / ngn;
-    const uint16_t* xp = a.x + (bh / a.H) * a.sxb + (bh % a.H) * a.sxh + int64_t(gi) * G * a.sxt + d;
-#pragma unroll
-    for (int i = 0; i < G; ++i) v[i] = act2f(xp[int64_t(i) * a.sxt], bf);
-    unit = (bh * o.cap_units + o.t_off / G + gi) * a.D + d;
-    ref.el0 = (bh * a.n + int64_t(gi) * G) * a.D + d;
-    ref.el_step = a.D;
-    ref.red = r * a.D + d;
-  }
-  const bool any_ref = o.codes_i32 || o.signs16 || o.scale16 || o.zero16;
-  quant_group_rt<G>(v, a.bits, a.mode, bf, o.codes ? o.codes + unit * ((G * a.bits) >> 5) : nullptr, o.meta, unit,
-                    any_ref ? &ref : nullptr);
-}
-
-// bf16 quantization, or a small fp16 K call: one lane per value where the
-// format allows (G <= 64, asym / sym), else one thread per group at run time
-int launch_lane_or_rt(const LaneArgs& a, const QuantOut& o, int group, hipStream_t st) {
-  const int64_t groups = a.axis == 0 ? int64_t(a.B) * a.H * a.n * (a.D / group)
-                                     : int64_t(a.B) * a.H * (a.n / group) * a.D;
-  if (groups == 0) return IQ_OK;
-  if (group <= 64 && a.mode != IQ_MODE_HYBRID) {
-    auto* kern = group == 64 ? quant_lane_kernel<64> : quant_lane_kernel<32>;
-    kern<<<dim3(unsigned(ceil_div(groups * group, 256))), 256, 0, st>>>(a, o);
-  } else {
-    auto* kern = group == 128 ? quant_rt_kernel<128> : group == 64 ? quant_rt_kernel<64> : quant_rt_kernel<32>;
-    kern<<<dim3(unsigned(ceil_div(groups, 256))), 256, 0, st>>>(a, o);
-  }
-  return launch_status();
-}
-
-// ---- V: groups along tokens, one thread per (b, h, token-group, d) --------
-template <int BITS, int G, bool DENSE, bool HYB = false>
-__global__ __launch_bounds__(256) void quant_v_kernel(const uint16_t* __restrict__ x, int64_t sxb, int64_t sxh,
-                                                      int64_t sxt, int B, int H, int n, int D, int sym,
-                                                      QuantOut o) {
-  const int ngn = n / G;
-  const int64_t gid = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int64_t total = int64_t(B) * H * ngn * D;
-  if (gid >= total) return;
-  const int d = int(gid % D);
-  int64_t r = gid / D;
-  const int gi = int(r % ngn);
-  r /= ngn;
-  const int h = int(r % H);
-  const int b = int(r / H);
-
-  const uint16_t* xp = x + b * sxb + h * sxh + int64_t(gi) * G * sxt + d;
-  float v[G];
-#pragma unroll
-  for (int i = 0; i < G; ++i) v[i] = h2f(xp[i * sxt]);
-  const int64_t bh = int64_t(b) * H + h;
-  const int64_t unit = (bh * o.cap_units + o.t_off / G + gi) * D + d;
-  uint32_t f[G];
-  if constexpr (HYB) {
-    if constexpr (BITS >= 2) {
-      uint32_t mw;
-      quantize_group_hybrid<BITS, G>(v, f, mw);
-      store_group<BITS, G>(o, unit, f, false, mw);
-    }
-    return;
-  }
-  int32_t c[G];
-  float sg[G];
-  float s, z;
-  quantize_group<BITS, G>(v, sym != 0, f, c, sg, s, z);
-  if (o.codes) store_group<BITS, G>(o, unit, f, sym != 0, meta_word(s, z));
-  if constexpr (DENSE) {  // the reference-format outputs (quant.py API)
-    if (o.codes_i32 || o.signs16) {
-#pragma unroll
-      for (int i = 0; i < G; ++i) {
-        const int64_t el = (bh * n + int64_t(gi) * G + i) * D + d;
-        if (o.codes_i32) o.codes_i32[el] = c[i];
-        if (o.signs16) o.signs16[el] = __half_as_ushort(__float2half_rn(sg[i]));
-      }
-    }
-    const int64_t red = (bh * ngn + gi) * D + d;
-    if (o.scale16) o.scale16[red] = __half_as_ushort(__float2half_rn(s));
-    if (o.zero16) o.zero16[red] = __half_as_ushort(__float2half_rn(z));
   }
 }
 
@@ -941,7 +440,7 @@ __global__ __launch_bounds__(256) void unpack_v_kernel(const uint32_t* __restric
 // the store, in one launch for both roles.  The quantizer here takes the bit
 // width, group size and mode at run time and reads each group from memory
 // once per pass (no per-group register arrays); every element goes through
-// the same fp16 ops as quantize_group / quantize_group_hybrid.
+// the same fp16 ops as the prompt quantizers.
 struct WinRole {
   uint16_t* buf;
   int64_t sb, sh, st;
@@ -1156,89 +655,6 @@ int iq_v_store_bytes(int64_t B, int64_t H, int64_t t_cap, int64_t D, int group, 
   *codes_bytes = B * H * t_cap * D * bits / 8;
   *meta_bytes = B * H * (t_cap / group) * D * meta_unit_bytes(mode);
   return IQ_OK;
-}
-
-int iq_quantize_k(const void* x, int64_t sx_b, int64_t sx_h, int64_t sx_t, const void* norm, int B, int H,
-                  int n, int D, int group, int bits, int mode, uint32_t* k_codes, uint16_t* k_meta,
-                  int64_t t_cap, int64_t t_off, int32_t* codes_i32, void* scale16, void* zero16, void* signs16,
-                  void* stream) {
-  IQ_CHECK(x, IQ_ERR_NULL);
-  const bool bf = act_bf16(mode);
-  mode = base_mode(mode);
-  if (int e = check_store(bits, group, mode)) return e;
-  IQ_CHECK(B >= 0 && H >= 0 && n >= 0 && D > 0, IQ_ERR_SHAPE);
-  IQ_CHECK(D % group == 0, IQ_ERR_GROUP);
-  IQ_CHECK(aligned(x, 16) && sx_b % 8 == 0 && sx_h % 8 == 0 && sx_t % 8 == 0, IQ_ERR_ALIGN);
-  IQ_CHECK((k_codes == nullptr) == (k_meta == nullptr), IQ_ERR_NULL);
-  if (k_codes) {
-    IQ_CHECK(t_cap % TOKEN_BLOCK == 0 && t_off >= 0, IQ_ERR_ALIGN);
-    IQ_CHECK(t_off + n <= t_cap, IQ_ERR_RANGE);
-    IQ_CHECK(aligned(k_codes, 4) && aligned(k_meta, 4), IQ_ERR_ALIGN);
-  }
-  IQ_CHECK(!(mode == IQ_MODE_SYM && zero16), IQ_ERR_MODE);
-  IQ_CHECK(!(mode == IQ_MODE_ASYM && signs16), IQ_ERR_MODE);
-  const bool dense = codes_i32 || scale16 || zero16 || signs16;
-  IQ_CHECK(mode != IQ_MODE_HYBRID || (k_codes && !dense), IQ_ERR_MODE);
-  const int64_t total = int64_t(B) * H * n * (D / group);
-  if (total == 0) return IQ_OK;
-  QuantOut o{k_codes, k_meta, t_cap / TOKEN_BLOCK, t_off, codes_i32, (uint16_t*)scale16, (uint16_t*)zero16,
-             (uint16_t*)signs16};
-  const int sym = mode == IQ_MODE_SYM;
-  // a call of few groups (a decode step's tokens) takes one lane per value:
-  // one thread per group would leave most of the device idle on long chains
-  if (bf || (mode != IQ_MODE_HYBRID && group <= 64 && total <= LANE_MAX_GROUPS)) {
-    const LaneArgs a{(const uint16_t*)x, sx_b, sx_h, sx_t, (const uint16_t*)norm, B, H, n, D, bits, mode, bf ? 1 : 0,
-                     0};
-    return launch_lane_or_rt(a, o, group, (hipStream_t)stream);
-  }
-  return dispatch_store_bits_group(bits, group, [&]<int BITS, int G>() {
-    // the store-only append (no reference-format outputs) drops their registers
-    auto* kern = mode == IQ_MODE_HYBRID ? quant_k_kernel<BITS, G, false, true>
-                 : dense               ? quant_k_kernel<BITS, G, true>
-                                       : quant_k_kernel<BITS, G, false>;
-    kern<<<dim3(unsigned(ceil_div(total, 256))), 256, 0, (hipStream_t)stream>>>(
-        (const uint16_t*)x, sx_b, sx_h, sx_t, (const uint16_t*)norm, B, H, n, D, sym, o);
-    return launch_status();
-  });
-}
-
-int iq_quantize_v(const void* x, int64_t sx_b, int64_t sx_h, int64_t sx_t, int B, int H, int n, int D,
-                  int group, int bits, int mode, uint32_t* v_codes, uint16_t* v_meta, int64_t t_cap,
-                  int64_t t_off, int32_t* codes_i32, void* scale16, void* zero16, void* signs16, void* stream) {
-  IQ_CHECK(x, IQ_ERR_NULL);
-  const bool bf = act_bf16(mode);
-  mode = base_mode(mode);
-  if (int e = check_store(bits, group, mode)) return e;
-  IQ_CHECK(B >= 0 && H >= 0 && n >= 0 && D > 0, IQ_ERR_SHAPE);
-  IQ_CHECK(n % group == 0, IQ_ERR_GROUP);
-  IQ_CHECK(aligned(x, 2), IQ_ERR_ALIGN);
-  IQ_CHECK((v_codes == nullptr) == (v_meta == nullptr), IQ_ERR_NULL);
-  if (v_codes) {
-    IQ_CHECK(t_cap % group == 0 && t_off % group == 0 && t_off >= 0, IQ_ERR_ALIGN);
-    IQ_CHECK(t_off + n <= t_cap, IQ_ERR_RANGE);
-    IQ_CHECK(aligned(v_codes, 4) && aligned(v_meta, 4), IQ_ERR_ALIGN);
-  }
-  IQ_CHECK(!(mode == IQ_MODE_SYM && zero16), IQ_ERR_MODE);
-  IQ_CHECK(!(mode == IQ_MODE_ASYM && signs16), IQ_ERR_MODE);
-  const bool dense = codes_i32 || scale16 || zero16 || signs16;
-  IQ_CHECK(mode != IQ_MODE_HYBRID || (v_codes && !dense), IQ_ERR_MODE);
-  const int64_t total = int64_t(B) * H * (n / group) * D;
-  if (total == 0) return IQ_OK;
-  QuantOut o{v_codes, v_meta, t_cap / group, t_off, codes_i32, (uint16_t*)scale16, (uint16_t*)zero16,
-             (uint16_t*)signs16};
-  if (bf) {
-    const LaneArgs a{(const uint16_t*)x, sx_b, sx_h, sx_t, nullptr, B, H, n, D, bits, mode, 1, 1};
-    return launch_lane_or_rt(a, o, group, (hipStream_t)stream);
-  }
-  const int sym = mode == IQ_MODE_SYM;
-  return dispatch_store_bits_group(bits, group, [&]<int BITS, int G>() {
-    auto* kern = mode == IQ_MODE_HYBRID ? quant_v_kernel<BITS, G, false, true>
-                 : dense               ? quant_v_kernel<BITS, G, true>
-                                       : quant_v_kernel<BITS, G, false>;
-    kern<<<dim3(unsigned(ceil_div(total, 256))), 256, 0, (hipStream_t)stream>>>(
-        (const uint16_t*)x, sx_b, sx_h, sx_t, B, H, n, D, sym, o);
-    return launch_status();
-  });
 }
 
 int iq_dequant_k(const uint32_t* k_codes, const uint16_t* k_meta, int64_t t_cap, const void* norm, int B, int H,

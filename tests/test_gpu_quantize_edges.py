@@ -1,0 +1,130 @@
+"""Prompt quantization at the sizes where the kernels' tiles and lanes end:
+one token, block edges, offsets inside a block, head_dims whose rows do not
+divide a workgroup (K) and odd or misaligned columns (V), strided inputs, every
+mode, width, group and activation type.  Bit-exact against the oracle: the
+quantizers are defined bit for bit (codes, scales, zero points)."""
+import numpy as np
+import pytest
+import torch
+
+from innerq_amd import ops
+from oracle import quant_ref as Q
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+TD = {"f16": torch.float16, "bf16": torch.bfloat16}
+MODES = [("asymmetric", (1, 2, 3, 4)), ("symmetric", (2, 3, 4)), ("hybrid", (2, 3, 4))]
+
+
+def planted(B, H, n, D, seed, act):
+    """Normal data with the groups that leave the fast arithmetic: zeros of both signs, constant
+    rows, exact ties, subnormals, NaN, infinities, a range that overflows fp16."""
+    rng = np.random.default_rng(seed)
+    x = rng.standard_normal((B, H, n, D)).astype(np.float32)
+    flat = x.reshape(B * H, n, D)
+    flat[-1, ::5] = 0.0
+    flat[-1, ::5, 1::2] = -0.0
+    flat[0, n // 2] = 1.5
+    flat[0, n // 3] = np.arange(D) % 16 + 0.5
+    flat[-1, n - 1] *= 1e-6
+    flat[-1, 0, D // 2] = np.nan
+    flat[0, n - 1, 0] = np.inf
+    flat[0, 0, :2] = [60000.0, -60000.0][:D]
+    return torch.from_numpy(x).to(TD[act])
+
+
+def host(t):
+    return t.float().numpy() if t.dtype == torch.bfloat16 else t.numpy()
+
+
+def act_bits(a, act):
+    return Q.f16_bits(a) if act == "f16" else Q.bf16_bits(a)
+
+
+def expected(x, G, bits, mode, axis, act):
+    """(fields, meta halves [.., M]) of the packed groups, from the oracle."""
+    ch = axis == "channel"
+    with np.errstate(all="ignore"):
+        if mode == "hybrid":
+            c, s, z = (Q.quantize_channeldim_hybrid if ch else Q.quantize_tokendim_hybrid)(x, G, bits, act)
+            mask = s["mask"]
+            el = np.repeat(mask, G, axis=-1 if ch else 2)
+            za = np.where(c["zp"] == Q.INT32_MIN, 0, c["zp"])
+            sy = np.where(c["nozp"] == Q.INT32_MIN, 0, c["nozp"]) * z["nozp"].astype(np.int32) + (1 << (bits - 1))
+            half = np.where(mask, act_bits(s["nozp"], act) | 0x8000, act_bits(s["zp"], act) & 0x7FFF)
+            zero = np.where(mask, 0, act_bits(z["zp"], act))
+            return np.where(el, sy, za), np.stack([half, zero], -1).astype(np.uint16)
+        f = {("symmetric", True): Q.quantize_channeldim_sym, ("symmetric", False): Q.quantize_tokendim_sym,
+             ("asymmetric", True): Q.quantize_channeldim_asym, ("asymmetric", False): Q.quantize_tokendim_asym}
+        c, s, z = f[mode, ch](x, G, bits, act)
+    c = np.where(c == Q.INT32_MIN, 0, c)
+    if mode == "symmetric":
+        return c * z.astype(np.int32) + (1 << (bits - 1)), act_bits(s, act)[..., None]
+    return c & ((1 << bits) - 1), np.stack([act_bits(s, act), act_bits(z, act)], -1)
+
+
+def same_meta(got, want, act):
+    """Equal bits, any NaN pattern standing for NaN and a zero of either sign for zero (torch's amin
+    and numpy's min may keep either of two zeros)."""
+    exp = 0x7C00 if act == "f16" else 0x7F80
+    nan = ((got & 0x7FFF) > exp) & ((want & 0x7FFF) > exp)
+    zero = ((got & 0x7FFF) == 0) & ((want & 0x7FFF) == 0)
+    return bool(np.all((got == want) | nan | zero))
+
+
+# the sign of an all-NaN hybrid group's flag and the like stay out of the comparison: the planted
+# NaN sits in one group, compared by its fields
+@pytest.mark.parametrize("act", ["f16", "bf16"])
+@pytest.mark.parametrize("mode,widths", MODES)
+@pytest.mark.parametrize("n,D,G,off,strided", [(1, 128, 32, 0, False), (63, 64, 32, 0, True), (65, 128, 64, 63, False),
+                                               (64, 128, 128, 1, True), (130, 96, 32, 5, False),
+                                               (17, 384, 128, 0, False), (1027, 64, 64, 0, True)])
+def test_keys(act, mode, widths, n, D, G, off, strided):
+    B, H = 2, 2
+    x = planted(B, H, n, D, n + D, act)
+    xd = x.to(DEV)
+    if strided:
+        xd = xd.transpose(1, 2).contiguous().transpose(1, 2)
+    for bits in widths:
+        st = ops.PackedStore("channel", B, H, D, G, bits, mode, DEV, dtype=TD[act])
+        if off:
+            st.append(torch.ones(B, H, off, D, device=DEV, dtype=TD[act]))
+        st.append(xd)
+        fields, meta = expected(host(x), G, bits, mode, "channel", act)
+        W, M, ng = G * bits // 32, meta.shape[-1], D // G
+        T = off + n
+        words = st.codes.cpu().numpy().view(np.uint32).reshape(B, H, -1, ng, 64, W)
+        got = words.transpose(0, 1, 2, 4, 3, 5).reshape(B, H, -1, ng, W)[:, :, off:T]
+        np.testing.assert_array_equal(Q.unpack_groups(got, bits, G).reshape(B, H, n, D), fields)
+        gm = st.meta.cpu().numpy().view(np.uint16).reshape(B, H, -1, ng, 64, M)
+        gm = gm.transpose(0, 1, 2, 4, 3, 5).reshape(B, H, -1, ng, M)[:, :, off:T]
+        assert same_meta(gm, meta, act)
+
+
+@pytest.mark.parametrize("act", ["f16", "bf16"])
+@pytest.mark.parametrize("mode,widths", MODES)
+@pytest.mark.parametrize("groups,D,G,off,layout", [(1, 128, 32, 0, "plain"), (3, 64, 64, 1, "heads last"),
+                                                   (2, 128, 128, 0, "heads last"), (5, 33, 32, 1, "plain"),
+                                                   (2, 1, 64, 0, "plain"), (2, 130, 32, 0, "odd rows")])
+def test_values(act, mode, widths, groups, D, G, off, layout):
+    B, H, n = 2, 2, groups * G
+    x = planted(B, H, n, D, n + D, act)
+    xd = x.to(DEV)
+    if layout == "heads last":
+        xd = xd.transpose(1, 2).contiguous().transpose(1, 2)
+    if layout == "odd rows":  # rows that start at odd elements
+        y = torch.empty(B, H, n, D + 1, dtype=TD[act], device=DEV)
+        y[..., 1:] = xd
+        xd = y[..., 1:]
+    for bits in widths:
+        st = ops.PackedStore("token", B, H, D, G, bits, mode, DEV, dtype=TD[act])
+        if off:
+            st.append(torch.ones(B, H, off * G, D, device=DEV, dtype=TD[act]))
+        st.append(xd)
+        fields, meta = expected(host(x), G, bits, mode, "token", act)
+        W, M = G * bits // 32, meta.shape[-1]
+        words = st.codes.cpu().numpy().view(np.uint32).reshape(B, H, -1, D, W)[:, :, off:off + groups]
+        got = Q.unpack_groups(words, bits, G).transpose(0, 1, 2, 4, 3).reshape(B, H, n, D)
+        np.testing.assert_array_equal(got, fields)
+        gm = st.meta.cpu().numpy().view(np.uint16).reshape(B, H, -1, D, M)[:, :, off:off + groups]
+        assert same_meta(gm, meta, act)
