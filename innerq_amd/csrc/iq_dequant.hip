@@ -1,0 +1,325 @@
+// Dense values of packed stores (gfx950): iq_dequant_k (groups along head_dim)
+// and iq_dequant_v (groups along tokens), the reads of the reference's dense
+// path (cache.py:235-281).
+//
+// value = fp32(c * s + z) with c * s exact (quant.py:83-93, 121-131; hybrid
+// groups as their flag says, quant.py:153-176), times the key normalization
+// factor in fp32 (cache.py:132), rounded once to the output's type.
+//
+// Bound: HBM, and by its writes (2 B out against b/8 + m/G B in per value), so
+// the split follows the output: a lane writes 16 bytes of a row (K) or 8 (V)
+// and a wave writes whole rows.  (A thread per group, the form before, wrote
+// single halves 2 G bytes apart: 217 us for 4 x 8 heads x 16256 tokens, D =
+// 128; now 42 us for 3-bit keys with a factor and 33 us for 2-bit values, 3.8
+// and 4.7 TB/s.)  Fields become fp16 integers two at a time: one shift
+// and one and-or with an exponent pattern, one packed subtraction.
+#include "iq_common.h"
+#include "iq_device.h"
+
+using namespace iq;
+
+namespace {
+
+typedef float f2_t __attribute__((ext_vector_type(2)));
+typedef float f4_t __attribute__((ext_vector_type(4)));
+typedef __bf16 b2_t __attribute__((ext_vector_type(2)));
+
+struct DeqOut {
+  uint16_t* out16;  // in the activation dtype
+  float* out32;
+  int64_t sob, soh, sot;
+  int vec16, vec32;  // rows take 16-byte (K) / 8-byte (V) stores of out16, 16-byte stores of out32
+};
+
+// {scale, zero} of a unit and the integer subtracted from its fields:
+// value = (field - off) * s + z
+template <bool BF>
+__device__ __forceinline__ void unit_params(const uint16_t* meta, int64_t unit, int mode, int bits, float& s, float& z,
+                                            int& off) {
+  if (mode == IQ_MODE_SYM) {
+    s = act2f(meta[unit], BF);
+    z = 0.f;
+    off = 1 << (bits - 1);
+    return;
+  }
+  const uint32_t mw = reinterpret_cast<const uint32_t*>(meta)[unit];
+  const bool sym = mode == IQ_MODE_HYBRID && hyb_sym(mw);
+  s = mode == IQ_MODE_HYBRID ? hyb_scale(mw, BF) : act2f(uint16_t(mw & 0xffffu), BF);
+  z = sym ? 0.f : act2f(uint16_t(mw >> 16), BF);
+  off = sym ? 1 << (bits - 1) : 0;
+}
+
+// fields at bit p of both halves of y as fp16 integers less off2
+__device__ __forceinline__ h2_t pair_at(uint32_t y, int p, uint32_t mask, h2_t bias) {
+  return __builtin_bit_cast(h2_t, ((y >> p) & mask) | 0x64006400u) - bias;
+}
+__device__ __forceinline__ h2_t bias_of(int off0, int off1) {  // {1024 + off} halves
+  return __builtin_bit_cast(h2_t, 0x64006400u + uint32_t(off0) + (uint32_t(off1) << 16));
+}
+
+template <bool BF>
+__device__ __forceinline__ uint32_t out_pair(float a, float b) {
+  if constexpr (BF) return uint32_t(f2bf(a)) | (uint32_t(f2bf(b)) << 16);
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2_t{a, b}, h2_t));
+}
+// the same for values known to be numbers (v_cvt_pk_bf16_f32 keeps a NaN's sign and payload, f2bf does not)
+template <bool BF>
+__device__ __forceinline__ uint32_t out_pair_num(float a, float b) {
+  if constexpr (BF) return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2_t{a, b}, b2_t));
+  return out_pair<BF>(a, b);
+}
+__device__ __forceinline__ bool tame(float s, float z) { return fabsf(s) < 0x1p100f && fabsf(z) < 0x1p100f; }
+
+// ---- K: one lane per 8 values of a row, four rows in flight per lane --------
+struct KDeq {
+  const uint32_t* codes;
+  const uint16_t* meta;
+  const uint16_t* norm;
+  int64_t cap_blocks;
+  int H, t0, T, D, mode;
+  int lpr, lpr_sh;  // lanes per row, log2 where it is a power of two <= 256, else -1
+  int64_t tiles;    // workgroups per (batch, head)
+};
+constexpr int KU = 4;
+
+template <int BITS, int G, bool BF>
+__global__ __launch_bounds__(256) void dequant_k_kernel(KDeq a, DeqOut o) {
+  constexpr int LPG = G / 8, W = G * BITS / 32;
+  const int64_t bh = int64_t(blockIdx.x) / a.tiles, tile = int64_t(blockIdx.x) % a.tiles;
+  const int ng = a.D / G;
+  const bool fixed = a.lpr_sh >= 0;
+  int row[KU], c8[KU];
+  uint32_t w[KU];
+  float s[KU], z[KU];
+  int off[KU];
+#pragma unroll
+  for (int u = 0; u < KU; ++u) {
+    const int64_t e = (tile * KU + u) * 256 + threadIdx.x;
+    const int64_t r64 = fixed ? e >> a.lpr_sh : e / a.lpr;
+    row[u] = r64 < a.T ? int(r64) : a.T;  // a.T: past the end
+    c8[u] = fixed ? int(threadIdx.x) & (a.lpr - 1) : int(e - r64 * a.lpr);
+    if (row[u] < a.T) {
+      const int g = c8[u] / LPG, j = c8[u] % LPG, q = j & 3;
+      const int64_t tt = int64_t(a.t0) + row[u];
+      const int64_t unit = ((bh * a.cap_blocks + tt / TOKEN_BLOCK) * ng + g) * TOKEN_BLOCK + tt % TOKEN_BLOCK;
+      const int wi = BITS == 4 ? j : BITS == 3 ? (j >> 2) * 3 + (q < 3 ? q : 2) : BITS == 2 ? j >> 1 : j >> 2;
+      w[u] = a.codes[unit * W + wi];
+      unit_params<BF>(a.meta, unit, a.mode, BITS, s[u], z[u], off[u]);
+    }
+  }
+  float nf[8];
+  bool nt = true;
+  auto load_norm = [&](int c) {
+    const uint16_t* p = a.norm + bh * a.D + c * 8;
+    nt = true;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      nf[i] = act2f(p[i], BF);
+      nt = nt && tame(nf[i], 0.f);
+    }
+  };
+  if (a.norm && fixed) load_norm(c8[0]);
+#pragma unroll
+  for (int u = 0; u < KU; ++u) {
+    if (row[u] >= a.T) break;  // whole rows of lanes
+    const int j = c8[u] % LPG, q = j & 3;
+    // the lane's 8 fields: two runs of four, in the halves of y
+    uint32_t y;
+    if constexpr (BITS == 4) {
+      y = w[u];
+    } else if constexpr (BITS == 3) {  // 24 bits at 24 q of the quad's three words
+      const uint32_t pv = uint32_t(__builtin_amdgcn_mov_dpp(int(w[u]), 0x90, 0xf, 0xf, true));  // quad_perm [0,0,1,2]
+      const uint32_t b = __builtin_amdgcn_alignbit(w[u], pv, (32 - 8 * q) & 31);
+      y = (b & 0xfffu) | ((b << 4) & 0x0fff0000u);
+    } else if constexpr (BITS == 2) {
+      const uint32_t b = w[u] >> (16 * (j & 1));
+      y = (b & 0xffu) | ((b << 8) & 0x00ff0000u);
+    } else {
+      const uint32_t b = w[u] >> (8 * q);
+      y = (b & 0xfu) | ((b << 12) & 0x000f0000u);
+    }
+    const h2_t bias = bias_of(off[u], off[u]);
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const h2_t c = pair_at(y, BITS * i, ((1u << BITS) - 1u) * 0x10001u, bias);
+      v[i] = __builtin_fmaf(float(c.x), s[u], z[u]);  // quant.py:84-85 (c*s exact)
+      v[i + 4] = __builtin_fmaf(float(c.y), s[u], z[u]);
+    }
+    if (a.norm) {  // cache.py:132
+      if (!fixed) load_norm(c8[u]);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = __fmul_rn(v[i], nf[i]);
+    }
+    const int64_t at = (bh / a.H) * o.sob + (bh % a.H) * o.soh + int64_t(row[u]) * o.sot + c8[u] * 8;
+    if (o.out16) {
+      uint32_t p[4];
+      if (nt && tame(s[u], z[u])) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) p[i] = out_pair_num<BF>(v[2 * i], v[2 * i + 1]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) p[i] = out_pair<BF>(v[2 * i], v[2 * i + 1]);
+      }
+      if (o.vec16) {
+        *reinterpret_cast<uint4*>(o.out16 + at) = make_uint4(p[0], p[1], p[2], p[3]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o.out16[at + i] = uint16_t(p[i / 2] >> (16 * (i & 1)));
+      }
+    }
+    if (o.out32) {
+      if (o.vec32) {
+        *reinterpret_cast<f4_t*>(o.out32 + at) = f4_t{v[0], v[1], v[2], v[3]};
+        *reinterpret_cast<f4_t*>(o.out32 + at + 4) = f4_t{v[4], v[5], v[6], v[7]};
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o.out32[at + i] = v[i];
+      }
+    }
+  }
+}
+
+// ---- V: one thread per 4 columns of 32 tokens --------------------------------
+struct VDeq {
+  const uint32_t* codes;
+  const uint16_t* meta;
+  int64_t cap_groups;
+  int H, g0, D, mode;
+  int nch;        // 32-token chunks read
+  int dq;         // column quads per row, ceil(D / 4)
+  int64_t items;  // B * H * nch * dq
+};
+
+template <int BITS, int G, bool BF>
+__global__ __launch_bounds__(256) void dequant_v_kernel(VDeq a, DeqOut o) {
+  constexpr int W = G * BITS / 32, CPG = G / 32;  // chunks per group
+  constexpr int CH = 16 / BITS;                   // fields per half
+  const int64_t e = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (e >= a.items) return;
+  const int64_t r = e / a.dq;
+  const int d = int(e - r * a.dq) * 4;
+  const int64_t bh = r / a.nch;
+  const int k = int(r - bh * a.nch);
+  const int nd = min(4, a.D - d);
+  uint32_t w[4][BITS];
+  float s[4], z[4];
+  int off[4];
+  bool num = true;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const int64_t unit = (bh * a.cap_groups + a.g0 + k / CPG) * a.D + d + (c < nd ? c : 0);
+#pragma unroll
+    for (int i = 0; i < BITS; ++i) w[c][i] = a.codes[unit * W + (k % CPG) * BITS + i];
+    unit_params<BF>(a.meta, unit, a.mode, BITS, s[c], z[c], off[c]);
+    num = num && tame(s[c], z[c]);
+  }
+  const h2_t b01 = bias_of(off[0], off[1]), b23 = bias_of(off[2], off[3]);
+  const int64_t at = (bh / a.H) * o.sob + (bh % a.H) * o.soh + int64_t(k) * 32 * o.sot + d;
+  // fields of tokens [CH x, CH x + CH) of two columns, in the halves of a dword
+  auto halves = [](const uint32_t* p, const uint32_t* q, int x) {
+    if constexpr (BITS != 3) {
+      return __builtin_amdgcn_perm(q[x / 2], p[x / 2], x & 1 ? 0x07060302u : 0x05040100u);
+    } else {  // 15 bits at 15 x
+      const int wi = (15 * x) >> 5, sh = (15 * x) & 31;
+      uint32_t u = p[wi] >> sh, v = q[wi] >> sh;
+      if (sh > 17 && wi + 1 < BITS) {
+        u |= p[wi + 1] << (32 - sh);
+        v |= q[wi + 1] << (32 - sh);
+      }
+      return (u & 0x7fffu) | (v << 16);
+    }
+  };
+  constexpr uint32_t M = ((1u << BITS) - 1u) * 0x10001u;
+#pragma unroll
+  for (int x = 0; x * CH < 32; ++x) {
+    const uint32_t y01 = halves(w[0], w[1], x), y23 = halves(w[2], w[3], x);
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      const int t = x * CH + i;
+      if (t >= 32) break;
+      const h2_t c01 = pair_at(y01, BITS * i, M, b01), c23 = pair_at(y23, BITS * i, M, b23);
+      const float v[4] = {__builtin_fmaf(float(c01.x), s[0], z[0]), __builtin_fmaf(float(c01.y), s[1], z[1]),
+                          __builtin_fmaf(float(c23.x), s[2], z[2]), __builtin_fmaf(float(c23.y), s[3], z[3])};
+      const int64_t at_t = at + int64_t(t) * o.sot;
+      if (o.out16) {
+        uint32_t p0, p1;
+        if (num) { p0 = out_pair_num<BF>(v[0], v[1]); p1 = out_pair_num<BF>(v[2], v[3]); }
+        else { p0 = out_pair<BF>(v[0], v[1]); p1 = out_pair<BF>(v[2], v[3]); }
+        if (o.vec16) {
+          *reinterpret_cast<uint2*>(o.out16 + at_t) = make_uint2(p0, p1);
+        } else {
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+            if (c < nd) o.out16[at_t + c] = uint16_t((c < 2 ? p0 : p1) >> (16 * (c & 1)));
+        }
+      }
+      if (o.out32) {
+        if (o.vec32) {
+          *reinterpret_cast<f4_t*>(o.out32 + at_t) = f4_t{v[0], v[1], v[2], v[3]};
+        } else {
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+            if (c < nd) o.out32[at_t + c] = v[c];
+        }
+      }
+    }
+  }
+}
+
+}  // namespace
+
+extern "C" {
+
+int iq_dequant_k(const uint32_t* k_codes, const uint16_t* k_meta, int64_t t_cap, const void* norm, int B, int H,
+                 int t0, int T, int D, int group, int bits, int mode, void* out16, float* out32, int64_t so_b,
+                 int64_t so_h, int64_t so_t, void* stream) {
+  IQ_CHECK(k_codes && k_meta, IQ_ERR_NULL);
+  IQ_CHECK(out16 || out32, IQ_ERR_NULL);
+  const bool bf = act_bf16(mode);
+  mode = base_mode(mode);
+  if (int e = check_store(bits, group, mode)) return e;
+  IQ_CHECK(B >= 0 && H >= 0 && T >= 0 && t0 >= 0 && D > 0, IQ_ERR_SHAPE);
+  IQ_CHECK(D % group == 0, IQ_ERR_GROUP);
+  IQ_CHECK(t_cap % TOKEN_BLOCK == 0, IQ_ERR_ALIGN);
+  IQ_CHECK(int64_t(t0) + T <= t_cap, IQ_ERR_RANGE);
+  if (int64_t(B) * H * T == 0) return IQ_OK;
+  const bool s8 = so_b % 8 == 0 && so_h % 8 == 0 && so_t % 8 == 0, s4 = so_b % 4 == 0 && so_h % 4 == 0 && so_t % 4 == 0;
+  const DeqOut o{(uint16_t*)out16, out32, so_b, so_h, so_t, aligned(out16, 16) && s8, aligned(out32, 16) && s4};
+  const int lpr = D / 8;
+  const bool pow2 = (lpr & (lpr - 1)) == 0 && lpr <= 256;
+  const KDeq a{k_codes, k_meta, (const uint16_t*)norm, t_cap / TOKEN_BLOCK, H, t0, T, D, mode, lpr,
+               pow2 ? __builtin_ctz(unsigned(lpr)) : -1, ceil_div(int64_t(T) * lpr, 256 * KU)};
+  const dim3 grid(unsigned(int64_t(B) * H * a.tiles));
+  return dispatch_store_bits_group(bits, group, [&]<int BITS, int G>() {
+    auto* kern = bf ? dequant_k_kernel<BITS, G, true> : dequant_k_kernel<BITS, G, false>;
+    kern<<<grid, 256, 0, (hipStream_t)stream>>>(a, o);
+    return launch_status();
+  });
+}
+
+int iq_dequant_v(const uint32_t* v_codes, const uint16_t* v_meta, int64_t t_cap, int B, int H, int t0, int T,
+                 int D, int group, int bits, int mode, void* out16, float* out32, int64_t so_b, int64_t so_h,
+                 int64_t so_t, void* stream) {
+  IQ_CHECK(v_codes && v_meta, IQ_ERR_NULL);
+  IQ_CHECK(out16 || out32, IQ_ERR_NULL);
+  const bool bf = act_bf16(mode);
+  mode = base_mode(mode);
+  if (int e = check_store(bits, group, mode)) return e;
+  IQ_CHECK(B >= 0 && H >= 0 && T >= 0 && t0 >= 0 && D > 0, IQ_ERR_SHAPE);
+  IQ_CHECK(T % group == 0 && t0 % group == 0 && t_cap % group == 0, IQ_ERR_GROUP);
+  IQ_CHECK(int64_t(t0) + T <= t_cap, IQ_ERR_RANGE);
+  const int nch = T / 32, dq = (D + 3) / 4;
+  const int64_t items = int64_t(B) * H * nch * dq;
+  if (items == 0) return IQ_OK;
+  const bool s4 = D % 4 == 0 && so_b % 4 == 0 && so_h % 4 == 0 && so_t % 4 == 0;
+  const DeqOut o{(uint16_t*)out16, out32, so_b, so_h, so_t, aligned(out16, 8) && s4, aligned(out32, 16) && s4};
+  const VDeq a{v_codes, v_meta, t_cap / group, H, t0 / group, D, mode, nch, dq, items};
+  return dispatch_store_bits_group(bits, group, [&]<int BITS, int G>() {
+    auto* kern = bf ? dequant_v_kernel<BITS, G, true> : dequant_v_kernel<BITS, G, false>;
+    kern<<<dim3(unsigned(ceil_div(items, 256))), 256, 0, (hipStream_t)stream>>>(a, o);
+    return launch_status();
+  });
+}
+
+}  // extern "C"

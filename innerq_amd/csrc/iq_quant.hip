@@ -220,105 +220,6 @@ __device__ __forceinline__ void quant_group_rt(const float* v, int bits, int mod
   }
 }
 
-// ---- dequantization (dense read path) --------------------------------------
-struct DeqOut {
-  uint16_t* out16;  // in the activation dtype
-  float* out32;
-  int64_t sob, soh, sot;
-  int bf;           // bf16 activations: meta, norm and out16
-};
-
-__device__ __forceinline__ void put(const DeqOut& o, int64_t off, float v) {
-  if (o.out16) o.out16[off] = f2act(v, o.bf != 0);
-  if (o.out32) o.out32[off] = v;
-}
-
-// signed codes and {scale, zero} of one group such that value = c*s + z:
-// asym {s, z}; sym offset binary, z = 0; hybrid as the group's flag says
-// (quant.py:153-176: the sym codes where the mask is set)
-template <int BITS, int G>
-__device__ __forceinline__ void group_deq_params(const uint32_t* w, const uint16_t* meta, int64_t unit, int mode,
-                                                 bool bf, int32_t* c, float& s, float& z) {
-  unpack_fields<BITS, G>(w, mode == IQ_MODE_SYM, c);
-  z = 0.f;
-  if (mode == IQ_MODE_SYM) {
-    s = act2f(meta[unit], bf);
-    return;
-  }
-  const uint32_t mw = reinterpret_cast<const uint32_t*>(meta)[unit];
-  if (mode == IQ_MODE_HYBRID && hyb_sym(mw)) {
-#pragma unroll
-    for (int i = 0; i < G; ++i) c[i] -= 1 << (BITS - 1);
-    s = hyb_scale(mw, bf);
-    return;
-  }
-  s = mode == IQ_MODE_HYBRID ? hyb_scale(mw, bf) : act2f(uint16_t(mw & 0xffffu), bf);
-  z = act2f(uint16_t(mw >> 16), bf);
-}
-
-template <int BITS, int G>
-__global__ __launch_bounds__(256) void dequant_k_kernel(const uint32_t* __restrict__ kc,
-                                                        const uint16_t* __restrict__ km, int64_t cap_blocks,
-                                                        const uint16_t* __restrict__ norm, int B, int H, int t0,
-                                                        int T, int D, int mode, DeqOut o) {
-  constexpr int W = G * BITS / 32;
-  const int ng = D / G;
-  const int64_t gid = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int64_t total = int64_t(B) * H * T * ng;
-  if (gid >= total) return;
-  const int g = int(gid % ng);
-  int64_t r = gid / ng;
-  const int t = int(r % T);
-  r /= T;
-  const int h = int(r % H);
-  const int b = int(r / H);
-  const int64_t bh = int64_t(b) * H + h;
-  const int64_t tt = int64_t(t0) + t;
-  const int64_t unit = ((bh * cap_blocks + tt / TOKEN_BLOCK) * ng + g) * TOKEN_BLOCK + tt % TOKEN_BLOCK;
-  uint32_t w[W];
-#pragma unroll
-  for (int j = 0; j < W; ++j) w[j] = kc[unit * W + j];
-  int32_t c[G];
-  float s, z;
-  group_deq_params<BITS, G>(w, km, unit, mode, o.bf != 0, c, s, z);
-  const int64_t base = b * o.sob + h * o.soh + t * o.sot + g * G;
-#pragma unroll
-  for (int i = 0; i < G; ++i) {
-    float v = __fadd_rn(__fmul_rn(float(c[i]), s), z);       // quant.py:84-85 (c*s exact)
-    if (norm) v = __fmul_rn(v, act2f(norm[bh * D + g * G + i], o.bf != 0));  // cache.py:132
-    put(o, base + i, v);
-  }
-}
-
-template <int BITS, int G>
-__global__ __launch_bounds__(256) void dequant_v_kernel(const uint32_t* __restrict__ vc,
-                                                        const uint16_t* __restrict__ vm, int64_t cap_groups,
-                                                        int B, int H, int g0, int ngT, int D, int mode, DeqOut o) {
-  constexpr int W = G * BITS / 32;
-  const int64_t gid = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int64_t total = int64_t(B) * H * ngT * D;
-  if (gid >= total) return;
-  const int d = int(gid % D);
-  int64_t r = gid / D;
-  const int gi = int(r % ngT);
-  r /= ngT;
-  const int h = int(r % H);
-  const int b = int(r / H);
-  const int64_t bh = int64_t(b) * H + h;
-  const int64_t unit = (bh * cap_groups + g0 + gi) * D + d;
-  uint32_t w[W];
-#pragma unroll
-  for (int j = 0; j < W; ++j) w[j] = vc[unit * W + j];
-  int32_t c[G];
-  float s, z;
-  group_deq_params<BITS, G>(w, vm, unit, mode, o.bf != 0, c, s, z);
-#pragma unroll
-  for (int i = 0; i < G; ++i) {
-    const float v = __fadd_rn(__fmul_rn(float(c[i]), s), z);  // quant.py:90-91
-    put(o, b * o.sob + h * o.soh + (int64_t(gi) * G + i) * o.sot + d, v);
-  }
-}
-
 // ---- dense int32 codes -> values (the quant.py dequantize_* API) ----------
 // tensor [outer, n, inner] grouped along n; scale/zero [outer, n/G, inner];
 // signs [outer, n, inner].  op in fp32 (out_f16 = 0) or fp16 (out_f16 = 1),
@@ -655,49 +556,6 @@ int iq_v_store_bytes(int64_t B, int64_t H, int64_t t_cap, int64_t D, int group, 
   *codes_bytes = B * H * t_cap * D * bits / 8;
   *meta_bytes = B * H * (t_cap / group) * D * meta_unit_bytes(mode);
   return IQ_OK;
-}
-
-int iq_dequant_k(const uint32_t* k_codes, const uint16_t* k_meta, int64_t t_cap, const void* norm, int B, int H,
-                 int t0, int T, int D, int group, int bits, int mode, void* out16, float* out32, int64_t so_b,
-                 int64_t so_h, int64_t so_t, void* stream) {
-  IQ_CHECK(k_codes && k_meta, IQ_ERR_NULL);
-  IQ_CHECK(out16 || out32, IQ_ERR_NULL);
-  const bool bf = act_bf16(mode);
-  mode = base_mode(mode);
-  if (int e = check_store(bits, group, mode)) return e;
-  IQ_CHECK(B >= 0 && H >= 0 && T >= 0 && t0 >= 0 && D > 0, IQ_ERR_SHAPE);
-  IQ_CHECK(D % group == 0, IQ_ERR_GROUP);
-  IQ_CHECK(t_cap % TOKEN_BLOCK == 0, IQ_ERR_ALIGN);
-  IQ_CHECK(int64_t(t0) + T <= t_cap, IQ_ERR_RANGE);
-  const int64_t total = int64_t(B) * H * T * (D / group);
-  if (total == 0) return IQ_OK;
-  DeqOut o{(uint16_t*)out16, out32, so_b, so_h, so_t, bf ? 1 : 0};
-  return dispatch_store_bits_group(bits, group, [&]<int BITS, int G>() {
-    dequant_k_kernel<BITS, G><<<dim3(unsigned(ceil_div(total, 256))), 256, 0, (hipStream_t)stream>>>(
-        k_codes, k_meta, t_cap / TOKEN_BLOCK, (const uint16_t*)norm, B, H, t0, T, D, mode, o);
-    return launch_status();
-  });
-}
-
-int iq_dequant_v(const uint32_t* v_codes, const uint16_t* v_meta, int64_t t_cap, int B, int H, int t0, int T,
-                 int D, int group, int bits, int mode, void* out16, float* out32, int64_t so_b, int64_t so_h,
-                 int64_t so_t, void* stream) {
-  IQ_CHECK(v_codes && v_meta, IQ_ERR_NULL);
-  IQ_CHECK(out16 || out32, IQ_ERR_NULL);
-  const bool bf = act_bf16(mode);
-  mode = base_mode(mode);
-  if (int e = check_store(bits, group, mode)) return e;
-  IQ_CHECK(B >= 0 && H >= 0 && T >= 0 && t0 >= 0 && D > 0, IQ_ERR_SHAPE);
-  IQ_CHECK(T % group == 0 && t0 % group == 0 && t_cap % group == 0, IQ_ERR_GROUP);
-  IQ_CHECK(int64_t(t0) + T <= t_cap, IQ_ERR_RANGE);
-  const int64_t total = int64_t(B) * H * (T / group) * D;
-  if (total == 0) return IQ_OK;
-  DeqOut o{(uint16_t*)out16, out32, so_b, so_h, so_t, bf ? 1 : 0};
-  return dispatch_store_bits_group(bits, group, [&]<int BITS, int G>() {
-    dequant_v_kernel<BITS, G><<<dim3(unsigned(ceil_div(total, 256))), 256, 0, (hipStream_t)stream>>>(
-        v_codes, v_meta, t_cap / G, B, H, t0 / G, T / G, D, mode, o);
-    return launch_status();
-  });
 }
 
 int iq_dequant_dense(const int32_t* codes, const void* scale16, const void* zs16, int64_t outer, int64_t n,

@@ -1,0 +1,59 @@
+"""Dense reads of packed stores at the sizes where the kernels' tiles end: single tokens and block
+edges, ranges that start inside a block, head_dims whose rows do not divide a workgroup (K), odd
+column counts (V), and outputs whose rows do or do not take vector stores.  The values are defined
+bit for bit: fp32(c * s + z), times the factor in fp32, one rounding to the output type (oracle)."""
+import numpy as np
+import pytest
+import torch
+
+from innerq_amd import ops
+from oracle import quant_ref as Q
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+TD = {"f16": torch.float16, "bf16": torch.bfloat16}
+MODES = [("asymmetric", (1, 2, 3, 4)), ("symmetric", (2, 3, 4)), ("hybrid", (2, 3, 4))]
+FN = {(m, ax): (getattr(Q, f"quantize_{ax}dim_{s}"), getattr(Q, f"dequantize_{ax}dim_{s}"))
+      for m, s in (("asymmetric", "asym"), ("symmetric", "sym"), ("hybrid", "hybrid")) for ax in ("channel", "token")}
+
+
+def view(B, H, T, D, dtype, layout):
+    if layout == "plain":
+        return torch.zeros(B, H, T, D, dtype=dtype, device=DEV)
+    if layout == "inside":  # the slice that update() fills between sinks and window
+        return torch.zeros(B, H, T + 5, D, dtype=dtype, device=DEV)[:, :, 2:T + 2]
+    if layout == "heads last":
+        return torch.zeros(B, T, H, D, dtype=dtype, device=DEV).transpose(1, 2)
+    return torch.zeros(B, H, T, D + 1, dtype=dtype, device=DEV)[..., 1:]  # odd rows
+
+
+@pytest.mark.parametrize("act", ["f16", "bf16"])
+@pytest.mark.parametrize("mode,widths", MODES)
+@pytest.mark.parametrize("axis,n,t0,D,G,layout,norm", [
+    ("channel", 1, 0, 128, 32, "plain", False), ("channel", 65, 1, 64, 64, "inside", True),
+    ("channel", 130, 63, 96, 32, "heads last", True), ("channel", 513, 0, 128, 128, "odd rows", False),
+    ("channel", 33, 0, 384, 128, "inside", True), ("token", 32, 0, 128, 32, "plain", False),
+    ("token", 320, 64, 64, 64, "inside", False), ("token", 256, 128, 130, 128, "heads last", False),
+    ("token", 96, 32, 33, 32, "odd rows", False), ("token", 64, 0, 1, 64, "plain", False)])
+def test_dequant(act, mode, widths, axis, n, t0, D, G, layout, norm):
+    B, H = 2, 2
+    rng = np.random.default_rng(n + D + G)
+    x = torch.from_numpy(rng.standard_normal((B, H, n, D)).astype(np.float32)).to(TD[act])
+    xh = x.float().numpy() if act == "bf16" else x.numpy()
+    nf = torch.from_numpy(rng.uniform(0.2, 3.0, (B, H, 1, D)).astype(np.float32)).to(TD[act]) if norm else None
+    quant, deq = FN[mode, axis]
+    xq = xh
+    if norm:
+        xq = Q._div16(xh, nf.float().numpy() if act == "bf16" else nf.numpy(), act)
+    for bits in widths:
+        want = deq(*quant(xq, G, bits, act), G).astype(np.float32)
+        if norm:
+            want = want * nf.float().numpy()
+        want = want[:, :, t0:]
+        st = ops.PackedStore(axis, B, H, D, G, bits, mode, DEV, dtype=TD[act])
+        st.append(x.to(DEV), norm=None if nf is None else nf.to(DEV))
+        for dtype in (TD[act], torch.float32):
+            out = view(B, H, n - t0, D, dtype, layout)
+            st.dequant(t0, n - t0, out=out, norm=None if nf is None else nf.to(DEV))
+            ref = torch.from_numpy(np.ascontiguousarray(want)).to(dtype)
+            assert torch.equal(out.cpu(), ref)  # equal values: -0 == +0
