@@ -79,7 +79,12 @@ enum iq_mode {
    * bf16 model's tensors (LongBench/pred.py:240 loads the model in bf16).
    * The decode GEMVs and decode attention take fp16 only and refuse a
    * flagged store with IQ_ERR_MODE. */
-  IQ_MODE_BF16 = 0x100
+  IQ_MODE_BF16 = 0x100,
+  /* OR-ed into the mode of iq_quantize_k: the rows of the last 64-token block
+   * past t_off + n are written as zeros (codes and metadata), for a block of a
+   * store whose memory was never cleared.  Rows that hold tokens there would
+   * be lost: only for an append at the store's end. */
+  IQ_MODE_ZERO_TAIL = 0x200
 };
 
 /* ABI version (IQ_ABI_VERSION) and error names. */
@@ -170,7 +175,12 @@ int iq_unpack_v(const uint32_t* v_codes, const uint16_t* v_meta, int64_t t_cap, 
  * T tokens of k (fp16, element strides sk_b, sk_h, sk_t; D contiguous).
  * mode: 0, or IQ_MODE_BF16 for bf16 k and out16 (any other bit:
  * IQ_ERR_MODE).  Replaces key_states.abs().max(dim=-2).values.sqrt()
- * (cache.py:121-126). */
+ * (cache.py:121-126).  The _ws form splits each head's tokens over workgroups
+ * (partial maxima in the workspace, 16-byte aligned, then a second launch);
+ * the other reads a head by one workgroup.  The results are the same bits. */
+size_t iq_key_norm_workspace_bytes(int B, int H, int T, int D);
+int iq_key_norm_factor_ws(const void* k, int64_t sk_b, int64_t sk_h, int64_t sk_t, int B, int H, int T, int D,
+                          int mode, void* out16, void* workspace, size_t workspace_bytes, void* stream);
 int iq_key_norm_factor(const void* k, int64_t sk_b, int64_t sk_h, int64_t sk_t, int B, int H, int T, int D,
                        int mode, void* out16, void* stream);
 

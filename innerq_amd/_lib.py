@@ -16,6 +16,7 @@ IQ_MODE_ASYM = 0
 IQ_MODE_SYM = 1
 IQ_MODE_HYBRID = 2
 IQ_MODE_BF16 = 0x100  # OR-ed into a mode: bf16 activations
+IQ_MODE_ZERO_TAIL = 0x200  # OR-ed into iq_quantize_k's mode: zero the last block's rows past the tokens
 ABI_VERSION = 3
 TOKEN_BLOCK = 64
 
@@ -85,6 +86,8 @@ SIGNATURES = {
     "iq_dequant_dense": (I, [P, P, P, L, L, L, I, I, I, P, P]),
     "iq_unpack_k": (I, [P, P, L, I, I, I, I, I, I, I, I, P, P, P, P]),
     "iq_unpack_v": (I, [P, P, L, I, I, I, I, I, I, I, I, P, P, P, P]),
+    "iq_key_norm_workspace_bytes": (S, [I, I, I, I]),
+    "iq_key_norm_factor_ws": (I, [P, L, L, L, I, I, I, I, I, P, P, S, P]),
     "iq_key_norm_factor": (I, [P, L, L, L, I, I, I, I, I, P, P]),
     "iq_hybrid_mask": (I, [P, P, P, P, L, I, I, I, I, I, P, P]),
     "iq_hybrid_select": (I, [P, P, P, L, I, I, I, I, I, P, P]),

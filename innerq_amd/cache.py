@@ -207,8 +207,8 @@ class InnerqDynamicLayer(CacheLayerMixin):
         else:
             viable_recent_size_key = key_states.shape[-2]
         nq = key_states.shape[-2] - viable_recent_size_key
-        self.keys_recent = key_states[:, :, nq:, :].contiguous()
-        return key_states[:, :, :nq, :].contiguous()
+        self._kwin = ops.RecentWindow(key_states[:, :, nq:, :], front=self._front_rows(key_states)[0])
+        return key_states[:, :, :nq, :]
 
     def initialize_values_recent(self, value_states: torch.Tensor) -> torch.Tensor:
         if self.value_quantize:
@@ -219,8 +219,8 @@ class InnerqDynamicLayer(CacheLayerMixin):
         else:
             viable_recent_size_value = value_states.shape[-2]
         nq = value_states.shape[-2] - viable_recent_size_value
-        self.values_recent = value_states[:, :, nq:, :].contiguous()
-        return value_states[:, :, :nq, :].contiguous()
+        self._vwin = ops.RecentWindow(value_states[:, :, nq:, :], front=self._front_rows(value_states)[1])
+        return value_states[:, :, :nq, :]
 
     def _kq_for(self, like: torch.Tensor) -> _Quantized:
         if self._kq is None:
@@ -290,6 +290,21 @@ class InnerqDynamicLayer(CacheLayerMixin):
         """cache.py:341-365: quantize these values and append them."""
         self._quantize_values(value_states)
 
+    def _kept_rows(self, dtype) -> tuple[int, int]:
+        """How many rows before each role's window a move keeps (0: none are, see
+        _keep_dequantized_rows)."""
+        if not (self.key_quantize and not self.key_quantize_over_token and self.value_quantize
+                and self.value_quantize_over_token and dtype == torch.float16):
+            return 0, 0
+        k = self.value_w_recent + self.value_flush_size + 64 if self.key_group_size <= 64 else 0
+        v = self.key_w_recent + self.key_flush_size + self.value_group_size + 64 if self.value_group_size <= 64 else 0
+        return k, v
+
+    def _front_rows(self, like: torch.Tensor) -> tuple[int, int]:
+        """Room before each role's window for the rows a prefill leaves there."""
+        k, v = self._kept_rows(like.dtype)
+        return k, v + self.value_group_size if v else 0
+
     def _keep_dequantized_rows(self) -> None:
         """Tokens packed in one role while the other role still holds them in its
         window (K flushes token by token, V by groups of tokens) are attended as
@@ -301,26 +316,25 @@ class InnerqDynamicLayer(CacheLayerMixin):
         that boundary packed so far (window flushes keep them up).  fp16 layers:
         a bf16 row would hold the values 8 bits short of the fp32 dequantization
         that the packed reads give."""
-        if not (self.key_quantize and not self.key_quantize_over_token and self.value_quantize
-                and self.value_quantize_over_token and self.dtype == torch.float16):
-            return
+        kkeep, vkeep = self._kept_rows(self.dtype)
         kq = self._kq.length if self._kq is not None else 0
         vq = self._vq.length if self._vq is not None else 0
         e = self._packed_end()
         kend, vend = self.keys_sink.shape[-2] + kq, self.values_sink.shape[-2] + vq
-        if self._kwin is not None and self.key_group_size <= 64:
-            keep = self.value_w_recent + self.value_flush_size + 64
-            p = min(kend - e, keep) if e is not None else 0
-            pre = self._kq.store.dequant(kq - p, p, norm=self.key_normalization_factor) if p > 0 else None
-            self._kwin = ops.RecentWindow(self._kwin.tensor, pre=pre, deq_rows=True, keep=keep)
-        if self._vwin is not None and self.value_group_size <= 64:
-            keep = self.key_w_recent + self.key_flush_size + self.value_group_size + 64
-            p = min(vend - e, keep) if e is not None else 0
-            pre = None
-            if p > 0:  # dequantized by whole groups, the last p rows kept
-                t0 = (vq - p) // self.value_group_size * self.value_group_size
-                pre = self._vq.store.dequant(t0, vq - t0)[:, :, vq - t0 - p:]
-            self._vwin = ops.RecentWindow(self._vwin.tensor, pre=pre, deq_rows=True, keep=keep)
+        for role, keep, q, nq, end, norm in (("_kwin", kkeep, self._kq, kq, kend, self.key_normalization_factor),
+                                             ("_vwin", vkeep, self._vq, vq, vend, None)):
+            win = getattr(self, role)
+            if win is None or not keep:
+                continue
+            p = min(end - e, keep) if e is not None else 0
+            # dequantized in place, by whole groups along tokens; the last p rows count
+            t0 = nq - p if q is None or q.axis == "channel" else (nq - p) // q.group * q.group
+            if win.rows_into(nq - t0) is None:  # a window without that room in front
+                win = ops.RecentWindow(win.tensor, front=nq - t0)
+                setattr(self, role, win)
+            if p > 0:
+                q.store.dequant(t0, nq - t0, out=win.rows_into(nq - t0), norm=norm)
+            win.deq_rows, win.keep, win.shadow = True, keep, p
 
     def _packed_end(self) -> Optional[int]:
         """The token where a decode's packed segments of both roles end: the end of

@@ -27,22 +27,28 @@ __global__ __launch_bounds__(256) void key_norm_kernel(const uint16_t* __restric
   out[i] = f2act(__fsqrt_rn(act2f(uint16_t(mx), bf != 0)), bf != 0);
 }
 
-// The same factor for head_dim 64 and 128 (the prompt lengths of a prefill):
-// one 1024-thread workgroup per (batch, head); thread (token lane tl,
-// 8-channel group cg) reads 16 bytes of every TL-th row, so a wave reads
-// whole rows.  |x| of fp16 and bf16 values orders like its bit pattern with
+// The same factor for head_dim 64 and 128 (the prompt lengths of a prefill).
+// Bound: HBM (it reads the keys once).  1024-thread workgroups, grid.y slices
+// of `rows` tokens per (batch, head); thread (token lane tl, 8-channel group
+// cg) reads 16 bytes of every TL-th row, so a wave reads whole rows.  With
+// one slice the workgroup writes the factor; with more (FINAL = false) it
+// writes its slice's maxima as bit patterns [bh, slice, D], over which a
+// second launch runs as over keys.  One workgroup per head left most of the
+// device idle at 4 x 8 heads x 8062 tokens: 35 us, now 15 + 4.  |x| of fp16 and bf16 values orders like its bit pattern with
 // the sign bit cleared (a NaN above every number, as torch's max propagates
 // it), so the maximum is a packed 16-bit integer max, exact in any order;
-// the token lanes' maxima meet in LDS.  One thread per channel walked the
-// tokens one row at a time: 13.2 ms for a 32k-token prompt of 8 x 8 heads.
-template <int D>
+// the token lanes' maxima meet in LDS.  (One thread per channel walked the
+// tokens one row at a time: 13.2 ms for a 32k-token prompt of 8 x 8 heads.)
+template <int D, bool FINAL>
 __global__ __launch_bounds__(1024) void key_norm_rows_kernel(const uint16_t* __restrict__ k, int64_t skb,
-                                                             int64_t skh, int64_t skt, int H, int T, int bf,
-                                                             int vec, uint16_t* __restrict__ out) {
-  constexpr int CG = D / 8, TL = 1024 / CG;
-  __shared__ uint4 red[TL][CG];
+                                                             int64_t skh, int64_t skt, int H, int T, int rows,
+                                                             int bf, int vec, uint16_t* __restrict__ out) {
+  constexpr int CG = D / 8, TL = 1024 / CG, NW = 1024 / 64;
+  __shared__ uint4 red[NW][CG];
   const int bh = blockIdx.x, tid = threadIdx.x, cg = tid % CG, tl = tid / CG;
-  const uint16_t* p = k + int64_t(bh / H) * skb + int64_t(bh % H) * skh + cg * 8;
+  const int t0 = blockIdx.y * rows;
+  T = min(T - t0, rows);
+  const uint16_t* p = k + int64_t(bh / H) * skb + int64_t(bh % H) * skh + t0 * skt + cg * 8;
   uint32_t m[4] = {0u, 0u, 0u, 0u};  // |x| bit patterns, two channels per dword
   auto fold = [&](const uint32_t (&w)[4]) {
 #pragma unroll
@@ -53,17 +59,14 @@ __global__ __launch_bounds__(1024) void key_norm_rows_kernel(const uint16_t* __r
     }
   };
   if (vec) {
-    int t = tl;
-    for (; t + 3 * TL < T; t += 4 * TL) {  // four rows in flight per thread
+    // four rows in flight per thread; past the end the last row again (a
+    // maximum does not mind)
+    for (int t = tl; t < T; t += 4 * TL) {
       uint4 r[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) r[u] = *reinterpret_cast<const uint4*>(p + int64_t(t + u * TL) * skt);
+      for (int u = 0; u < 4; ++u) r[u] = *reinterpret_cast<const uint4*>(p + int64_t(min(t + u * TL, T - 1)) * skt);
 #pragma unroll
       for (int u = 0; u < 4; ++u) fold({r[u].x, r[u].y, r[u].z, r[u].w});
-    }
-    for (; t < T; t += TL) {
-      const uint4 r = *reinterpret_cast<const uint4*>(p + int64_t(t) * skt);
-      fold({r.x, r.y, r.z, r.w});
     }
   } else {
     for (int t = tl; t < T; t += TL) {
@@ -74,18 +77,54 @@ __global__ __launch_bounds__(1024) void key_norm_rows_kernel(const uint16_t* __r
       fold(w);
     }
   }
-  red[tl][cg] = make_uint4(m[0], m[1], m[2], m[3]);
+  // the wave's token lanes first (lanes of one channel group are CG apart)
+#pragma unroll
+  for (int x = CG; x < 64; x <<= 1) {
+    uint32_t w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[j] = uint32_t(__shfl_xor(int(m[j]), x, 64));
+    fold(w);
+  }
+  if ((tid & 63) < CG) red[tid >> 6][cg] = make_uint4(m[0], m[1], m[2], m[3]);
   __syncthreads();
   if (tid < D) {  // channel d = tid: its token lanes' maxima
     const int c = tid / 8, j = (tid % 8) / 2, hi = tid % 2;
     uint32_t mx = 0u;
-    for (int r = 0; r < TL; ++r) {
+#pragma unroll
+    for (int r = 0; r < NW; ++r) {
       const uint4 v = red[r][c];
       const uint32_t w = j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w;
       mx = max(mx, hi ? w >> 16 : w & 0xffffu);
     }
-    out[int64_t(bh) * D + tid] = f2act(__fsqrt_rn(act2f(uint16_t(mx), bf != 0)), bf != 0);
+    out[(int64_t(bh) * gridDim.y + blockIdx.y) * D + tid] =
+        FINAL ? f2act(__fsqrt_rn(act2f(uint16_t(mx), bf != 0)), bf != 0) : uint16_t(mx);
   }
+}
+
+// slices per head: enough workgroups for two per CU, at least 256 rows (the
+// pass of a workgroup at D = 128 with four rows per thread) each
+int norm_slices(int64_t bh, int T) {
+  const int64_t want = ceil_div(512, bh > 0 ? bh : 1), most = ceil_div(T, 256);
+  return int(want < 1 ? 1 : want < most ? want : most);
+}
+
+template <int D>
+int launch_key_norm(const uint16_t* k, int64_t sk_b, int64_t sk_h, int64_t sk_t, int B, int H, int T, int bf,
+                    uint16_t* out, uint16_t* ws, hipStream_t st) {
+  // 16-byte row loads where every row's channels start 16-byte aligned
+  const int vec = aligned(k, 16) && sk_b % 8 == 0 && sk_h % 8 == 0 && sk_t % 8 == 0;
+  const unsigned bh = unsigned(int64_t(B) * H);
+  constexpr int PASS = 4 * 1024 / (D / 8);  // rows of one pass of a workgroup
+  const int want = ws ? norm_slices(bh, T) : 1;
+  const int rows = int(ceil_div(ceil_div(T, want), PASS)) * PASS, S = int(ceil_div(T, rows));
+  if (S == 1) {
+    key_norm_rows_kernel<D, true><<<dim3(bh), 1024, 0, st>>>(k, sk_b, sk_h, sk_t, H, T, T, bf, vec, out);
+    return launch_status();
+  }
+  key_norm_rows_kernel<D, false><<<dim3(bh, S), 1024, 0, st>>>(k, sk_b, sk_h, sk_t, H, T, rows, bf, vec, ws);
+  key_norm_rows_kernel<D, true><<<dim3(bh), 1024, 0, st>>>(ws, int64_t(H) * S * D, int64_t(S) * D, D, H, S, S, bf, 1,
+                                                            out);
+  return launch_status();
 }
 
 // Hybrid selection mask (quant.py:133-151): per group, the L1 error of the
@@ -167,8 +206,15 @@ int check_hybrid(int64_t BH, int T, int D, int group, int axis) {
 
 extern "C" {
 
-int iq_key_norm_factor(const void* k, int64_t sk_b, int64_t sk_h, int64_t sk_t, int B, int H, int T, int D,
-                       int mode, void* out16, void* stream) {
+size_t iq_key_norm_workspace_bytes(int B, int H, int T, int D) {
+  if (B <= 0 || H <= 0 || T <= 0 || (D != 64 && D != 128)) return 0;
+  const int64_t bh = int64_t(B) * H;
+  const int S = norm_slices(bh, T);
+  return S > 1 ? size_t(bh) * S * D * 2 : 0;
+}
+
+int iq_key_norm_factor_ws(const void* k, int64_t sk_b, int64_t sk_h, int64_t sk_t, int B, int H, int T, int D,
+                          int mode, void* out16, void* workspace, size_t workspace_bytes, void* stream) {
   IQ_CHECK(k && out16, IQ_ERR_NULL);
   IQ_CHECK(base_mode(mode) == 0, IQ_ERR_MODE);  // only the dtype flag
   IQ_CHECK(B >= 0 && H >= 0 && T > 0 && D > 0, IQ_ERR_SHAPE);
@@ -176,20 +222,20 @@ int iq_key_norm_factor(const void* k, int64_t sk_b, int64_t sk_h, int64_t sk_t, 
   if (n == 0) return IQ_OK;
   const int bf = act_bf16(mode) ? 1 : 0;
   if (D == 64 || D == 128) {
-    // 16-byte row loads where every row's channels start 16-byte aligned
-    const int vec = aligned(k, 16) && sk_b % 8 == 0 && sk_h % 8 == 0 && sk_t % 8 == 0;
-    const dim3 grid{unsigned(int64_t(B) * H)};
-    if (D == 128)
-      key_norm_rows_kernel<128><<<grid, 1024, 0, (hipStream_t)stream>>>((const uint16_t*)k, sk_b, sk_h, sk_t, H, T,
-                                                                         bf, vec, (uint16_t*)out16);
-    else
-      key_norm_rows_kernel<64><<<grid, 1024, 0, (hipStream_t)stream>>>((const uint16_t*)k, sk_b, sk_h, sk_t, H, T,
-                                                                        bf, vec, (uint16_t*)out16);
-    return launch_status();
+    IQ_CHECK(!workspace || workspace_bytes >= iq_key_norm_workspace_bytes(B, H, T, D), IQ_ERR_WORKSPACE);
+    IQ_CHECK(aligned(workspace, 16), IQ_ERR_ALIGN);
+    auto* go = D == 128 ? launch_key_norm<128> : launch_key_norm<64>;
+    return go((const uint16_t*)k, sk_b, sk_h, sk_t, B, H, T, bf, (uint16_t*)out16, (uint16_t*)workspace,
+              (hipStream_t)stream);
   }
   key_norm_kernel<<<dim3(unsigned(ceil_div(n, 256))), 256, 0, (hipStream_t)stream>>>(
       (const uint16_t*)k, sk_b, sk_h, sk_t, H, T, D, n, bf, (uint16_t*)out16);
   return launch_status();
+}
+
+int iq_key_norm_factor(const void* k, int64_t sk_b, int64_t sk_h, int64_t sk_t, int B, int H, int T, int D,
+                       int mode, void* out16, void* stream) {
+  return iq_key_norm_factor_ws(k, sk_b, sk_h, sk_t, B, H, T, D, mode, out16, nullptr, 0, stream);
 }
 
 int iq_hybrid_mask(const void* x16, const void* norm16, const float* deq_a, const float* deq_s, int64_t BH, int T,

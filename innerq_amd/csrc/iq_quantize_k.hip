@@ -11,6 +11,7 @@ struct KArgs {
   int64_t sxb, sxh, sxt;
   const uint16_t* norm;  // [B,H,D] key normalization factor, or null
   int H, n, D;
+  int n_pad;             // rows written: n, or up to the block's end (the rest as zeros)
   int lpr, lpr_sh;       // lanes (8 values each) per row, and its log2 where it is a power of two <= 256, else -1
   int64_t tiles;         // workgroups per (batch, head)
 };
@@ -38,14 +39,14 @@ __device__ __forceinline__ NormRegs load_norm(const uint16_t* p) {
   for (int i = 0; i < 8; ++i) {
     q.n[i] = act2f(p[i], BF);
     q.ok = q.ok && (BF ? q.n[i] >= 0x1p-60f && q.n[i] <= 0x1p60f : q.n[i] > 0.f && q.n[i] < INFINITY);
-    q.r[i] = __fdiv_rn(1.0f, q.n[i]);
+    q.r[i] = BF ? __builtin_amdgcn_rcpf(q.n[i]) : __fdiv_rn(1.0f, q.n[i]);
   }
   return q;
 }
 // x / factor rounded to the activation type (cache.py:125), packed.  fp16:
 // the exact division step.  bf16: an 8-bit quotient is never closer to a
-// rounding boundary than 2^-17, so one multiplication rounds alike wherever
-// the result is normal: every |x| is 0 or at least 2^-60 (else per value).
+// rounding boundary than 2^-17, so one multiplication (by a reciprocal within
+// one ulp) rounds alike wherever the result is normal: every |x| is 0 or at least 2^-60 (else per value).
 template <bool BF>
 __device__ __forceinline__ void normalize(uint32_t (&w)[4], const NormRegs& q) {
   bool ok = q.ok;
@@ -321,7 +322,8 @@ __device__ __forceinline__ void quant_k8(uint32_t (&w)[4], int j, const QuantOut
 // A thread per group, the form before, read 64 B per lane at a 64 B stride and
 // spent ~25 instructions a value.  PackedStore.append of 8 x 8 heads x 32768
 // tokens, 4-bit asym G = 32 (537 MB read, 168 MB written): 180 -> 161 us a
-// call, of which ~25 us clear the new store.
+// call (kernel 184 -> 134 us, 5.3 TB/s), 136 once it no longer clears the
+// whole new store first.
 constexpr int KU = 4;  // loads in flight per lane
 template <int BITS, int G, int MODE, bool BF>
 __global__ __launch_bounds__(256) void quant_k_kernel(KArgs a, QuantOut o) {
@@ -347,14 +349,23 @@ __global__ __launch_bounds__(256) void quant_k_kernel(KArgs a, QuantOut o) {
   const int ng = a.D / G;
 #pragma unroll
   for (int u = 0; u < KU; ++u) {
-    if (row[u] >= a.n) break;  // whole groups of lanes
+    if (row[u] >= a.n_pad) break;  // whole groups of lanes
+    const int g = c8[u] / LPG, j = c8[u] % LPG;
+    const int64_t tt = o.t_off + row[u];
+    const int64_t unit = ((bh * o.cap_units + tt / TOKEN_BLOCK) * ng + g) * TOKEN_BLOCK + tt % TOKEN_BLOCK;
+    if (row[u] >= a.n) {  // the block's rows past the tokens
+      constexpr int W = G * BITS / 32;
+      if (j < W) o.codes[unit * W + j] = 0u;
+      if (j == 0) {
+        if constexpr (MODE == IQ_MODE_SYM) o.meta[unit] = 0;
+        else reinterpret_cast<uint32_t*>(o.meta)[unit] = 0u;
+      }
+      continue;
+    }
     if (a.norm) {
       if (!fixed) nr = load_norm<BF>(a.norm + bh * a.D + c8[u] * 8);
       normalize<BF>(w[u], nr);
     }
-    const int g = c8[u] / LPG, j = c8[u] % LPG;
-    const int64_t tt = o.t_off + row[u];
-    const int64_t unit = ((bh * o.cap_units + tt / TOKEN_BLOCK) * ng + g) * TOKEN_BLOCK + tt % TOKEN_BLOCK;
     const int64_t r = bh * a.n + row[u];
     quant_k8<BITS, G, MODE, BF>(w[u], j, o, unit, r * a.D + c8[u] * 8, r * ng + g);
   }
@@ -374,8 +385,8 @@ int iq_quantize_k(const void* x, int64_t sx_b, int64_t sx_h, int64_t sx_t, const
                   int64_t t_cap, int64_t t_off, int32_t* codes_i32, void* scale16, void* zero16, void* signs16,
                   void* stream) {
   IQ_CHECK(x, IQ_ERR_NULL);
-  const bool bf = act_bf16(mode);
-  mode = base_mode(mode);
+  const bool bf = act_bf16(mode), zero_tail = (mode & IQ_MODE_ZERO_TAIL) != 0;
+  mode = base_mode(mode) & ~int(IQ_MODE_ZERO_TAIL);
   if (int e = check_store(bits, group, mode)) return e;
   IQ_CHECK(B >= 0 && H >= 0 && n >= 0 && D > 0, IQ_ERR_SHAPE);
   IQ_CHECK(D % group == 0, IQ_ERR_GROUP);
@@ -395,8 +406,9 @@ int iq_quantize_k(const void* x, int64_t sx_b, int64_t sx_h, int64_t sx_t, const
              (uint16_t*)signs16};
   const int lpr = D / 8;
   const bool pow2 = (lpr & (lpr - 1)) == 0 && lpr <= 256;
-  KArgs a{(const uint16_t*)x, sx_b, sx_h, sx_t, (const uint16_t*)norm, H, n, D, lpr,
-          pow2 ? __builtin_ctz(unsigned(lpr)) : -1, ceil_div(int64_t(n) * lpr, 256 * KU)};
+  const int pad = zero_tail && k_codes ? int((TOKEN_BLOCK - (t_off + n) % TOKEN_BLOCK) % TOKEN_BLOCK) : 0;
+  KArgs a{(const uint16_t*)x, sx_b, sx_h, sx_t, (const uint16_t*)norm, H, n, D, n + pad, lpr,
+          pow2 ? __builtin_ctz(unsigned(lpr)) : -1, ceil_div(int64_t(n + pad) * lpr, 256 * KU)};
   return dispatch_format(bits, group, mode, [&]<int BITS, int G, int MODE>() {
     const int64_t blocks = int64_t(B) * H * a.tiles;
     return bf ? launch_k<BITS, G, MODE, true>(a, o, blocks, (hipStream_t)stream)

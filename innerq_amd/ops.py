@@ -214,26 +214,35 @@ class PackedStore:
 
     def reserve(self, n_tokens: int) -> None:
         """Ensure capacity for ``n_tokens`` tokens (amortized doubling; old data is kept)."""
+        self._grow(n_tokens, self.t_cap)
+
+    def _grow(self, n_tokens: int, written: int) -> bool:
+        """reserve(), whose caller then writes the new units of tokens [length, written) before
+        anything reads them (an append's): those units are not cleared.  True if the store grew."""
         u = self.unit
         need = -(-max(n_tokens, 0) // u) * u
         if need <= self.t_cap:
-            return
+            return False
         new_cap = max(need, 2 * self.t_cap, 4 * u)
         new_cap = -(-new_cap // u) * u
         cb, mb = self._bytes(new_cap)
         codes = torch.empty(cb // 4, dtype=torch.int32, device=self.device)
         meta = torch.empty(mb // 2, dtype=torch.int16, device=self.device)
         # new capacity starts zeroed: the rows of a partly filled 64-token K block
-        # past ``length`` are never written by a quantize, and to_bytes() ships the
-        # whole block, so they must not carry stale device memory
+        # past ``length`` are never written by a quantize (but an append's own, which
+        # clears its last block's rest), and to_bytes() ships the whole block, so they
+        # must not carry stale device memory
         ou, nu, bh = self.t_cap // u, new_cap // u, self.B * self.H
         cv, mv = codes.view(bh, nu, -1), meta.view(bh, nu, -1)
         if ou:
             cv[:, :ou].copy_(self.codes.view(bh, ou, -1))
             mv[:, :ou].copy_(self.meta.view(bh, ou, -1))
-        cv[:, ou:].zero_()
-        mv[:, ou:].zero_()
+        zu = max(ou, -(-written // u))
+        if zu < nu:
+            cv[:, zu:].zero_()
+            mv[:, zu:].zero_()
         self.codes, self.meta, self.t_cap = codes, meta, new_cap
+        return True
 
     def batch_view(self, b0: int, b1: int) -> "PackedStore":
         """Sequences [b0, b1) of this store as a store of B = b1 - b0 that shares its
@@ -362,7 +371,21 @@ class PackedStore:
             _shape_error(f"append: a token-grouped store takes whole groups of {self.group} tokens, got {n}")
         if n == 0:
             return
-        self.reserve(self.length + n)
+        grew = self._grow(self.length + n, self.length + n)
+        try:
+            self._quantize(x, norm, _lib.IQ_MODE_ZERO_TAIL if grew else 0)
+        except BaseException:
+            if grew:  # the new units were never written
+                used = -(-self.length // self.unit)
+                self.codes.view(B * H, self.t_cap // self.unit, -1)[:, used:].zero_()
+                self.meta.view(B * H, self.t_cap // self.unit, -1)[:, used:].zero_()
+            raise
+        self.length += n
+
+    def _quantize(self, x: torch.Tensor, norm: Optional[torch.Tensor], tail: int) -> None:
+        """Tokens x quantized into the store's rows from ``length`` on (K: ``tail`` may ask for the
+        rest of the last block to be cleared)."""
+        B, H, n, D = x.shape
         if self.axis == "channel":
             if x.stride(-1) != 1 or x.data_ptr() % 16 or any(s % 8 for s in x.stride()[:3]):
                 x = x.contiguous()
@@ -370,15 +393,14 @@ class PackedStore:
                 require_device(norm, "norm", self.dtype)
                 norm = norm.reshape(B, H, D).contiguous()
             call("iq_quantize_k", _p(x), x.stride(0), x.stride(1), x.stride(2), _p(norm), B, H, n, D, self.group,
-                 self.bits, self.mode_arg, _p(self.codes), _p(self.meta), self.t_cap, self.length, None, None, None,
-                 None, _stream(x.device))
+                 self.bits, self.mode_arg | tail, _p(self.codes), _p(self.meta), self.t_cap, self.length, None, None,
+                 None, None, _stream(x.device))
         else:
             if x.stride(-1) != 1:
                 x = x.contiguous()
             call("iq_quantize_v", _p(x), x.stride(0), x.stride(1), x.stride(2), B, H, n, D, self.group, self.bits,
                  self.mode_arg, _p(self.codes), _p(self.meta), self.t_cap, self.length, None, None, None, None,
                  _stream(x.device))
-        self.length += n
 
     # --- reads --------------------------------------------------------------
     def dequant(self, t0: int = 0, T: Optional[int] = None, out: Optional[torch.Tensor] = None,
@@ -423,19 +445,25 @@ class RecentWindow:
     activation dtype): the ``shadow`` rows before ``start`` are the tokens
     just before the window, as update() returns them (at most ``keep`` of them
     survive a move to a larger buffer).  A view taken earlier then sees its
-    flushed rows change to those values."""
+    flushed rows change to those values.  ``front`` leaves room for that many
+    rows before the window (rows_into())."""
 
     def __init__(self, x: torch.Tensor, pre: Optional[torch.Tensor] = None, deq_rows: bool = False,
-                 keep: int = 0):
+                 keep: int = 0, front: int = 0):
         require_act(x, "recent window")
         B, H, n, D = x.shape
         p = 0 if pre is None else pre.shape[2]
-        self.buf = torch.empty(B, H, max(2 * (n + p), n + p + 64), D, dtype=x.dtype, device=x.device)
+        f = max(front, p)
+        self.buf = torch.empty(B, H, max(2 * n + f + p, n + f + 64), D, dtype=x.dtype, device=x.device)
         if p:
-            self.buf[:, :, :p].copy_(pre)
-        self.buf[:, :, p:p + n].copy_(x)
-        self.start, self.n = p, n
+            self.buf[:, :, f - p:f].copy_(pre)
+        self.buf[:, :, f:f + n].copy_(x)
+        self.start, self.n = f, n
         self.deq_rows, self.keep, self.shadow = deq_rows, keep, p
+
+    def rows_into(self, p: int) -> Optional[torch.Tensor]:
+        """The p rows before the window, to be written (None: no room for them)."""
+        return self.buf[:, :, self.start - p:self.start] if p <= self.start else None
 
     @property
     def tensor(self) -> torch.Tensor:
@@ -827,8 +855,10 @@ def key_norm_factor(k: torch.Tensor) -> torch.Tensor:
         k = k.contiguous()
     B, H, T, D = k.shape
     out = torch.empty(B, H, 1, D, dtype=k.dtype, device=k.device)
-    call("iq_key_norm_factor", _p(k), k.stride(0), k.stride(1), k.stride(2), B, H, T, D, act_flag(k.dtype), _p(out),
-         _stream(k.device))
+    nbytes = _lib.lib().iq_key_norm_workspace_bytes(B, H, T, D)
+    ws = _workspace(k.device, nbytes) if nbytes else None
+    call("iq_key_norm_factor_ws", _p(k), k.stride(0), k.stride(1), k.stride(2), B, H, T, D, act_flag(k.dtype),
+         _p(out), _p(ws), ws.numel() if nbytes else 0, _stream(k.device))
     return out
 
 

@@ -128,3 +128,41 @@ def test_values(act, mode, widths, groups, D, G, off, layout):
         np.testing.assert_array_equal(got, fields)
         gm = st.meta.cpu().numpy().view(np.uint16).reshape(B, H, -1, D, M)[:, :, off:off + groups]
         assert same_meta(gm, meta, act)
+
+
+@pytest.mark.parametrize("n,t0", [(1, 0), (65, 0), (30, 50), (64, 0)])
+@pytest.mark.parametrize("mode", ["asymmetric", "symmetric"])
+def test_appended_store_clears_its_last_block(mode, n, t0):
+    """A store that an append made or grew is not cleared as a whole: the append clears the rows of
+    its last 64-token block past the tokens, here over memory that held other values."""
+    B, H, D = 2, 3, 128
+    poison = [torch.full((1 << 20,), -1, dtype=torch.int32, device=DEV) for _ in range(8)]
+    del poison
+    st = ops.PackedStore("channel", B, H, D, 32, 3, mode, DEV)
+    x = torch.randn(B, H, t0 + n, D, device=DEV).half()
+    if t0:
+        st.append(x[:, :, :t0])
+    st.append(x[:, :, t0:])
+    T, nb = t0 + n, st.t_cap // 64
+    codes = st.codes.view(B * H, nb, D // 32, 64, -1).transpose(2, 3).reshape(B * H, nb * 64, -1)
+    meta = st.meta.view(B * H, nb, D // 32, 64, -1).transpose(2, 3).reshape(B * H, nb * 64, -1)
+    assert int((codes[:, T:] != 0).sum()) == 0 and int((meta[:, T:] != 0).sum()) == 0
+    assert bool((meta[:, :T] != 0).any())
+
+
+@pytest.mark.parametrize("act", ["f16", "bf16"])
+@pytest.mark.parametrize("D,T,strided", [(128, 1, False), (128, 255, True), (128, 257, False), (64, 513, True),
+                                         (64, 4099, False), (128, 2049, True)])
+def test_key_norm_slices(act, D, T, strided):
+    """The factor over one slice, whole slices and ragged ones, against numpy (exact: one square root)."""
+    k = torch.randn(2, 3, T, D, device=DEV).to(TD[act])
+    k[0, 0, T - 1, 3] = 40.0
+    k[1, 2, T // 2, 5] = -50.0
+    k[1, 1, 0, 7] = float("nan")
+    top = k.cpu().abs().max(dim=-2, keepdim=True).values.float().numpy()
+    root = np.sqrt(top)  # correctly rounded in fp32, then to the type
+    want = torch.from_numpy(root.astype(np.float16) if act == "f16" else Q.round_bf16(root)).to(TD[act])
+    x = k.transpose(1, 2).contiguous().transpose(1, 2) if strided else k
+    got = ops.key_norm_factor(x).cpu()
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(got.nan_to_num(0.0), want.nan_to_num(0.0))
