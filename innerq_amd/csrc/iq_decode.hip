@@ -4,10 +4,11 @@
 // The token axis is cut into
 //   * the fused range: tokens packed in both the K and the V store (the
 //     middle segment of cache.py:235-276 for both), in splits of
-//     flash_split_tokens() tokens.  When K and V share their group size (bit
-//     widths may differ), one persistent kernel runs QK^T, the softmax and
-//     attn.V over every split (iq_flash.h) and writes one partial per run of
-//     splits.  Otherwise QK^T runs with its flash epilogue (per split max m,
+//     flash_split_tokens() tokens.  One persistent kernel runs QK^T, the
+//     softmax and attn.V over every split (iq_flash.h; bit widths may differ,
+//     and in fp16 layers of asym or sym stores the group sizes too) and writes
+//     one partial per run of splits.  Otherwise (a hybrid V of another group
+//     size, stores past 32-bit offsets) QK^T runs with its flash epilogue (per split max m,
 //     sum l and fp16 probabilities written as attn.V operand records), then
 //     attn.V writes one unnormalized partial output per split;
 //   * the dense tokens: everything else (fp16 sinks and recent windows, plus
@@ -945,15 +946,18 @@ int launch_splits(const void* q, int64_t sq_b, int64_t sq_h, const void* norm, c
                               k[1].mode};
   const detail::FusedStore fv{v[1].codes, v[1].meta, v[1].t_cap, v[1].t0 + (a0 - vs), v[1].bits, v[1].group,
                               v[1].mode};
-  const bool fused =
-      c && k[1].group == v[1].group && detail::flash_fused_supported(q, sq_b, sq_h, norm, fk, fv, Hq, Hkv, D);
+  // K and V of different group sizes: fp16 layers, asym or sym stores
+  const bool one_group = k[1].group == v[1].group;
+  const bool fused = c && (one_group || (!bf && mode_ok(k[1].mode) && mode_ok(v[1].mode))) &&
+                     detail::flash_fused_supported(q, sq_b, sq_h, norm, fk, fv, Hq, Hkv, D);
   // A combine that reads every split slot (the unfused kernels write one per
   // split; the split stage alone leaves empty statistics in the slots past
   // the fused runs) holds at most MAXSPLIT of them: checked before any launch.
   // A full call on the fused path reads only the live slots (a head's fused
   // runs, at most one per workgroup, and the dense slices), so the context
   // length is bounded by the workspace alone.
-  if (c && !(fused && live) && nsf + NSD_MAX > MAXSPLIT) return IQ_ERR_SHAPE;
+  // (With different group sizes that bound stands on either path.)
+  if (c && !(fused && one_group && live) && nsf + NSD_MAX > MAXSPLIT) return IQ_ERR_SHAPE;
   // bf16 layers: the fused kernel (K and V of one group size) and the dense
   // kernels; the unfused packed kernels take fp16 only
   if (c && !fused && bf) return IQ_ERR_MODE;

@@ -1,6 +1,6 @@
 // Fused flash-decoding kernel (gfx950): QK^T, softmax and attn.V over the
-// packed range of every (batch, KV head), for K and V stores that share their
-// group size (bit widths may differ: KB for K, VB for V).  Its output is one
+// packed range of every (batch, KV head), for K and V stores of any bit widths
+// (KB for K, VB for V) and group sizes (the kernel's G is the smaller).  Its output is one
 // partial (m, l, unnormalized o) per run in the split slots of the decode
 // workspace; the combine kernel (iq_decode.hip) merges the slots.
 //
@@ -253,6 +253,9 @@ __device__ __forceinline__ float seg_sum(float v) {
 // 0: the arguments' ksym / vsym).  A known mode drops the meta word's shift
 // and the zero point's select from every group's decode: -0.3 us per
 // headline launch and -0.7 to -1.3 us per 3-bit sym launch (same-box A/B).
+// 3: modes at run time and stores of different group sizes (a.kgs, a.vgs); an
+// instance of its own, since those shifts in the SM = 0 instances cost a
+// 28.3 us bf16 step 0.36 us.
 template <int KB, int VB, int G, int D, int NREP, bool QS, bool AVO = false, bool QKO = false, bool VH = false,
           bool BF = false, int SM = 0>
 __global__ __launch_bounds__((FusedShape<G, NREP, QS, AVO>::NT), (fused_waves_per_simd<G, NREP, QS, AVO>())) void flash_fused_kernel(FusedArgs a) {
@@ -275,11 +278,18 @@ __global__ __launch_bounds__((FusedShape<G, NREP, QS, AVO>::NT), (fused_waves_pe
   const int lane = tid & 63;
   const int hl = lane & 3;
   constexpr bool qsplit = QS;  // key normalization: hi/lo query rows
-  const int ksym = SM == 0 ? a.ksym : int(SM == 2), vsym = SM == 0 ? a.vsym : int(SM == 2);
+  constexpr bool RT = SM == 0 || SM == 3;  // store modes at run time
+  const int ksym = RT ? a.ksym : int(SM == 2), vsym = RT ? a.vsym : int(SM == 2);
   const int kms = ksym ? 2 : 4, vms = vsym ? 2 : 4;  // meta bytes per token / column
   const uint32_t kmv = meta_voff(lane, ksym), vmv = meta_voff(lane, vsym);
   const uint32_t ksh = meta_shift(lane, ksym), vsh = meta_shift(lane, vsym);
-  const uint32_t kcls = meta_sym_classes(ksym, a.khyb);  // SM == 0: the K groups read as sym
+  // stores of different group sizes (SM = 3): the kernel's group G is the
+  // smaller, and a group of the larger store is read as 2^kgs or 2^vgs groups
+  // that share its {scale, zero}: a G-piece of a group is a whole number of
+  // words, at a lane stride of the group's words
+  const int kgs = SM == 3 ? a.kgs : 0, vgs = SM == 3 ? a.vgs : 0;
+  const uint32_t klane = (uint32_t(lane) * (KW * 4)) << kgs, vlane = (uint32_t(lane) * (VW * 4)) << vgs;
+  const uint32_t kcls = meta_sym_classes(ksym, a.khyb);  // RT: the K groups read as sym
   const int64_t rows = int64_t(a.nitems / a.nsplit) * NREP;
 
   struct KRegs { uint32_t w[NG][FBPW][KW]; uint32_t m[NG][FBPW]; };
@@ -293,28 +303,32 @@ __global__ __launch_bounds__((FusedShape<G, NREP, QS, AVO>::NT), (fused_waves_pe
   auto load_k = [&](int bh, int blk, bool real, KRegs& k) {
     const int64_t blk0 = int64_t(bh) * a.k_cap_blocks + a.kblk0;
     const rsrc_t rc = make_rsrc(a.kc + blk0 * (NG * TOKEN_BLOCK * KW), real ? a.k_code_bytes : 0u);
-    const rsrc_t rm = make_rsrc(a.km + blk0 * (NG * TOKEN_BLOCK * (kms / 2)), real ? a.k_meta_bytes : 0u);
+    const rsrc_t rm = make_rsrc(a.km + blk0 * ((NG >> kgs) * TOKEN_BLOCK * (kms / 2)), real ? a.k_meta_bytes : 0u);
     const int b0 = blk * FBPW;
 #pragma unroll
     for (int g = 0; g < NG; ++g)
 #pragma unroll
       for (int j = 0; j < FBPW; ++j) {
-        const uint32_t u = uint32_t((b0 + j) * NG + g) * TOKEN_BLOCK;  // first token slot of the unit
-        bload_words<KW>(rc, uint32_t(lane) * (KW * 4), u * (KW * 4), k.w[g][j]);
+        // first token slot of the unit; the kernel's group g is piece g & (2^kgs - 1) of a store group
+        const uint32_t u = uint32_t((b0 + j) * (NG >> kgs) + (g >> kgs)) * TOKEN_BLOCK;
+        const uint32_t part = uint32_t(g & ((1 << kgs) - 1)) * (KW * 4);
+        bload_words<KW>(rc, klane, ((u * (KW * 4)) << kgs) + part, k.w[g][j]);
         k.m[g][j] = bload_u32(rm, kmv, u * kms);
       }
   };
   auto load_v = [&](int bh, int blk, bool real, VRegs& v) {
     const int64_t g0 = int64_t(bh) * a.v_cap_groups + a.vg0;
-    const rsrc_t rc = make_rsrc(a.vc + g0 * (D * VW), real ? a.v_code_bytes : 0u);
+    const rsrc_t rc = make_rsrc(a.vc + ((g0 * (D * VW)) << vgs), real ? a.v_code_bytes : 0u);
     const rsrc_t rm = make_rsrc(a.vm + g0 * (D * (vms / 2)), real ? a.v_meta_bytes : 0u);
     const int vgw = blk * WTOK / G;  // the block's first V group
 #pragma unroll
     for (int u = 0; u < VPW; ++u)
 #pragma unroll
       for (int e = 0; e < DPL; ++e) {
-        const uint32_t c0 = uint32_t((vgw + u) * D + 64 * e);  // first column slot of the unit
-        bload_words<VW>(rc, uint32_t(lane) * (VW * 4), c0 * (VW * 4), v.w[u][e]);
+        // first column slot of the unit, and the group's piece of it
+        const uint32_t c0 = uint32_t(((vgw + u) >> vgs) * D + 64 * e);
+        const uint32_t part = uint32_t((vgw + u) & ((1 << vgs) - 1)) * (VW * 4);
+        bload_words<VW>(rc, vlane, ((c0 * (VW * 4)) << vgs) + part, v.w[u][e]);
         v.m[u][e] = bload_u32(rm, vmv, c0 * vms);
       }
   };
@@ -540,7 +554,7 @@ __global__ __launch_bounds__((FusedShape<G, NREP, QS, AVO>::NT), (fused_waves_pe
 #pragma unroll
           for (int j = 0; j < FBPW; ++j) {
             float s, z;
-            if constexpr (SM == 0) meta_sz_rt<KB, BF>(kc.m[g][j], ksh, kcls, s, z);
+            if constexpr (RT) meta_sz_rt<KB, BF>(kc.m[g][j], ksh, kcls, s, z);
             else meta_sz<KB, BF>(kc.m[g][j], ksh, ksym, s, z);
 #pragma unroll
             for (int h = 0; h < NREP; ++h) {
@@ -730,6 +744,31 @@ __global__ __launch_bounds__((FusedShape<G, NREP, QS, AVO>::NT), (fused_waves_pe
   lds_barrier();
   while (step(ka, kb) && step(kb, ka)) {
   }
+}
+
+// Launch for K and V of different group sizes (a.kgs, a.vgs; group: the smaller,
+// 32 or 64; fp16 layers, asym or sym): the SM = 3 instances.  At 4-bit K of 32
+// and 2-bit V of 64, B = 8, 8 KV heads, 16384 tokens with a window, the decode
+// call takes 33.9 us against 81.9 us with the unfused QK^T and attn.V kernels.
+template <int KB>
+int fused_launch_mixed(const FusedArgs& a, int vbits, int group, int D, int nrep, bool norm, int* grid_out,
+                       hipStream_t stream, bool launch) {
+  return dispatch_shape(vbits, group, D, nrep, 0, [&]<int VB, int G, int DD, int R, bool S>() -> int {
+    if constexpr (G > 64) {
+      return IQ_ERR_GROUP;
+    } else {
+      auto* kern = norm ? flash_fused_kernel<KB, VB, G, DD, R, true, false, false, false, false, 3>
+                        : flash_fused_kernel<KB, VB, G, DD, R, false, false, false, false, false, 3>;
+      const int nt = norm ? FusedShape<G, R, true>::NT : FusedShape<G, R, false>::NT;
+      static detail::OccCache occ[2];
+      const int pc = detail::blocks_per_cu(kern, nt, occ[norm ? 1 : 0]);
+      const int grid = int(std::min<int64_t>(a.nitems, int64_t(pc) * detail::num_cus()));
+      if (grid_out) *grid_out = grid;
+      if (!launch) return int(IQ_OK);
+      kern<<<dim3(grid), nt, 0, stream>>>(a);
+      return launch_status();
+    }
+  });
 }
 
 // Launch of the fused kernel for K bit width KB (the arguments filled by

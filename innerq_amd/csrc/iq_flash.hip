@@ -28,12 +28,12 @@ int flash_fused_launch(const void* q, int64_t sq_b, int64_t sq_h, const void* no
                        const FusedStore& v, int B, int Hq, int Hkv, int T, int D, float scale, float* ml,
                        float* part, int* grid, hipStream_t stream, bool launch) {
   if (B == 0 || T == 0) return IQ_OK;
-  if (k.group != v.group) return IQ_ERR_GROUP;
+  const int G = std::min(k.group, v.group);  // the kernel's group
   // a bf16 layer: IQ_MODE_BF16 on both stores (the query, factor and metadata in bf16)
   const bool bf = act_bf16(k.mode);
   if (bf != act_bf16(v.mode)) return IQ_ERR_MODE;
   const int kmode = base_mode(k.mode), vmode = base_mode(v.mode);
-  if (T % k.group || FSPLIT != flash_split_tokens()) return IQ_ERR_GROUP;
+  if (T % v.group || (k.group | v.group) % G || FSPLIT != flash_split_tokens()) return IQ_ERR_GROUP;
   if (k.t0 % TOKEN_BLOCK || v.t0 % v.group) return IQ_ERR_ALIGN;
   if (!flash_fused_supported(q, sq_b, sq_h, norm, k, v, Hq, Hkv, D)) return IQ_ERR_SHAPE;
   FusedArgs a{};
@@ -56,32 +56,43 @@ int flash_fused_launch(const void* q, int64_t sq_b, int64_t sq_h, const void* no
   a.scale_log2 = scale * 1.4426950408889634f;
   a.ml = ml; a.part = part;
   a.empty_stats = grid ? 0 : 1;  // a caller that takes the workgroup count reads only the run slots
+  a.kgs = __builtin_ctz(unsigned(k.group / G));
+  a.vgs = __builtin_ctz(unsigned(v.group / G));
   a.pair_e0 = fused_pair_e0(k.bits, v.bits, vmode == IQ_MODE_HYBRID);
   const bool nm = norm != nullptr;
+  if (k.group != v.group) {  // fp16 layers, asym or sym stores
+    if (bf || kmode == IQ_MODE_HYBRID || vmode == IQ_MODE_HYBRID) return IQ_ERR_MODE;
+    switch (k.bits) {
+      case 2: return flash_fused_launch_mg_k2(a, v.bits, G, D, Hq / Hkv, nm, grid, stream, launch);
+      case 3: return flash_fused_launch_mg_k3(a, v.bits, G, D, Hq / Hkv, nm, grid, stream, launch);
+      case 4: return flash_fused_launch_mg_k4(a, v.bits, G, D, Hq / Hkv, nm, grid, stream, launch);
+      default: return IQ_ERR_BITS;
+    }
+  }
   if (bf) {
     const bool vh = vmode == IQ_MODE_HYBRID;
     switch (k.bits) {
-      case 2: return vh ? flash_fused_launch_bf_vh_k2(a, v.bits, k.group, D, Hq / Hkv, nm, grid, stream, launch)
-                        : flash_fused_launch_bf_k2(a, v.bits, k.group, D, Hq / Hkv, nm, grid, stream, launch);
-      case 3: return vh ? flash_fused_launch_bf_vh_k3(a, v.bits, k.group, D, Hq / Hkv, nm, grid, stream, launch)
-                        : flash_fused_launch_bf_k3(a, v.bits, k.group, D, Hq / Hkv, nm, grid, stream, launch);
-      case 4: return vh ? flash_fused_launch_bf_vh_k4(a, v.bits, k.group, D, Hq / Hkv, nm, grid, stream, launch)
-                        : flash_fused_launch_bf_k4(a, v.bits, k.group, D, Hq / Hkv, nm, grid, stream, launch);
+      case 2: return vh ? flash_fused_launch_bf_vh_k2(a, v.bits, G, D, Hq / Hkv, nm, grid, stream, launch)
+                        : flash_fused_launch_bf_k2(a, v.bits, G, D, Hq / Hkv, nm, grid, stream, launch);
+      case 3: return vh ? flash_fused_launch_bf_vh_k3(a, v.bits, G, D, Hq / Hkv, nm, grid, stream, launch)
+                        : flash_fused_launch_bf_k3(a, v.bits, G, D, Hq / Hkv, nm, grid, stream, launch);
+      case 4: return vh ? flash_fused_launch_bf_vh_k4(a, v.bits, G, D, Hq / Hkv, nm, grid, stream, launch)
+                        : flash_fused_launch_bf_k4(a, v.bits, G, D, Hq / Hkv, nm, grid, stream, launch);
       default: return IQ_ERR_BITS;
     }
   }
   if (vmode == IQ_MODE_HYBRID) {
     switch (k.bits) {
-      case 2: return flash_fused_launch_vh_k2(a, v.bits, k.group, D, Hq / Hkv, norm != nullptr, grid, stream, launch);
-      case 3: return flash_fused_launch_vh_k3(a, v.bits, k.group, D, Hq / Hkv, norm != nullptr, grid, stream, launch);
-      case 4: return flash_fused_launch_vh_k4(a, v.bits, k.group, D, Hq / Hkv, norm != nullptr, grid, stream, launch);
+      case 2: return flash_fused_launch_vh_k2(a, v.bits, G, D, Hq / Hkv, norm != nullptr, grid, stream, launch);
+      case 3: return flash_fused_launch_vh_k3(a, v.bits, G, D, Hq / Hkv, norm != nullptr, grid, stream, launch);
+      case 4: return flash_fused_launch_vh_k4(a, v.bits, G, D, Hq / Hkv, norm != nullptr, grid, stream, launch);
       default: return IQ_ERR_BITS;
     }
   }
   switch (k.bits) {
-    case 2: return flash_fused_launch_k2(a, v.bits, k.group, D, Hq / Hkv, norm != nullptr, grid, stream, launch);
-    case 3: return flash_fused_launch_k3(a, v.bits, k.group, D, Hq / Hkv, norm != nullptr, grid, stream, launch);
-    case 4: return flash_fused_launch_k4(a, v.bits, k.group, D, Hq / Hkv, norm != nullptr, grid, stream, launch);
+    case 2: return flash_fused_launch_k2(a, v.bits, G, D, Hq / Hkv, norm != nullptr, grid, stream, launch);
+    case 3: return flash_fused_launch_k3(a, v.bits, G, D, Hq / Hkv, norm != nullptr, grid, stream, launch);
+    case 4: return flash_fused_launch_k4(a, v.bits, G, D, Hq / Hkv, norm != nullptr, grid, stream, launch);
     default: return IQ_ERR_BITS;
   }
 }

@@ -557,6 +557,7 @@ struct FusedArgs {
   int empty_stats;
   int pair_e0;  // the partition (ShareMap e0_num; 0: plain)
   int khyb;     // 1: a hybrid K store (meta as asym, the group's flag picks sym)
+  int kgs, vgs;  // log2 of the stores' group sizes over the kernel's group G (0: the same; SM = 3 instances)
 };
 // its launch per K bit width (iq_flash_k{2,3,4}.hip)
 int flash_fused_launch_k2(const FusedArgs& a, int vbits, int group, int D, int nrep, bool norm, int* grid,
@@ -584,6 +585,13 @@ int flash_fused_launch_vh_k2(const FusedArgs& a, int vbits, int group, int D, in
 int flash_fused_launch_vh_k3(const FusedArgs& a, int vbits, int group, int D, int nrep, bool norm, int* grid,
                              hipStream_t stream, bool launch);
 int flash_fused_launch_vh_k4(const FusedArgs& a, int vbits, int group, int D, int nrep, bool norm, int* grid,
+                             hipStream_t stream, bool launch);
+// and for K and V of different group sizes (iq_flash_mg_k{2,3,4}.hip)
+int flash_fused_launch_mg_k2(const FusedArgs& a, int vbits, int group, int D, int nrep, bool norm, int* grid,
+                             hipStream_t stream, bool launch);
+int flash_fused_launch_mg_k3(const FusedArgs& a, int vbits, int group, int D, int nrep, bool norm, int* grid,
+                             hipStream_t stream, bool launch);
+int flash_fused_launch_mg_k4(const FusedArgs& a, int vbits, int group, int D, int nrep, bool norm, int* grid,
                              hipStream_t stream, bool launch);
 size_t qk_record_bytes(int B, int Hq, int D);
 size_t av_record_bytes(int B, int Hq, int T, int group);
