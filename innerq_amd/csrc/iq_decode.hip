@@ -31,7 +31,17 @@ namespace {
 constexpr int DT = 64;        // dense tokens per chunk
 constexpr int NSD_MAX = 4;    // split slots of the dense tokens, at most
 constexpr int DSLICE = 32;    // dense tokens per split slot, at least
-constexpr int MERGE_RUNS_MAX = 4;  // fused runs per (batch, KV head) the merging dense kernel preloads
+// Fused runs per (batch, KV head) that the merging dense kernel takes: the
+// first MERGE_PRE of them are loaded with the window's rows, the next beside
+// the sections' last barrier, the rest MERGE_PRE at a time.  Up to four query
+// heads per KV head, fp16: 16 runs (4-bit, 8 KV heads of 4 query heads, 8192
+// tokens and a 128-token window, a call: B = 4, 8 runs, 21.2 us with the dense
+// slices and the combine, 19.4 merged; B = 2, 16 runs, 18.4 and 18.1; past 16
+// they measure the same).  Eight query heads per KV head and bf16 layers, whose
+// window takes longer in two sections than in four slices: 4 runs (8 runs of
+// eight bf16 query heads: 24.7 us with the slices, 27.9 merged).
+constexpr int MERGE_RUNS_MAX = 16, MERGE_PRE = 4;
+constexpr int merge_runs_max(bool bf, int nrep) { return bf || nrep > 4 ? MERGE_PRE : MERGE_RUNS_MAX; }
 // 256-thread sections of the merging dense kernel: three where the window
 // holds packed rows (32 sinks, a 96-token recent window and the <= 31 packed
 // keys short of a V group, 129-159 tokens that two sections take in two
@@ -360,22 +370,27 @@ __global__ __launch_bounds__(MERGE ? 256 * NS : 256) void dense_attn_kernel(Dens
     vpk = gather_row<RE>(a.v, b, kvh, t, gq * RE, vr);
   };
   // the first chunk's rows and the query are loaded together (one round trip);
-  // MERGE: so are the fused runs' statistics and partials of the thread's
-  // first output element (up to NRPRE runs; more are read at the merge)
-  constexpr int NRPRE = MERGE_RUNS_MAX;
-  float pm[NRPRE], pl[NRPRE], po[NRPRE];
+  // MERGE: so are the fused runs' statistics (thread = (run, head)) and the
+  // first MERGE_PRE runs' partials of the thread's output elements
+  constexpr int EPT = MERGE ? (NREP * D + NTH - 1) / NTH : 1;  // output elements per thread
+  float po[EPT][MERGE_PRE];
+  float2 rst = make_float2(-INFINITY, 0.f);
   int nr = 0;
+  // element e's partials of runs [sp0, sp0 + MERGE_PRE), clamped so that every load is issued at once
+  auto load_runs = [&](int e, int sp0, float (&p)[MERGE_PRE]) {
+    const int r = min(int(threadIdx.x) + e * NTH, NREP * D - 1);
+    const int64_t row = int64_t(bh) * NREP + r / D;
+#pragma unroll
+    for (int sp = 0; sp < MERGE_PRE; ++sp)
+      p[sp] = a.fpart[(int64_t(min(sp0 + sp, nr - 1)) * rows + row) * D + r % D];
+  };
   if constexpr (MERGE) {
     nr = detail::ShareMap::make(a.fgrid, int(gridDim.y), a.fnsf, a.fpair_e0).nruns(bh);
-    const int r = int(threadIdx.x);
-    const int64_t row = int64_t(bh) * NREP + min(r / D, NREP - 1);
+    if (int(threadIdx.x) < nr * NREP)
+      rst = *reinterpret_cast<const float2*>(
+          a.fml + (int64_t(int(threadIdx.x) / NREP) * rows + int64_t(bh) * NREP + int(threadIdx.x) % NREP) * 2);
 #pragma unroll
-    for (int sp = 0; sp < NRPRE; ++sp) {
-      const int64_t sr = int64_t(min(sp, nr - 1)) * rows + row;  // clamped: every load issued at once
-      pm[sp] = a.fml[sr * 2];
-      pl[sp] = a.fml[sr * 2 + 1];
-      po[sp] = a.fpart[sr * D + r % D];
-    }
+    for (int e = 0; e < EPT; ++e) load_runs(e, 0, po[e]);
   }
   if (i0 < i1) gather(i0);
   for (int i = int(threadIdx.x); i < NREP * TW; i += NTH) {
@@ -594,6 +609,14 @@ __global__ __launch_bounds__(MERGE ? 256 * NS : 256) void dense_attn_kernel(Dens
   if constexpr (MERGE) {
     // ---- merge: the sections' states and the fused runs' partials ----
     __shared__ float mh[NH][NREP], lh[NH][NREP];
+    __shared__ float2 rml[MERGE_RUNS_MAX][NREP];  // the runs' statistics
+    static_assert(MERGE_RUNS_MAX * 4 <= NTH && MERGE_PRE * 8 <= NTH, "one thread per run and head");
+    float po2[EPT][MERGE_PRE];
+    if (nr > MERGE_PRE) {
+#pragma unroll
+      for (int e = 0; e < EPT; ++e) load_runs(e, MERGE_PRE, po2[e]);
+    }
+    if (int(threadIdx.x) < nr * NREP) rml[int(threadIdx.x) / NREP][int(threadIdx.x) % NREP] = rst;
     __shared__ float oh[BF ? NH : 1][BF ? NREP : 1][BF ? D : 1];  // BF: the sections' outputs
 #pragma unroll
     for (int hh = 0; hh < HPW; ++hh) {
@@ -615,34 +638,29 @@ __global__ __launch_bounds__(MERGE ? 256 * NS : 256) void dense_attn_kernel(Dens
       }
     }
     __syncthreads();
-    for (int r = int(threadIdx.x); r < NREP * D; r += NTH) {
+#pragma unroll
+    for (int e = 0; e < EPT; ++e) {
+      const int r = int(threadIdx.x) + e * NTH;
+      if (r >= NREP * D) break;
       const int h = r / D, dd = r % D;
-      const int64_t row = int64_t(bh) * NREP + h;
-      const bool pre = r < NTH;  // the preloaded element (registers indexed by constants only)
       float M = -INFINITY;
 #pragma unroll
       for (int hf = 0; hf < NH; ++hf) M = fmaxf(M, mh[hf][h]);
-#pragma unroll
-      for (int sp = 0; sp < NRPRE; ++sp)
-        if (sp < nr) M = fmaxf(M, pre ? pm[sp] : a.fml[(int64_t(sp) * rows + row) * 2]);
-      for (int sp = NRPRE; sp < nr; ++sp) M = fmaxf(M, a.fml[(int64_t(sp) * rows + row) * 2]);
+      for (int sp = 0; sp < nr; ++sp) M = fmaxf(M, rml[sp][h].x);
       float L = 0.f, acc = 0.f;
-      auto add_run = [&](float ms, float ls, float pv) {  // the runs in slot order, then the sections
-        const float w = ms == -INFINITY ? 0.f : __expf(ms - M);
-        L = fmaf(w, ls, L);
+      auto add_run = [&](float2 s, float pv) {  // the runs in slot order, then the sections
+        const float w = s.x == -INFINITY ? 0.f : __expf(s.x - M);
+        L = fmaf(w, s.y, L);
         acc = w != 0.f ? fmaf(w, pv, acc) : acc;
       };
 #pragma unroll
-      for (int sp = 0; sp < NRPRE; ++sp) {
-        if (sp < nr) {
-          const int64_t sr = int64_t(sp) * rows + row;
-          if (pre) add_run(pm[sp], pl[sp], po[sp]);
-          else add_run(a.fml[sr * 2], a.fml[sr * 2 + 1], a.fpart[sr * D + dd]);
-        }
-      }
-      for (int sp = NRPRE; sp < nr; ++sp) {
-        const int64_t sr = int64_t(sp) * rows + row;
-        add_run(a.fml[sr * 2], a.fml[sr * 2 + 1], a.fpart[sr * D + dd]);
+      for (int sp = 0; sp < MERGE_PRE; ++sp)
+        if (sp < nr) add_run(rml[sp][h], po[e][sp]);
+      for (int s0 = MERGE_PRE; s0 < nr; s0 += MERGE_PRE) {
+        if (s0 > MERGE_PRE) load_runs(e, s0, po2[e]);
+#pragma unroll
+        for (int sp = 0; sp < MERGE_PRE; ++sp)
+          if (s0 + sp < nr) add_run(rml[s0 + sp][h], po2[e][sp]);
       }
 #pragma unroll
       for (int hf = 0; hf < NH; ++hf) {
@@ -1029,7 +1047,7 @@ int launch_splits(const void* q, int64_t sq_b, int64_t sq_h, const void* norm, c
   // dense kernel, which also merges the fused runs and writes the output (no
   // dense slots, no combine): chosen once the fused kernel's workgroup count
   // is known, if no (batch, KV head) has more fused runs than that kernel
-  // preloads.  Heads spread over more workgroups (a small batch over a long
+  // takes.  Heads spread over more workgroups (a small batch over a long
   // context) take the slices and the combine, which reads every slot in one
   // round of loads.
   const bool merge_cand = mo && live && fused && n_dense > 0 && n_dense <= MERGE_DENSE_MAX;
@@ -1046,7 +1064,7 @@ int launch_splits(const void* q, int64_t sq_b, int64_t sq_h, const void* norm, c
     bool merge_dense = merge_cand;
     if (merge_cand) {
       const detail::ShareMap sm = detail::ShareMap::make(grid, int(bhs), nsf, plan->pair_e0);
-      for (int h = 0; h < int(bhs) && merge_dense; ++h) merge_dense = sm.nruns(h) <= MERGE_RUNS_MAX;
+      for (int h = 0; h < int(bhs) && merge_dense; ++h) merge_dense = sm.nruns(h) <= merge_runs_max(bf, Hq / Hkv);
       if (!merge_dense)
         if (int e = launch_slices()) return e;
     }
