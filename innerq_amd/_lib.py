@@ -134,6 +134,21 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+FAST_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_iqfast.so")
+
+
+def load_fast():
+    """The native call front (csrc/iq_pyfast.cpp)."""
+    import importlib.machinery
+    import importlib.util
+    if not os.path.exists(FAST_PATH):
+        raise RuntimeError(f"{FAST_PATH} is missing: build it with `python -m innerq_amd.build`")
+    loader = importlib.machinery.ExtensionFileLoader("_iqfast", FAST_PATH)
+    m = importlib.util.module_from_spec(importlib.util.spec_from_loader("_iqfast", loader))
+    loader.exec_module(m)
+    return m
+
+
 def strerror(status: int) -> str:
     try:
         return lib().iq_strerror(status).decode()

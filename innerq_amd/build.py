@@ -1,4 +1,5 @@
-"""Build libinnerq_hip.so in-tree with hipcc for gfx950.
+"""Build libinnerq_hip.so in-tree with hipcc for gfx950, and the native call front _iqfast.so
+(a CPython extension over libtorch, host code only) with the host compiler.
 
     python -m innerq_amd.build            # compile (always recompiles)
 
@@ -21,6 +22,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libinnerq_hip.so")
+FAST = os.path.join(HERE, "_iqfast.so")
 OBJ_DIR = os.path.join(HERE, "_build")
 ARCH = "gfx950"
 
@@ -60,12 +62,32 @@ def _compile(src: str) -> str:
     return obj
 
 
+def build_fast() -> str:
+    """csrc/iq_pyfast.cpp -> innerq_amd/_iqfast.so."""
+    import sysconfig
+
+    import torch
+    t = os.path.dirname(torch.__file__)
+    abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={abi}",
+           f"-I{t}/include", f"-I{t}/include/torch/csrc/api/include", f"-I{sysconfig.get_paths()['include']}",
+           os.path.join(CSRC, "iq_pyfast.cpp"), "-o", FAST + ".tmp", f"-L{t}/lib", "-ltorch_python", "-ltorch_cpu",
+           "-lc10", f"-Wl,-rpath,{t}/lib"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"host compiler failed for iq_pyfast.cpp:\n{r.stderr[-8000:]}")
+    os.replace(FAST + ".tmp", FAST)
+    return FAST
+
+
 def build(verbose: bool = True) -> str:
     os.makedirs(OBJ_DIR, exist_ok=True)
     srcs = sources()
     jobs = max(1, min(len(srcs), int(os.environ.get("MAX_JOBS", os.cpu_count() or 4))))
     with cf.ThreadPoolExecutor(jobs) as ex:
+        fast = ex.submit(build_fast)
         objs = list(ex.map(_compile, srcs))
+        fast.result()
     tmp = LIB + ".tmp"
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp]
     r = subprocess.run(cmd, capture_output=True, text=True)

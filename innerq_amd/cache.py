@@ -466,7 +466,46 @@ class InnerqDynamicLayer(CacheLayerMixin):
         -> [B, Hq, 1, D] of that dtype.  pads: per sequence, how many of its first
         tokens a padding mask hides (left padding; None: none)."""
         self._check_attend(query_states)
-        return self._attend_rows(query_states[:, :, 0], scaling, self._attend_start(), pads)[:, :, None]
+        return self._attend(query_states, scaling, pads)
+
+    def _attend(self, query_states: torch.Tensor, scaling: float, pads: Optional[Sequence[int]]) -> torch.Tensor:
+        s0 = self._attend_start()
+        out = self._attend_native(query_states, scaling, s0) if pads is None else None
+        return out if out is not None else self._attend_rows(query_states[:, :, 0], scaling, s0, pads)[:, :, None]
+
+    def _attend_native(self, query_states: torch.Tensor, scaling: float, s0: int) -> Optional[torch.Tensor]:
+        """_attend_from over the whole batch through the native call front, which takes the windows'
+        buffers and row ranges instead of views (None: the general path)."""
+        fast = ops._native(query_states)
+        kwin, vwin = self._kwin, self._vwin
+        if fast is None or kwin is None or vwin is None:
+            return None
+        kq, vq, nk, nv = self._packed_split()
+
+        def part(sink, quant, nq, win, before):
+            # sink and its first row, store, first token and end, window buffer, first row and rows
+            ns = sink.shape[-2]
+            r0 = max(s0 - ns - nq, 0)
+            n = win.n + before - r0
+            return (sink if s0 < ns else None, s0, None if quant is None else quant.store, min(max(s0 - ns, 0), nq),
+                    nq, win.buf if n > 0 else None, win.start - before + r0, n)
+
+        return fast.decode(query_states, *part(self.keys_sink, self._kq, kq, kwin, nk),
+                           *part(self.values_sink, self._vq, vq, vwin, nv), scaling,
+                           self.key_normalization_factor if self._kq is not None else None, None, 4)
+
+    def _packed_split(self) -> tuple[int, int, int, int]:
+        """(K, V) tokens that a decode reads packed, and the packed tokens after them that it reads
+        as the rows kept before the windows."""
+        kq = self._kq.length if self._kq is not None else 0
+        vq = self._vq.length if self._vq is not None else 0
+        e = self._packed_end()
+        if e is not None and self._kwin is not None and self._vwin is not None:
+            nk = self.keys_sink.shape[-2] + kq - e  # packed tokens past e, read as the rows kept
+            nv = self.values_sink.shape[-2] + vq - e
+            if nk <= self._kwin.shadow and nv <= self._vwin.shadow and (nk or nv):
+                return kq - nk, vq - nv, nk, nv
+        return kq, vq, 0, 0
 
     def _attend_start(self) -> int:
         """The first token attend() reads (0: all of them)."""
@@ -533,16 +572,10 @@ class InnerqDynamicLayer(CacheLayerMixin):
                     store.length = nq
             return dense_sink, store, t0, dense_recent
 
-        kq = self._kq.length if self._kq is not None else 0
-        vq = self._vq.length if self._vq is not None else 0
         krecent, vrecent = self.keys_recent, self.values_recent
-        e = self._packed_end()
-        if e is not None and self._kwin is not None and self._vwin is not None:
-            nk = self.keys_sink.shape[-2] + kq - e  # packed tokens past e, read as the rows kept
-            nv = self.values_sink.shape[-2] + vq - e
-            if nk <= self._kwin.shadow and nv <= self._vwin.shadow and (nk or nv):
-                kq, krecent = kq - nk, self._kwin.rows_before(nk)
-                vq, vrecent = vq - nv, self._vwin.rows_before(nv)
+        kq, vq, nk, nv = self._packed_split()
+        if nk or nv:
+            krecent, vrecent = self._kwin.rows_before(nk), self._vwin.rows_before(nv)
         ks, kst, kt0, kr = parts(self.keys_sink, self._kq, kq, krecent)
         vs, vst, vt0, vr = parts(self.values_sink, self._vq, vq, vrecent)
         norm = part_rows(self.key_normalization_factor) if self._kq is not None else None
@@ -630,7 +663,7 @@ class InnerqDynamicSlidingWindowLayer(InnerqDynamicLayer):
         if not self.fix_sliding_window:
             raise NotImplementedError("attend() of a sliding-window layer needs fix_sliding_window = True")
         self._check_attend(query_states)
-        return self._attend_rows(query_states[:, :, 0], scaling, self._attend_start(), pads)[:, :, None]
+        return self._attend(query_states, scaling, pads)
 
     def _attend_start(self) -> int:
         return max(self.cumulative_length - self.sliding_window, 0)

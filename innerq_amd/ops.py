@@ -23,8 +23,36 @@ def _p(t: Optional[torch.Tensor]):
     return None if t is None else ctypes.c_void_p(t.data_ptr())
 
 
+def _raw_stream(device: torch.device) -> int:
+    """The handle of the device's current stream."""
+    if device.index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
 def _stream(device: torch.device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    return ctypes.c_void_p(_raw_stream(device))
+
+
+_fast = None  # the native call front, once a device call has loaded it
+
+
+def _native(t):
+    """The native call front (_iqfast) for a call on tensor ``t``: None where ``t`` is no device
+    tensor, which the general path refuses."""
+    global _fast
+    if _fast is not None:
+        return _fast
+    if not isinstance(t, torch.Tensor) or not t.is_cuda:
+        return None
+    h = _lib.lib()
+    m = _lib.load_fast()
+    names = ("iq_decode_workspace_bytes", "iq_decode_attention", "iq_qk_workspace_bytes", "iq_qk_gemv",
+             "iq_av_workspace_bytes", "iq_av_gemv", "iq_window_append")
+    m.bind(tuple(ctypes.cast(getattr(h, n), ctypes.c_void_p).value for n in names), _WS,
+           torch._C._cuda_getCurrentRawStream)
+    _fast = m
+    return m
 
 
 def require_device(t: torch.Tensor, name: str, dtype=torch.float16) -> None:
@@ -495,6 +523,9 @@ def window_append(kwin: Optional[RecentWindow], knew: Optional[torch.Tensor], kf
     [B,H,m,D] go after each window, the first ``flush`` tokens of [window | new]
     are quantized into the store (cache.py:283-365), the windows advance past
     them and the stores grow by them."""
+    fast = _native(knew)
+    if fast is not None and fast.window_append(kwin, knew, kflush, kstore, knorm, vwin, vnew, vflush, vstore):
+        return
     roles, keep, shape = [], [], None
     for win, x, fl, st, norm in ((kwin, knew, kflush, kstore, knorm), (vwin, vnew, vflush, vstore, None)):
         if win is None:
@@ -615,7 +646,7 @@ _WS = {}
 
 
 def _workspace(device: torch.device, nbytes: int) -> torch.Tensor:
-    key = (device.index, torch.cuda.current_stream(device).cuda_stream)
+    key = (device.index, _raw_stream(device))
     ws = _WS.get(key)
     if ws is None or ws.numel() < nbytes:
         ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
@@ -626,6 +657,11 @@ def _workspace(device: torch.device, nbytes: int) -> torch.Tensor:
 def qk_gemv(q: torch.Tensor, k: PackedStore, scale: float, norm: Optional[torch.Tensor] = None, t0: int = 0,
             T: Optional[int] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """logits [B,Hq,T] fp32 = scale * q . K[t0:t0+T] over a channel-grouped store."""
+    fast = _native(q)
+    if fast is not None:
+        r = fast.qk(q, k, scale, norm, t0, -1 if T is None else T, out)
+        if r is not None:
+            return r
     require_f16_store(k, "qk_gemv")
     require_device(q, "q")
     T = k.length - t0 if T is None else T
@@ -652,6 +688,11 @@ def av_gemv(p: torch.Tensor, v: PackedStore, t0: int = 0, T: Optional[int] = Non
             out: Optional[torch.Tensor] = None, out32: Optional[torch.Tensor] = None,
             accumulate: bool = False) -> torch.Tensor:
     """out [B,Hq,D] = p . V[t0:t0+T] over a token-grouped store (fp16 and/or fp32 outputs)."""
+    fast = _native(p) if out32 is None and not accumulate else None
+    if fast is not None:
+        r = fast.av(p, v, t0, -1 if T is None else T, out)
+        if r is not None:
+            return r
     require_f16_store(v, "av_gemv")
     require_device(p, "p")
     T = v.length - t0 if T is None else T
@@ -745,6 +786,12 @@ def decode_attention(q: torch.Tensor, k_sink: Optional[torch.Tensor], k_store: O
     """One decode step of attention for q [B,Hq,D] over [sink | packed | recent] K and V
     (fp16 or bf16: the query's dtype, which every segment and the output share); the
     stores are read from token k_t0 / v_t0 on (a sliding window's start)."""
+    fast = _native(q)
+    if fast is not None:
+        r = fast.decode(q, k_sink, 0, k_store, k_t0, -1, k_recent, 0, -1, v_sink, 0, v_store, v_t0, -1, v_recent, 0,
+                        -1, scale, norm, out, 3)
+        if r is not None:
+            return r
     q, B, Hq, Hkv, T, D, ks, vs, norm, ws = _decode_args(q, k_sink, k_store, k_recent, v_sink, v_store, v_recent,
                                                          norm, out, k_t0, v_t0)
     if out is None:
