@@ -166,14 +166,14 @@ __global__ __launch_bounds__(WG) void av_kernel(AVArgs a) {
 template <int AB>
 __global__ __launch_bounds__(256) void av_combine_kernel(const float* __restrict__ part, int nsplit, int Hq, int D,
                                                          int64_t rows, detail::OutPair o, int accumulate, int grid,
-                                                         int nrep) {
+                                                         int nrep, detail::ShareMap smap) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= rows * D) return;
   const int64_t bq = i / D;
   const int d = int(i % D);
   int n = nsplit;
   if (grid > 0)  // the runs of the (batch, KV head) in the persistent kernel's shares
-    n = detail::ShareMap::make(grid, int(rows / nrep), nsplit, 0).nruns(int(bq / nrep));  // plain partition
+    n = smap.nruns(int(bq) / nrep);
   // the slots in order, their loads AB at a time (indices clamped so that a
   // round's loads are all in flight at once; the sum order is the slot order)
   float v = 0.f;
@@ -339,8 +339,9 @@ int av_combine_launch(const float* part, int nsplit, int B, int Hq, int D, const
   const int64_t heads = std::max<int64_t>(1, rows / std::max(nrep, 1));
   const int64_t runs = grid > 0 ? std::min<int64_t>(nsplit, ceil_div(grid, heads) + 1) : nsplit;
   const dim3 g{unsigned(ceil_div(rows * D, 256))};
-  if (runs > 8) av_combine_kernel<32><<<g, 256, 0, stream>>>(part, nsplit, Hq, D, rows, o, accumulate, grid, nrep);
-  else av_combine_kernel<8><<<g, 256, 0, stream>>>(part, nsplit, Hq, D, rows, o, accumulate, grid, nrep);
+  const ShareMap sm = grid > 0 ? ShareMap::make(grid, int(heads), nsplit, 0) : ShareMap{};  // plain partition
+  auto* kern = runs > 8 ? av_combine_kernel<32> : av_combine_kernel<8>;
+  kern<<<g, 256, 0, stream>>>(part, nsplit, Hq, D, rows, o, accumulate, grid, nrep, sm);
   return launch_status();
 }
 
@@ -375,7 +376,7 @@ int av_fused_launch(const void* p, int64_t sp_b, int64_t sp_h, const uint32_t* v
     static OccCache occ[2];  // workgroups per CU at once
     const int pc = blocks_per_cu(kern, nt, occ[hyb ? 1 : 0]);
     *grid = int(std::min<int64_t>(a.nitems, int64_t(pc) * num_cus()));
-    kern<<<dim3(*grid), nt, 0, stream>>>(a);
+    kern<<<dim3(*grid), nt, 0, stream>>>(fused_grid(a, *grid));
     return launch_status();
   });
 }

@@ -155,11 +155,11 @@ struct DenseArgs {
   float* ml;  // the dense split slots' statistics: slot s at ml + s * rows * 2
   float* o;   // and partial outputs: slot s at o + s * rows * D
   // merging instance (after the fused kernel): its run partials (slots
-  // [0, nruns) of the workspace, ShareMap(fgrid, B * Hkv, fnsf, fpair_e0))
+  // [0, nruns) of the workspace, by its partition)
   // and the output, fp16 [B, Hq, D] at b * sob + hq * soh
   const float* fml;
   const float* fpart;
-  int fgrid, fnsf, fpair_e0;
+  detail::ShareMap fmap;
   uint16_t* out;
   int64_t sob, soh;
 };
@@ -385,7 +385,7 @@ __global__ __launch_bounds__(MERGE ? 256 * NS : 256) void dense_attn_kernel(Dens
       p[sp] = a.fpart[(int64_t(min(sp0 + sp, nr - 1)) * rows + row) * D + r % D];
   };
   if constexpr (MERGE) {
-    nr = detail::ShareMap::make(a.fgrid, int(gridDim.y), a.fnsf, a.fpair_e0).nruns(bh);
+    nr = a.fmap.nruns(bh);
     if (int(threadIdx.x) < nr * NREP)
       rst = *reinterpret_cast<const float2*>(
           a.fml + (int64_t(int(threadIdx.x) / NREP) * rows + int64_t(bh) * NREP + int(threadIdx.x) % NREP) * 2);
@@ -727,8 +727,8 @@ constexpr int MAXSPLIT = 1024;  // split slots of one step, at most
 constexpr int CREST = 32;
 template <int DPL, int E, int CSPEC>
 __global__ __launch_bounds__(64) void flash_combine_kernel(const float* __restrict__ ml, const float* __restrict__ part,
-                                                           int nsplit, int nsf, int grid, int pair_e0, int nrep,
-                                                           int64_t rows, int Hq, uint16_t* __restrict__ out,
+                                                           int nsplit, int nsf, int grid, detail::ShareMap smap,
+                                                           int nrep, int64_t rows, int Hq, uint16_t* __restrict__ out,
                                                            int64_t sob, int64_t soh, int bf) {
   using Vec = float __attribute__((ext_vector_type(DPL)));
   constexpr int D = 64 * DPL;
@@ -738,7 +738,7 @@ __global__ __launch_bounds__(64) void flash_combine_kernel(const float* __restri
   const int lane = threadIdx.x;
   int nr = nsf;
   if (grid > 0)  // the runs of the (batch, KV head) in the fused kernel's shares
-    nr = detail::ShareMap::make(grid, int(rows / nrep), nsf, pair_e0).nruns(int(bq / nrep));
+    nr = smap.nruns(int(bq) / nrep);
   const int n = nr + (nsplit - nsf);                                   // live slots
   auto slot = [&](int i) { return i < nr ? i : nsf + (i - nr); };     // i-th live slot
   const float2* st = reinterpret_cast<const float2*>(ml) + bq;         // slot s: st[s * rows]
@@ -1071,9 +1071,7 @@ int launch_splits(const void* q, int64_t sq_b, int64_t sq_h, const void* norm, c
     if (merge_dense) {
       da.fml = w.ml;
       da.fpart = w.part;
-      da.fgrid = grid;
-      da.fnsf = nsf;
-      da.fpair_e0 = plan->pair_e0;
+      da.fmap = detail::ShareMap::make(grid, int(bhs), nsf, plan->pair_e0);
       da.out = (uint16_t*)mo->out;
       da.sob = mo->so_b;
       da.soh = mo->so_h;
@@ -1131,9 +1129,10 @@ int launch_combine(const Workspace& w, const SplitPlan& plan, int B, int Hq, int
   // most runs of any (batch, KV head) (the share arithmetic the kernel uses)
   // and the dense slices; else every slot
   int nlive = nsplit;
+  detail::ShareMap sm{};
   if (plan.grid > 0) {
     const int heads = int(rows / std::max(plan.nrep, 1));
-    const detail::ShareMap sm = detail::ShareMap::make(plan.grid, heads, plan.nsf, plan.pair_e0);
+    sm = detail::ShareMap::make(plan.grid, heads, plan.nsf, plan.pair_e0);
     int maxr = 0;
     for (int h = 0; h < heads; ++h) maxr = std::max(maxr, sm.nruns(h));
     nlive = std::min(nsplit, maxr + (nsplit - plan.nsf));
@@ -1142,7 +1141,7 @@ int launch_combine(const Workspace& w, const SplitPlan& plan, int B, int Hq, int
   auto go = [&]<int DPL, int E>() {
     auto* kern = nlive > 8 ? flash_combine_kernel<DPL, E, 32> : flash_combine_kernel<DPL, E, 8>;
     kern<<<dim3(unsigned(rows)), 64, 0, st>>>(w.ml, w.part, nsplit, plan.nsf, plan.grid,
-                                                                      plan.pair_e0, plan.nrep, rows, Hq,
+                                                                      sm, plan.nrep, rows, Hq,
                                                                       (uint16_t*)out, so_b, so_h, plan.bf);
   };
   auto by_e = [&]<int DPL>() {

@@ -225,11 +225,23 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
-// sum over aligned segments of N lanes (every lane gets its segment's sum)
+// sum over aligned segments of N lanes (every lane gets its segment's sum):
+// inside a 16-lane row by DPP (quad xor 1, quad xor 2, half-row mirror, row
+// mirror: the lanes of a step's two halves hold equal sums, so a mirror pairs
+// the same partial sums as an xor), then rows by swizzle and shuffle
 template <int N>
 __device__ __forceinline__ float seg_sum(float v) {
-#pragma unroll
-  for (int o = 1; o < N; o <<= 1) v += __shfl_xor(v, o, 64);
+  static_assert(N == 16 || N == 32 || N == 64);
+  auto dpp = [&]<int CTRL>() {
+    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+  };
+  dpp.template operator()<0xb1>();
+  dpp.template operator()<0x4e>();
+  dpp.template operator()<0x141>();
+  dpp.template operator()<0x140>();
+  if constexpr (N >= 32)
+    v += __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, v), 0x401f));  // lane ^ 16
+  if constexpr (N == 64) v += __shfl_xor(v, 32, 64);
   return v;
 }
 
@@ -290,7 +302,8 @@ __global__ __launch_bounds__((FusedShape<G, NREP, QS, AVO>::NT), (fused_waves_pe
   const int kgs = SM == 3 ? a.kgs : 0, vgs = SM == 3 ? a.vgs : 0;
   const uint32_t klane = (uint32_t(lane) * (KW * 4)) << kgs, vlane = (uint32_t(lane) * (VW * 4)) << vgs;
   const uint32_t kcls = meta_sym_classes(ksym, a.khyb);  // RT: the K groups read as sym
-  const int64_t rows = int64_t(a.nitems / a.nsplit) * NREP;
+  const detail::ShareMap& smap = a.smap;
+  const int64_t rows = int64_t(smap.nhead) * NREP;
 
   struct KRegs { uint32_t w[NG][FBPW][KW]; uint32_t m[NG][FBPW]; };
   struct VRegs { uint32_t w[VPW][DPL][VW]; uint32_t m[VPW][DPL]; };
@@ -402,7 +415,6 @@ __global__ __launch_bounds__((FusedShape<G, NREP, QS, AVO>::NT), (fused_waves_pe
   // waves claim wave blocks from a counter in LDS (the first two per wave are
   // fixed), so they all finish the run within about one block of each other
   // whatever the issue arbitration favours. ----
-  const detail::ShareMap smap = detail::ShareMap::make(int(gridDim.x), a.nitems / a.nsplit, a.nsplit, a.pair_e0);
   int side, sh;
   smap.share(int(blockIdx.x), side, sh);
   const int plen = smap.len(side), pfirst = smap.first(side);  // a head's splits on this side
@@ -437,10 +449,9 @@ __global__ __launch_bounds__((FusedShape<G, NREP, QS, AVO>::NT), (fused_waves_pe
       return;
     }
     // plain: the shares holding the head's first and last split
-    auto share_of = [&](int s) { return int(((int64_t(s) + 1) * gridDim.x + a.nitems - 1) / a.nitems) - 1; };
-    const int c0 = share_of(r.bh * a.nsplit);
+    const int c0 = smap.share_of(int64_t(r.bh) * a.nsplit);
     slot = sh - c0;
-    nr = share_of((r.bh + 1) * a.nsplit - 1) - c0 + 1;
+    nr = smap.share_of(int64_t(r.bh + 1) * a.nsplit - 1) - c0 + 1;
   };
 
   // running softmax state of the wave over the current run (log2 domain)
@@ -734,12 +745,12 @@ __global__ __launch_bounds__((FusedShape<G, NREP, QS, AVO>::NT), (fused_waves_pe
 
   XRegs ka, kb;
   reset_run();
+  // the query first: loads return in order, so its records are built while the
+  // first blocks' K and V are still on their way
+  if constexpr (!AVO) load_q(run.bh, true, qq);
   load_x(run.bh, block_of(run, max(cur, 0)), cur >= 0, ka);
   if constexpr (!QKO) load_v(run.bh, block_of(run, max(cur, 0)), cur >= 0, v);
-  if constexpr (!AVO) {
-    load_q(run.bh, true, qq);
-    build_records(qq);
-  }
+  if constexpr (!AVO) build_records(qq);
   if (tid == 0) sm.next_block = 2 * NW;
   lds_barrier();
   while (step(ka, kb) && step(kb, ka)) {
@@ -765,7 +776,7 @@ int fused_launch_mixed(const FusedArgs& a, int vbits, int group, int D, int nrep
       const int grid = int(std::min<int64_t>(a.nitems, int64_t(pc) * detail::num_cus()));
       if (grid_out) *grid_out = grid;
       if (!launch) return int(IQ_OK);
-      kern<<<dim3(grid), nt, 0, stream>>>(a);
+      kern<<<dim3(grid), nt, 0, stream>>>(detail::fused_grid(a, grid));
       return launch_status();
     }
   });
@@ -801,7 +812,7 @@ int fused_launch_kb(const FusedArgs& a, int vbits, int group, int D, int nrep, b
     const int grid = int(std::min<int64_t>(a.nitems, int64_t(pc) * detail::num_cus()));
     if (grid_out) *grid_out = grid;
     if (!launch) return int(IQ_OK);
-    kern<<<dim3(grid), nt, 0, stream>>>(a);
+    kern<<<dim3(grid), nt, 0, stream>>>(detail::fused_grid(a, grid));
     return launch_status();
   });
 }

@@ -501,10 +501,18 @@ struct ShareMap {
     side = paired ? x & 1 : 0;
     sh = (paired ? x >> 1 : x) * per + r;
   }
+  // p / d for p, d >= 0: a 32-bit division where p fits (every list up to
+  // 2^31 / grid splits; a 64-bit one is ~100 dependent instructions on the
+  // device, ahead of a workgroup's first load)
+  __host__ __device__ static int64_t quot(int64_t p, int64_t d) {
+    return (uint64_t(p) | uint64_t(d)) >> 32 ? p / d : int64_t(uint32_t(p) / uint32_t(d));
+  }
   // first list position of share sh of a side (sh = width(): the list's end)
-  __host__ __device__ int64_t begin(int side, int sh) const { return int64_t(sh) * items(side) / width(); }
+  __host__ __device__ int64_t begin(int side, int sh) const { return quot(int64_t(sh) * items(side), width()); }
   // plain: the share holding list position j
-  __host__ __device__ int share_of(int64_t j) const { return int(((j + 1) * grid + items(0) - 1) / items(0)) - 1; }
+  __host__ __device__ int share_of(int64_t j) const {
+    return int(quot((j + 1) * grid + items(0) - 1, items(0))) - 1;
+  }
   // runs (= partial slots) of head h
   __host__ __device__ int nruns(int h) const {
     if (paired) return 2 * kk;
@@ -556,9 +564,15 @@ struct FusedArgs {
   // launch's workgroup count reads only the run slots)
   int empty_stats;
   int pair_e0;  // the partition (ShareMap e0_num; 0: plain)
+  ShareMap smap;  // the partition over the launch's grid (fused_grid)
   int khyb;     // 1: a hybrid K store (meta as asym, the group's flag picks sym)
   int kgs, vgs;  // log2 of the stores' group sizes over the kernel's group G (0: the same; SM = 3 instances)
 };
+// the arguments of a launch over `grid` workgroups
+inline FusedArgs fused_grid(FusedArgs a, int grid) {
+  a.smap = ShareMap::make(grid, a.nitems / a.nsplit, a.nsplit, a.pair_e0);
+  return a;
+}
 // its launch per K bit width (iq_flash_k{2,3,4}.hip)
 int flash_fused_launch_k2(const FusedArgs& a, int vbits, int group, int D, int nrep, bool norm, int* grid,
                           hipStream_t stream, bool launch);

@@ -352,7 +352,7 @@ int qk_fused_launch(const void* q, int64_t sq_b, int64_t sq_h, const void* norm,
     static detail::OccCache occ[2];  // workgroups per CU at once
     const int pc = detail::blocks_per_cu(kern, nt, occ[norm ? 1 : 0]);
     const int grid = int(std::min<int64_t>(a.nitems, int64_t(pc) * detail::num_cus()));
-    kern<<<dim3(grid), nt, 0, stream>>>(a);
+    kern<<<dim3(grid), nt, 0, stream>>>(detail::fused_grid(a, grid));
     return launch_status();
   });
   return 1;
