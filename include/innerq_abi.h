@@ -257,6 +257,14 @@ typedef struct iq_segment {
                                  IQ_MODE_BF16 bit (its rows are bf16) */
 } iq_segment;
 
+/* The dense K (axis 0: a K store, norm as iq_dequant_k) or V (axis 1: a V
+ * store, norm NULL) of seg[0..2] = [sink | packed | recent] in one launch: the
+ * dense rows copied, the packed tokens (at least one) dequantized, to out16
+ * [B,H,n0+n1+n2,D] in the segments' activation type at element strides so_b,
+ * so_h, so_t (cache.py:235-281).  D % 8 == 0. */
+int iq_read_dense(const iq_segment* seg, int axis, const void* norm, int B, int H, int D, void* out16, int64_t so_b,
+                  int64_t so_h, int64_t so_t, void* stream);
+
 /* One role (K or V) of a layer's decode-step append: the fp16 recent window
  * lives in a caller-owned buffer, and the oldest tokens flush into the
  * layer's packed store. */

@@ -83,6 +83,7 @@ SIGNATURES = {
     "iq_quantize_v": (I, [P, L, L, L, I, I, I, I, I, I, I, P, P, L, L, P, P, P, P, P]),
     "iq_dequant_k": (I, [P, P, L, P, I, I, I, I, I, I, I, I, P, P, L, L, L, P]),
     "iq_dequant_v": (I, [P, P, L, I, I, I, I, I, I, I, I, P, P, L, L, L, P]),
+    "iq_read_dense": (I, [ctypes.POINTER(iq_segment), I, P, I, I, I, P, L, L, L, P]),
     "iq_dequant_dense": (I, [P, P, P, L, L, L, I, I, I, P, P]),
     "iq_unpack_k": (I, [P, P, L, I, I, I, I, I, I, I, I, P, P, P, P]),
     "iq_unpack_v": (I, [P, P, L, I, I, I, I, I, I, I, I, P, P, P, P]),

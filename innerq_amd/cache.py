@@ -388,6 +388,9 @@ class InnerqDynamicLayer(CacheLayerMixin):
         fp32 dequantized values, as the reference's cat + .to(dtype)."""
         ns, nq, nr = sink.shape[-2], (q.length if q is not None else 0), recent.shape[-2]
         B, H, _, D = recent.shape
+        if (nq and dtype == q.store.dtype == sink.dtype == recent.dtype and D % 8 == 0
+                and sink.stride(-1) == 1 and recent.stride(-1) == 1):
+            return ops.read_dense(sink, q.store, recent, norm)
         out = torch.empty(B, H, ns + nq + nr, D, dtype=dtype, device=self.device)
         if ns:
             out[:, :, :ns].copy_(sink)

@@ -31,6 +31,35 @@ struct DeqOut {
   int vec16, vec32;  // rows take 16-byte (K) / 8-byte (V) stores of out16, 16-byte stores of out32
 };
 
+// Dense rows copied beside the packed ones (iq_read_dense): the first ns and
+// last nr tokens of every (batch, head), by the workgroups from blocks0 on,
+// one lane per 8 values.
+struct CopyRows {
+  int64_t blocks0;
+  const uint16_t *sink, *recent;
+  int64_t ss_b, ss_h, ss_t, sr_b, sr_h, sr_t;
+  uint16_t* out;        // the output's first row
+  int ns, nq, nr;       // sink, packed and recent rows
+  int H, lpr, vec;      // vec: every row takes 16-byte loads and stores
+  uint32_t items;       // B * H * (ns + nr) * lpr
+};
+__device__ __forceinline__ void copy_rows(const CopyRows& c, const DeqOut& o) {
+  const uint32_t e = uint32_t(int64_t(blockIdx.x) - c.blocks0) * 256u + threadIdx.x;
+  if (e >= c.items) return;
+  const uint32_t r = e / uint32_t(c.lpr), col = (e - r * uint32_t(c.lpr)) * 8u, per = uint32_t(c.ns + c.nr);
+  const uint32_t bh = r / per, b = bh / uint32_t(c.H), h = bh - b * uint32_t(c.H);
+  const int t = int(r - bh * per);
+  const uint16_t* src = t < c.ns ? c.sink + b * c.ss_b + h * c.ss_h + t * c.ss_t
+                                 : c.recent + b * c.sr_b + h * c.sr_h + int64_t(t - c.ns) * c.sr_t;
+  uint16_t* dst = c.out + b * o.sob + h * o.soh + int64_t(t < c.ns ? t : t + c.nq) * o.sot;
+  if (c.vec) {
+    *reinterpret_cast<uint4*>(dst + col) = *reinterpret_cast<const uint4*>(src + col);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) dst[col + i] = src[col + i];
+  }
+}
+
 // {scale, zero} of a unit and the integer subtracted from its fields:
 // value = (field - off) * s + z
 template <bool BF>
@@ -83,8 +112,12 @@ struct KDeq {
 constexpr int KU = 4;
 
 template <int BITS, int G, bool BF>
-__global__ __launch_bounds__(256) void dequant_k_kernel(KDeq a, DeqOut o) {
+__global__ __launch_bounds__(256) void dequant_k_kernel(KDeq a, DeqOut o, CopyRows cr) {
   constexpr int LPG = G / 8, W = G * BITS / 32;
+  if (int64_t(blockIdx.x) >= cr.blocks0) {
+    copy_rows(cr, o);
+    return;
+  }
   const int64_t bh = int64_t(blockIdx.x) / a.tiles, tile = int64_t(blockIdx.x) % a.tiles;
   const int ng = a.D / G;
   const bool fixed = a.lpr_sh >= 0;
@@ -192,9 +225,13 @@ struct VDeq {
 };
 
 template <int BITS, int G, bool BF>
-__global__ __launch_bounds__(256) void dequant_v_kernel(VDeq a, DeqOut o) {
+__global__ __launch_bounds__(256) void dequant_v_kernel(VDeq a, DeqOut o, CopyRows cr) {
   constexpr int W = G * BITS / 32, CPG = G / 32;  // chunks per group
   constexpr int CH = 16 / BITS;                   // fields per half
+  if (int64_t(blockIdx.x) >= cr.blocks0) {
+    copy_rows(cr, o);
+    return;
+  }
   const int64_t e = int64_t(blockIdx.x) * 256 + threadIdx.x;
   if (e >= a.items) return;
   const int64_t r = e / a.dq;
@@ -267,6 +304,35 @@ __global__ __launch_bounds__(256) void dequant_v_kernel(VDeq a, DeqOut o) {
   }
 }
 
+int launch_k(const uint32_t* codes, const uint16_t* meta, int64_t t_cap, const void* norm, int B, int H, int t0, int T,
+             int D, int group, int bits, int mode, bool bf, const DeqOut& o, CopyRows cr, int64_t copy_blocks,
+             hipStream_t st) {
+  const int lpr = D / 8;
+  const bool pow2 = (lpr & (lpr - 1)) == 0 && lpr <= 256;
+  const KDeq a{codes, meta, (const uint16_t*)norm, t_cap / TOKEN_BLOCK, H, t0, T, D, mode, lpr,
+               pow2 ? __builtin_ctz(unsigned(lpr)) : -1, ceil_div(int64_t(T) * lpr, 256 * KU)};
+  cr.blocks0 = int64_t(B) * H * a.tiles;
+  const dim3 grid(unsigned(cr.blocks0 + copy_blocks));
+  return dispatch_store_bits_group(bits, group, [&]<int BITS, int G>() {
+    auto* kern = bf ? dequant_k_kernel<BITS, G, true> : dequant_k_kernel<BITS, G, false>;
+    kern<<<grid, 256, 0, st>>>(a, o, cr);
+    return launch_status();
+  });
+}
+int launch_v(const uint32_t* codes, const uint16_t* meta, int64_t t_cap, int B, int H, int t0, int T, int D, int group,
+             int bits, int mode, bool bf, const DeqOut& o, CopyRows cr, int64_t copy_blocks, hipStream_t st) {
+  const int nch = T / 32, dq = (D + 3) / 4;
+  const VDeq a{codes, meta, t_cap / group, H, t0 / group, D, mode, nch, dq, int64_t(B) * H * nch * dq};
+  cr.blocks0 = ceil_div(a.items, 256);
+  const dim3 grid(unsigned(cr.blocks0 + copy_blocks));
+  return dispatch_store_bits_group(bits, group, [&]<int BITS, int G>() {
+    auto* kern = bf ? dequant_v_kernel<BITS, G, true> : dequant_v_kernel<BITS, G, false>;
+    kern<<<grid, 256, 0, st>>>(a, o, cr);
+    return launch_status();
+  });
+}
+bool strides_of(int64_t m, int64_t b, int64_t h, int64_t t) { return b % m == 0 && h % m == 0 && t % m == 0; }
+
 }  // namespace
 
 extern "C" {
@@ -284,18 +350,10 @@ int iq_dequant_k(const uint32_t* k_codes, const uint16_t* k_meta, int64_t t_cap,
   IQ_CHECK(t_cap % TOKEN_BLOCK == 0, IQ_ERR_ALIGN);
   IQ_CHECK(int64_t(t0) + T <= t_cap, IQ_ERR_RANGE);
   if (int64_t(B) * H * T == 0) return IQ_OK;
-  const bool s8 = so_b % 8 == 0 && so_h % 8 == 0 && so_t % 8 == 0, s4 = so_b % 4 == 0 && so_h % 4 == 0 && so_t % 4 == 0;
-  const DeqOut o{(uint16_t*)out16, out32, so_b, so_h, so_t, aligned(out16, 16) && s8, aligned(out32, 16) && s4};
-  const int lpr = D / 8;
-  const bool pow2 = (lpr & (lpr - 1)) == 0 && lpr <= 256;
-  const KDeq a{k_codes, k_meta, (const uint16_t*)norm, t_cap / TOKEN_BLOCK, H, t0, T, D, mode, lpr,
-               pow2 ? __builtin_ctz(unsigned(lpr)) : -1, ceil_div(int64_t(T) * lpr, 256 * KU)};
-  const dim3 grid(unsigned(int64_t(B) * H * a.tiles));
-  return dispatch_store_bits_group(bits, group, [&]<int BITS, int G>() {
-    auto* kern = bf ? dequant_k_kernel<BITS, G, true> : dequant_k_kernel<BITS, G, false>;
-    kern<<<grid, 256, 0, (hipStream_t)stream>>>(a, o);
-    return launch_status();
-  });
+  const DeqOut o{(uint16_t*)out16, out32, so_b, so_h, so_t, aligned(out16, 16) && strides_of(8, so_b, so_h, so_t),
+                 aligned(out32, 16) && strides_of(4, so_b, so_h, so_t)};
+  return launch_k(k_codes, k_meta, t_cap, norm, B, H, t0, T, D, group, bits, mode, bf, o, CopyRows{}, 0,
+                  (hipStream_t)stream);
 }
 
 int iq_dequant_v(const uint32_t* v_codes, const uint16_t* v_meta, int64_t t_cap, int B, int H, int t0, int T,
@@ -309,17 +367,46 @@ int iq_dequant_v(const uint32_t* v_codes, const uint16_t* v_meta, int64_t t_cap,
   IQ_CHECK(B >= 0 && H >= 0 && T >= 0 && t0 >= 0 && D > 0, IQ_ERR_SHAPE);
   IQ_CHECK(T % group == 0 && t0 % group == 0 && t_cap % group == 0, IQ_ERR_GROUP);
   IQ_CHECK(int64_t(t0) + T <= t_cap, IQ_ERR_RANGE);
-  const int nch = T / 32, dq = (D + 3) / 4;
-  const int64_t items = int64_t(B) * H * nch * dq;
-  if (items == 0) return IQ_OK;
-  const bool s4 = D % 4 == 0 && so_b % 4 == 0 && so_h % 4 == 0 && so_t % 4 == 0;
+  if (int64_t(B) * H * T == 0) return IQ_OK;
+  const bool s4 = D % 4 == 0 && strides_of(4, so_b, so_h, so_t);
   const DeqOut o{(uint16_t*)out16, out32, so_b, so_h, so_t, aligned(out16, 8) && s4, aligned(out32, 16) && s4};
-  const VDeq a{v_codes, v_meta, t_cap / group, H, t0 / group, D, mode, nch, dq, items};
-  return dispatch_store_bits_group(bits, group, [&]<int BITS, int G>() {
-    auto* kern = bf ? dequant_v_kernel<BITS, G, true> : dequant_v_kernel<BITS, G, false>;
-    kern<<<dim3(unsigned(ceil_div(items, 256))), 256, 0, (hipStream_t)stream>>>(a, o);
-    return launch_status();
-  });
+  return launch_v(v_codes, v_meta, t_cap, B, H, t0, T, D, group, bits, mode, bf, o, CopyRows{}, 0, (hipStream_t)stream);
+}
+
+int iq_read_dense(const iq_segment* s, int axis, const void* norm, int B, int H, int D, void* out16, int64_t so_b,
+                  int64_t so_h, int64_t so_t, void* stream) {
+  IQ_CHECK(s && out16, IQ_ERR_NULL);
+  IQ_CHECK(B >= 0 && H >= 0 && D > 0 && D % 8 == 0 && (axis == 0 || axis == 1), IQ_ERR_SHAPE);
+  const iq_segment &k = s[1], &a0 = s[0], &a2 = s[2];
+  IQ_CHECK(a0.n >= 0 && k.n > 0 && a2.n >= 0, IQ_ERR_SHAPE);
+  IQ_CHECK((a0.n == 0 || a0.dense) && (a2.n == 0 || a2.dense) && k.codes && k.meta, IQ_ERR_NULL);
+  const bool bf = act_bf16(k.mode);
+  const int mode = base_mode(k.mode);
+  for (const iq_segment* d : {&a0, &a2}) IQ_CHECK(d->n == 0 || d->mode == (bf ? int(IQ_MODE_BF16) : 0), IQ_ERR_MODE);
+  if (int e = check_store(k.bits, k.group, mode)) return e;
+  IQ_CHECK(k.t0 >= 0 && int64_t(k.t0) + k.n <= k.t_cap, IQ_ERR_RANGE);
+  if (axis == 0) {
+    IQ_CHECK(D % k.group == 0, IQ_ERR_GROUP);
+    IQ_CHECK(k.t_cap % TOKEN_BLOCK == 0, IQ_ERR_ALIGN);
+  } else {
+    IQ_CHECK(!norm, IQ_ERR_SHAPE);
+    IQ_CHECK(k.n % k.group == 0 && k.t0 % k.group == 0 && k.t_cap % k.group == 0, IQ_ERR_GROUP);
+  }
+  const int64_t items = int64_t(B) * H * (int64_t(a0.n) + a2.n) * (D / 8);
+  IQ_CHECK(items < (int64_t(1) << 31) && int64_t(a0.n) + k.n + a2.n < (int64_t(1) << 31), IQ_ERR_SHAPE);
+  if (int64_t(B) * H == 0) return IQ_OK;
+  uint16_t* out = (uint16_t*)out16;
+  uint16_t* mid = out + int64_t(a0.n) * so_t;
+  const bool s8 = strides_of(8, so_b, so_h, so_t), s4 = D % 4 == 0 && strides_of(4, so_b, so_h, so_t);
+  const DeqOut o{mid, nullptr, so_b, so_h, so_t, axis == 0 ? aligned(mid, 16) && s8 : aligned(mid, 8) && s4, 0};
+  auto rows16 = [](const iq_segment& d) { return d.n == 0 || (aligned(d.dense, 16) && strides_of(8, d.s_b, d.s_h, d.s_t)); };
+  CopyRows c{0, (const uint16_t*)a0.dense, (const uint16_t*)a2.dense, a0.s_b, a0.s_h, a0.s_t, a2.s_b, a2.s_h, a2.s_t,
+             out, a0.n, k.n, a2.n, H, D / 8, aligned(out, 16) && s8 && rows16(a0) && rows16(a2), uint32_t(items)};
+  const int64_t blocks = ceil_div(items, 256);
+  return axis == 0 ? launch_k(k.codes, k.meta, k.t_cap, norm, B, H, k.t0, k.n, D, k.group, k.bits, mode, bf, o, c, blocks,
+                              (hipStream_t)stream)
+                   : launch_v(k.codes, k.meta, k.t_cap, B, H, k.t0, k.n, D, k.group, k.bits, mode, bf, o, c, blocks,
+                              (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -854,6 +854,26 @@ def decode_attention_combine_live(plan, B: int, Hq: int, T: int, D: int, device,
 
 
 # --- cache-side helpers --------------------------------------------------------
+def read_dense(sink: torch.Tensor, store: PackedStore, recent: torch.Tensor,
+               norm: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """[sink | dequantized (times norm) | recent] [B,H,T,D] in the store's dtype, in one launch; the
+    store holds at least one token, sink and recent are [B,H,n,D] of its dtype."""
+    B, H, D = store.B, store.H, store.D
+    for t, role in ((sink, "sink"), (recent, "recent")):
+        require_device(t, role, store.dtype)
+        check_out((t.shape[0], t.shape[1], t.shape[3]), (B, H, D), role)
+    ns, nr = sink.shape[2], recent.shape[2]
+    seg = (_lib.iq_segment * 3)(_segment(sink, None, ns, dtype=store.dtype), _segment(None, store, store.length),
+                                _segment(recent, None, nr, dtype=store.dtype))
+    if norm is not None:
+        require_device(norm, "norm", store.dtype)
+        norm = norm.reshape(B, H, D).contiguous()
+    out = torch.empty(B, H, ns + store.length + nr, D, dtype=store.dtype, device=store.device)
+    call("iq_read_dense", seg, 0 if store.axis == "channel" else 1, _p(norm), B, H, D, _p(out), out.stride(0),
+         out.stride(1), out.stride(2), _stream(out.device))
+    return out
+
+
 def unpack_store(store: PackedStore, t0: int = 0, T: Optional[int] = None):
     """Reference-format (codes int32, scale fp16, zero | signs fp16) of store tokens [t0, t0+T);
     for a hybrid store the dicts of quant.py:146-149 (see split_hybrid)."""

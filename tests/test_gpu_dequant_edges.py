@@ -57,3 +57,26 @@ def test_dequant(act, mode, widths, axis, n, t0, D, G, layout, norm):
             st.dequant(t0, n - t0, out=out, norm=None if nf is None else nf.to(DEV))
             ref = torch.from_numpy(np.ascontiguousarray(want)).to(dtype)
             assert torch.equal(out.cpu(), ref)  # equal values: -0 == +0
+
+
+@pytest.mark.parametrize("act", ["f16", "bf16"])
+@pytest.mark.parametrize("axis,D,ns,n,nr,layout", [("channel", 128, 32, 70, 96, "plain"), ("token", 128, 0, 64, 7, "plain"),
+                                                   ("token", 64, 3, 96, 0, "plain"), ("channel", 96, 1, 1, 1, "plain"),
+                                                   ("channel", 64, 5, 129, 9, "heads last"),
+                                                   ("token", 128, 33, 32, 40, "odd rows")])
+def test_read_dense(act, axis, D, ns, n, nr, layout):
+    """[sink | packed | recent] in one launch equals the parts, for sources whose rows do or do not take
+    vector loads."""
+    B, H = 2, 3
+    dt = TD[act]
+
+    def rows(m):
+        t = view(B, H, m, D, dt, layout)
+        return t.copy_(torch.randn(B, H, m, D, device=DEV).to(dt))
+
+    sink, recent = rows(ns), rows(nr)
+    st = ops.PackedStore(axis, B, H, D, 32, 3, "symmetric", DEV, dtype=dt)
+    norm = torch.rand(B, H, 1, D, device=DEV).to(dt) + 0.5 if axis == "channel" else None
+    st.append(torch.randn(B, H, n, D, device=DEV).to(dt), norm=norm)
+    got = ops.read_dense(sink, st, recent, norm)
+    assert torch.equal(got, torch.cat([sink, st.dequant(norm=norm), recent], dim=2))
