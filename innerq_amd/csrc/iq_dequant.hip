@@ -10,8 +10,8 @@
 // the split follows the output: a lane writes 16 bytes of a row (K) or 8 (V)
 // and a wave writes whole rows.  (A thread per group, the form before, wrote
 // single halves 2 G bytes apart: 217 us for 4 x 8 heads x 16256 tokens, D =
-// 128; now 42 us for 3-bit keys with a factor and 33 us for 2-bit values, 3.8
-// and 4.7 TB/s.)  Fields become fp16 integers two at a time: one shift
+// 128; with this split 42 us for 3-bit keys with a factor and 33 us for 2-bit
+// values, and less with the stores of put.)  Fields become fp16 integers two at a time: one shift
 // and one and-or with an exponent pattern, one packed subtraction.
 #include "iq_common.h"
 #include "iq_device.h"
@@ -23,6 +23,23 @@ namespace {
 typedef float f2_t __attribute__((ext_vector_type(2)));
 typedef float f4_t __attribute__((ext_vector_type(4)));
 typedef __bf16 b2_t __attribute__((ext_vector_type(2)));
+typedef uint32_t u2_t __attribute__((ext_vector_type(2)));
+typedef uint32_t u4_t __attribute__((ext_vector_type(4)));
+
+// NT: the values leave with the non-temporal policy, where a launch writes
+// more than NT_BYTES.  Up to there the 256 MB Infinity Cache still holds a
+// layer's K and V when the model's attention reads them, and plain stores are
+// ahead over both; past it they run into its evictions.  K and V of 4 x 8
+// heads read and then reduced once, us a layer, plain / non-temporal: 64 MB
+// per tensor 70 / 76, 96 MB 91 / 99, 112 MB 119 / 113, 128 MB 150 / 134, 256
+// MB 287 / 263 (the read alone at 128 MB: 76 / 53, 6.1 TB/s).  The quantizers'
+// stores, a quarter of what they read, measure the same either way.
+constexpr int64_t NT_BYTES = int64_t(104) << 20;
+template <bool NT, typename V>
+__device__ __forceinline__ void put(void* p, V v) {
+  if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<V*>(p));
+  else *reinterpret_cast<V*>(p) = v;
+}
 
 struct DeqOut {
   uint16_t* out16;  // in the activation dtype
@@ -111,7 +128,7 @@ struct KDeq {
 };
 constexpr int KU = 4;
 
-template <int BITS, int G, bool BF>
+template <int BITS, int G, bool BF, bool NT>
 __global__ __launch_bounds__(256) void dequant_k_kernel(KDeq a, DeqOut o, CopyRows cr) {
   constexpr int LPG = G / 8, W = G * BITS / 32;
   if (int64_t(blockIdx.x) >= cr.blocks0) {
@@ -195,7 +212,7 @@ __global__ __launch_bounds__(256) void dequant_k_kernel(KDeq a, DeqOut o, CopyRo
         for (int i = 0; i < 4; ++i) p[i] = out_pair<BF>(v[2 * i], v[2 * i + 1]);
       }
       if (o.vec16) {
-        *reinterpret_cast<uint4*>(o.out16 + at) = make_uint4(p[0], p[1], p[2], p[3]);
+        put<NT>(o.out16 + at, u4_t{p[0], p[1], p[2], p[3]});
       } else {
 #pragma unroll
         for (int i = 0; i < 8; ++i) o.out16[at + i] = uint16_t(p[i / 2] >> (16 * (i & 1)));
@@ -203,8 +220,8 @@ __global__ __launch_bounds__(256) void dequant_k_kernel(KDeq a, DeqOut o, CopyRo
     }
     if (o.out32) {
       if (o.vec32) {
-        *reinterpret_cast<f4_t*>(o.out32 + at) = f4_t{v[0], v[1], v[2], v[3]};
-        *reinterpret_cast<f4_t*>(o.out32 + at + 4) = f4_t{v[4], v[5], v[6], v[7]};
+        put<NT>(o.out32 + at, f4_t{v[0], v[1], v[2], v[3]});
+        put<NT>(o.out32 + at + 4, f4_t{v[4], v[5], v[6], v[7]});
       } else {
 #pragma unroll
         for (int i = 0; i < 8; ++i) o.out32[at + i] = v[i];
@@ -224,7 +241,7 @@ struct VDeq {
   int64_t items;  // B * H * nch * dq
 };
 
-template <int BITS, int G, bool BF>
+template <int BITS, int G, bool BF, bool NT>
 __global__ __launch_bounds__(256) void dequant_v_kernel(VDeq a, DeqOut o, CopyRows cr) {
   constexpr int W = G * BITS / 32, CPG = G / 32;  // chunks per group
   constexpr int CH = 16 / BITS;                   // fields per half
@@ -284,7 +301,7 @@ __global__ __launch_bounds__(256) void dequant_v_kernel(VDeq a, DeqOut o, CopyRo
         if (num) { p0 = out_pair_num<BF>(v[0], v[1]); p1 = out_pair_num<BF>(v[2], v[3]); }
         else { p0 = out_pair<BF>(v[0], v[1]); p1 = out_pair<BF>(v[2], v[3]); }
         if (o.vec16) {
-          *reinterpret_cast<uint2*>(o.out16 + at_t) = make_uint2(p0, p1);
+          put<NT>(o.out16 + at_t, u2_t{p0, p1});
         } else {
 #pragma unroll
           for (int c = 0; c < 4; ++c)
@@ -293,7 +310,7 @@ __global__ __launch_bounds__(256) void dequant_v_kernel(VDeq a, DeqOut o, CopyRo
       }
       if (o.out32) {
         if (o.vec32) {
-          *reinterpret_cast<f4_t*>(o.out32 + at_t) = f4_t{v[0], v[1], v[2], v[3]};
+          put<NT>(o.out32 + at_t, f4_t{v[0], v[1], v[2], v[3]});
         } else {
 #pragma unroll
           for (int c = 0; c < 4; ++c)
@@ -304,6 +321,9 @@ __global__ __launch_bounds__(256) void dequant_v_kernel(VDeq a, DeqOut o, CopyRo
   }
 }
 
+bool streams(int64_t B, int64_t H, int64_t T, int64_t D, const DeqOut& o) {
+  return B * H * T * D * ((o.out16 ? 2 : 0) + (o.out32 ? 4 : 0)) > NT_BYTES;
+}
 int launch_k(const uint32_t* codes, const uint16_t* meta, int64_t t_cap, const void* norm, int B, int H, int t0, int T,
              int D, int group, int bits, int mode, bool bf, const DeqOut& o, CopyRows cr, int64_t copy_blocks,
              hipStream_t st) {
@@ -312,9 +332,12 @@ int launch_k(const uint32_t* codes, const uint16_t* meta, int64_t t_cap, const v
   const KDeq a{codes, meta, (const uint16_t*)norm, t_cap / TOKEN_BLOCK, H, t0, T, D, mode, lpr,
                pow2 ? __builtin_ctz(unsigned(lpr)) : -1, ceil_div(int64_t(T) * lpr, 256 * KU)};
   cr.blocks0 = int64_t(B) * H * a.tiles;
+  const bool nt = streams(B, H, T, D, o);
   const dim3 grid(unsigned(cr.blocks0 + copy_blocks));
   return dispatch_store_bits_group(bits, group, [&]<int BITS, int G>() {
-    auto* kern = bf ? dequant_k_kernel<BITS, G, true> : dequant_k_kernel<BITS, G, false>;
+    auto* kern = bf   ? (nt ? dequant_k_kernel<BITS, G, true, true> : dequant_k_kernel<BITS, G, true, false>)
+                 : nt ? dequant_k_kernel<BITS, G, false, true>
+                      : dequant_k_kernel<BITS, G, false, false>;
     kern<<<grid, 256, 0, st>>>(a, o, cr);
     return launch_status();
   });
@@ -324,9 +347,12 @@ int launch_v(const uint32_t* codes, const uint16_t* meta, int64_t t_cap, int B, 
   const int nch = T / 32, dq = (D + 3) / 4;
   const VDeq a{codes, meta, t_cap / group, H, t0 / group, D, mode, nch, dq, int64_t(B) * H * nch * dq};
   cr.blocks0 = ceil_div(a.items, 256);
+  const bool nt = streams(B, H, T, D, o);
   const dim3 grid(unsigned(cr.blocks0 + copy_blocks));
   return dispatch_store_bits_group(bits, group, [&]<int BITS, int G>() {
-    auto* kern = bf ? dequant_v_kernel<BITS, G, true> : dequant_v_kernel<BITS, G, false>;
+    auto* kern = bf   ? (nt ? dequant_v_kernel<BITS, G, true, true> : dequant_v_kernel<BITS, G, true, false>)
+                 : nt ? dequant_v_kernel<BITS, G, false, true>
+                      : dequant_v_kernel<BITS, G, false, false>;
     kern<<<grid, 256, 0, st>>>(a, o, cr);
     return launch_status();
   });

@@ -80,3 +80,15 @@ def test_read_dense(act, axis, D, ns, n, nr, layout):
     st.append(torch.randn(B, H, n, D, device=DEV).to(dt), norm=norm)
     got = ops.read_dense(sink, st, recent, norm)
     assert torch.equal(got, torch.cat([sink, st.dequant(norm=norm), recent], dim=2))
+
+
+@pytest.mark.parametrize("axis", ["channel", "token"])
+def test_large_reads_equal_small_ones(axis):
+    """A read past the size where the stores stream equals the same tokens read in pieces below it."""
+    B, H, T, D = 2, 8, 26624, 128  # 109 MB in fp16
+    st = ops.PackedStore(axis, B, H, D, 32, 3, "symmetric", DEV)
+    st.append(torch.randn(B, H, T, D, device=DEV).half())
+    for dtype in (torch.float16, torch.float32):
+        whole = st.dequant(dtype=dtype)
+        for t0 in range(0, T, 6656):
+            assert torch.equal(whole[:, :, t0:t0 + 6656], st.dequant(t0, 6656, dtype=dtype))
