@@ -9,10 +9,11 @@
 // Bound: HBM, and by its writes (2 B out against b/8 + m/G B in per value), so
 // the split follows the output: a lane writes 16 bytes of a row (K) or 8 (V)
 // and a wave writes whole rows.  (A thread per group, the form before, wrote
-// single halves 2 G bytes apart: 217 us for 4 x 8 heads x 16256 tokens, D =
-// 128; with this split 42 us for 3-bit keys with a factor and 33 us for 2-bit
-// values, and less with the stores of put.)  Fields become fp16 integers two at a time: one shift
-// and one and-or with an exponent pattern, one packed subtraction.
+// single halves, of keys 2 G bytes apart: 393 us for 3-bit keys with a factor
+// of 4 x 8 heads x 16256 tokens, D = 128, and 42 us for 2-bit values; with this
+// split 42 and 33 us, and 28 and 26 with the stores of put.)  Fields become
+// fp16 integers two at a time: one shift and one and-or with an exponent
+// pattern, one packed subtraction.
 #include "iq_common.h"
 #include "iq_device.h"
 

@@ -923,7 +923,9 @@ def key_norm_factor(k: torch.Tensor) -> torch.Tensor:
     B, H, T, D = k.shape
     out = torch.empty(B, H, 1, D, dtype=k.dtype, device=k.device)
     nbytes = _lib.lib().iq_key_norm_workspace_bytes(B, H, T, D)
-    ws = _workspace(k.device, nbytes) if nbytes else None
+    # a tensor of its own: a first call under graph capture must not leave the stream's kept workspace
+    # in the capture's memory pool
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=k.device) if nbytes else None
     call("iq_key_norm_factor_ws", _p(k), k.stride(0), k.stride(1), k.stride(2), B, H, T, D, act_flag(k.dtype),
          _p(out), _p(ws), ws.numel() if nbytes else 0, _stream(k.device))
     return out
