@@ -195,7 +195,7 @@ __global__ __launch_bounds__((avc_waves<VB, G, NREP>() * 64)) void av_cols_kerne
     for (int j = 0; j < SPL; ++j) o[h][j] = 0.f;
   auto compute = [&](const Buf& bf) {
     f4_t dv[SPL][NQ], dsum[NQ];
-    group_mfma_biased_sums<VB, G, NREP, SPL, RS>(bf.w, rec + gs * SS, hl, prv, srv, dv, dsum);
+    group_mfma_sums<VB, G, NREP, SPL, true, RS>(bf.w, rec + gs * SS, hl, prv, srv, dv, dsum);
     float ps[NREP], pbs[NREP];  // sum(p), sum(p * bias) of the lane's group: lanes hl = 0, 1 of each block
 #pragma unroll
     for (int h = 0; h < NREP; ++h) {

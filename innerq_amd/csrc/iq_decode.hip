@@ -1049,8 +1049,10 @@ int launch_splits(const void* q, int64_t sq_b, int64_t sq_h, const void* norm, c
   // is known, if no (batch, KV head) has more fused runs than that kernel
   // takes.  Heads spread over more workgroups (a small batch over a long
   // context) take the slices and the combine, which reads every slot in one
-  // round of loads.
-  const bool merge_cand = mo && live && fused && n_dense > 0 && n_dense <= MERGE_DENSE_MAX;
+  // round of loads.  So do K and V of different group sizes: a slice's
+  // probabilities are rounded against its own maximum, a section's second
+  // chunk's against a running one, and these calls keep the slices' values.
+  const bool merge_cand = mo && live && fused && one_group && n_dense > 0 && n_dense <= MERGE_DENSE_MAX;
   if (n_dense > 0 && !merge_cand)
     if (int e = launch_slices()) return e;
 

@@ -53,6 +53,7 @@ int flash_fused_launch(const void* q, int64_t sq_b, int64_t sq_h, const void* no
   a.v_meta_bytes = uint32_t(int64_t(T / v.group) * D * (a.vsym ? 2 : 4));
   a.q_bytes = uint32_t((int64_t(Hq / Hkv - 1) * sq_h + D) * 2);
   a.norm_bytes = norm ? uint32_t(D * 2) : 0u;
+  a.scale = scale;
   a.scale_log2 = scale * 1.4426950408889634f;
   a.ml = ml; a.part = part;
   a.empty_stats = grid ? 0 : 1;  // a caller that takes the workgroup count reads only the run slots

@@ -312,13 +312,14 @@ __device__ __forceinline__ void group_mfma_biased(const uint32_t (&w)[NB][G * BI
   mfma_chunks<BITS, G, NREP, NB, 0, NCH, true>(w, rec, hl, pr, dv);
 }
 
-// group_mfma_biased from zero accumulators, plus the record rows' sums:
-// dsum[q] element i holds, in the lanes with hl = 0, sum(p) of head 4q + i
-// over the group and, in the lanes with hl = 1, sum(p * bias) (SumRegs).
-template <int BITS, int G, int NREP, int NB, int RS = G / 2, typename P>
-__device__ __forceinline__ void group_mfma_biased_sums(const uint32_t (&w)[NB][G * BITS / 32], P rec, int hl,
-                                                       const PlanRegs<BITS>& pr, const SumRegs<BITS>& sr,
-                                                       f4_t (&dv)[NB][(NREP + 3) / 4], f4_t (&dsum)[(NREP + 3) / 4]) {
+// group_mfma (or, BIASED, the products of the biased pairs from zero
+// accumulators) plus the record rows' sums: dsum[q] element i holds, in the
+// lanes with hl = 0, sum(p) of head 4q + i over the group and, in the lanes
+// with hl = 1, sum(p * bias) (SumRegs).
+template <int BITS, int G, int NREP, int NB, bool BIASED, int RS = G / 2, typename P>
+__device__ __forceinline__ void group_mfma_sums(const uint32_t (&w)[NB][G * BITS / 32], P rec, int hl,
+                                                const PlanRegs<BITS>& pr, const SumRegs<BITS>& sr,
+                                                f4_t (&dv)[NB][(NREP + 3) / 4], f4_t (&dsum)[(NREP + 3) / 4]) {
   constexpr int NP = G / 2;
   constexpr int NCH = NP <= IQ_MFMA_CH ? 1 : NP / IQ_MFMA_CH;
 #pragma unroll
@@ -327,7 +328,7 @@ __device__ __forceinline__ void group_mfma_biased_sums(const uint32_t (&w)[NB][G
 #pragma unroll
     for (int j = 0; j < NB; ++j) dv[j][q] = f4_t{0.f, 0.f, 0.f, 0.f};
   }
-  mfma_chunks<BITS, G, NREP, NB, 0, NCH, true, true, RS>(w, rec, hl, pr, dv, &sr, &dsum[0]);
+  mfma_chunks<BITS, G, NREP, NB, 0, NCH, BIASED, true, RS>(w, rec, hl, pr, dv, &sr, &dsum[0]);
 }
 
 // Query dot products of NB code sets: d[j][h] = sum_i q'[h,i] c_j[i] over the
@@ -422,7 +423,7 @@ int av_main_launch(const uint32_t* rec, const uint32_t* v_codes, const uint16_t*
 int av_combine_launch(const float* part, int nsplit, int B, int Hq, int D, const OutPair& o, int accumulate,
                       hipStream_t stream, int grid = 0, int nrep = 1);
 // The fused flash-decoding kernel (QK^T + softmax + attn.V, persistent) for
-// K and V stores of the same group size (any bit widths); writes split
+// K and V stores of any bit widths and group sizes; writes split
 // statistics and partials that the same combine merges as the unfused path's.
 struct FusedStore {
   const uint32_t* codes;
@@ -567,6 +568,7 @@ struct FusedArgs {
   ShareMap smap;  // the partition over the launch's grid (fused_grid)
   int khyb;     // 1: a hybrid K store (meta as asym, the group's flag picks sym)
   int kgs, vgs;  // log2 of the stores' group sizes over the kernel's group G (0: the same; SM = 3 instances)
+  float scale;  // SM = 3 instances
 };
 // the arguments of a launch over `grid` workgroups
 inline FusedArgs fused_grid(FusedArgs a, int grid) {
