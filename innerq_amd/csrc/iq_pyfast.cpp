@@ -184,6 +184,12 @@ bool ints(PyObject* const* a, std::initializer_list<int> at, int64_t* v) {
   return true;
 }
 
+// the token count T of a GEMV from t0 on (None: to the store's end); a negative one stays negative
+bool tokens_of(PyObject* o, int64_t t0, const Store& s, int64_t* T) {
+  if (o == Py_None) { *T = s.length - t0; return true; }
+  return ints(&o, {0}, T);
+}
+
 // decode(q, k_sink, k_sink0, k_store, k_t0, k_len, k_recent, k_r0, k_rn, v_sink, v_sink0, v_store, v_t0, v_len,
 //        v_recent, v_r0, v_rn, scale, norm, out, nd): q [B,Hq,D] (nd = 3) or [B,Hq,1,D] (nd = 4); the sinks' rows from
 // *_sink0 on, the stores' tokens [t0, len) (len -1: all), the recents' rows [r0, r0 + rn) (rn -1: the rest).  Returns
@@ -244,20 +250,20 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t na) {
   return THPVariable_Wrap(std::move(out));
 }
 
-// qk(q, store, scale, norm, t0, T, out): T -1: to the store's end
+// qk(q, store, scale, norm, t0, T, out): T None: to the store's end
 PyObject* qk(PyObject*, PyObject* const* a, Py_ssize_t na) {
   if (na != 7) Py_RETURN_NONE;
-  int64_t v[2];
+  int64_t t0, T;
   const at::Tensor* q = tensor_of(a[0]);
   Store s;
-  if (!ints(a, {4, 5}, v) || !q || q->dim() != 3 || q->scalar_type() != at::kHalf || q->stride(2) != 1 ||
-      !store_of(a[1], &s))
+  if (!ints(a, {4}, &t0) || !q || q->dim() != 3 || q->scalar_type() != at::kHalf || q->stride(2) != 1 ||
+      !store_of(a[1], &s) || !tokens_of(a[5], t0, s, &T))
     Py_RETURN_NONE;
-  const int64_t B = q->size(0), Hq = q->size(1), D = q->size(2), t0 = v[0], T = v[1] < 0 ? s.length - t0 : v[1];
+  const int64_t B = q->size(0), Hq = q->size(1), D = q->size(2);
   const int dev = q->get_device();
   const void* norm;
   if (!s.channel || s.dtype != at::kHalf || s.device != dev || s.B != B || s.D != D || s.H <= 0 || Hq % s.H || t0 < 0 ||
-      T <= 0 || t0 + T > s.length || B <= 0 || !norm_of(a[3], B * s.H * D, at::kHalf, dev, &norm))
+      T <= 0 || t0 > s.length || T > s.length - t0 || B <= 0 || !norm_of(a[3], B * s.H * D, at::kHalf, dev, &norm))
     Py_RETURN_NONE;
   const double scale = PyFloat_AsDouble(a[2]);
   if (scale == -1.0 && PyErr_Occurred()) { PyErr_Clear(); Py_RETURN_NONE; }
@@ -292,19 +298,19 @@ PyObject* qk(PyObject*, PyObject* const* a, Py_ssize_t na) {
   return THPVariable_Wrap(std::move(out));
 }
 
-// av(p, store, t0, T, out): the fp16 output alone, written (not accumulated)
+// av(p, store, t0, T, out): the fp16 output alone, written (not accumulated); T None: to the store's end
 PyObject* av(PyObject*, PyObject* const* a, Py_ssize_t na) {
   if (na != 5) Py_RETURN_NONE;
-  int64_t v[2];
+  int64_t t0, T;
   const at::Tensor* p = tensor_of(a[0]);
   Store s;
-  if (!ints(a, {2, 3}, v) || !p || p->dim() != 3 || p->scalar_type() != at::kHalf || p->stride(2) != 1 ||
-      !store_of(a[1], &s))
+  if (!ints(a, {2}, &t0) || !p || p->dim() != 3 || p->scalar_type() != at::kHalf || p->stride(2) != 1 ||
+      !store_of(a[1], &s) || !tokens_of(a[3], t0, s, &T))
     Py_RETURN_NONE;
-  const int64_t B = p->size(0), Hq = p->size(1), t0 = v[0], T = v[1] < 0 ? s.length - t0 : v[1];
+  const int64_t B = p->size(0), Hq = p->size(1);
   const int dev = p->get_device();
   if (s.channel || s.dtype != at::kHalf || s.device != dev || s.B != B || s.H <= 0 || Hq % s.H || t0 < 0 || T <= 0 ||
-      t0 + T > s.length || p->size(2) < T || B <= 0)
+      t0 > s.length || T > s.length - t0 || p->size(2) < T || B <= 0)
     Py_RETURN_NONE;
   const at::Tensor* given = nullptr;
   if (a[4] != Py_None) {

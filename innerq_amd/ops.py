@@ -659,7 +659,7 @@ def qk_gemv(q: torch.Tensor, k: PackedStore, scale: float, norm: Optional[torch.
     """logits [B,Hq,T] fp32 = scale * q . K[t0:t0+T] over a channel-grouped store."""
     fast = _native(q)
     if fast is not None:
-        r = fast.qk(q, k, scale, norm, t0, -1 if T is None else T, out)
+        r = fast.qk(q, k, scale, norm, t0, T, out)
         if r is not None:
             return r
     require_f16_store(k, "qk_gemv")
@@ -690,7 +690,7 @@ def av_gemv(p: torch.Tensor, v: PackedStore, t0: int = 0, T: Optional[int] = Non
     """out [B,Hq,D] = p . V[t0:t0+T] over a token-grouped store (fp16 and/or fp32 outputs)."""
     fast = _native(p) if out32 is None and not accumulate else None
     if fast is not None:
-        r = fast.av(p, v, t0, -1 if T is None else T, out)
+        r = fast.av(p, v, t0, T, out)
         if r is not None:
             return r
     require_f16_store(v, "av_gemv")

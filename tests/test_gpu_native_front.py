@@ -112,6 +112,27 @@ def test_errors_are_the_general_paths(general, bad):
     assert type(fast.value) is type(slow.value) and str(fast.value) == str(slow.value)
 
 
+@pytest.mark.parametrize("t0,T", [(0, -1), (0, -5), (64, -1), (0, 257), (64, 193), (-64, None), (320, None), (0, 0),
+                                  (2 ** 62, 2 ** 62), (0, 10 ** 30), (0, 1.5)])
+@pytest.mark.parametrize("role", ["qk", "av"])
+def test_gemv_ranges_are_the_general_paths(general, role, t0, T):
+    """A token range outside the store's, a negative count among them, is refused as the general path
+    refuses it; an empty one gives what it gives."""
+    x, ks, vs = stores(torch.float16)
+    q = torch.randn(2, 8, 128, device=DEV).half()
+    p = torch.rand(2, 8, 256, device=DEV).half()
+
+    def call():
+        try:
+            return (ops.qk_gemv(q, ks, 0.1, t0=t0, T=T) if role == "qk" else ops.av_gemv(p, vs, t0=t0, T=T)).shape
+        except Exception as e:
+            return type(e), str(e)
+
+    got = call()
+    assert got == general(call)
+    assert T == 0 or not isinstance(got, torch.Size)
+
+
 @pytest.mark.parametrize("preset", ["innerq_base", "innerq_hybrid"])
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
 def test_layer_steps(general, preset, dt):
