@@ -69,8 +69,10 @@ const at::Tensor* tensor_of(PyObject* o) {
 bool act_dtype(at::ScalarType d) { return d == at::kHalf || d == at::kBFloat16; }
 int act_flag(at::ScalarType d) { return d == at::kBFloat16 ? IQ_MODE_BF16 : 0; }
 
-// a PackedStore's fields (its tensors kept alive by the store itself)
+// a PackedStore's fields.  The tensors are held here: while the kernels are
+// enqueued another thread may run, grow the store and drop them
 struct Store {
+  at::Tensor codes_t, meta_t;
   const uint32_t* codes;
   uint16_t* meta;
   int64_t B, H, D, t_cap, length, bits, group, mode;
@@ -91,6 +93,8 @@ bool store_of(PyObject* o, Store* s) {
     ok = ct && mt && ct->scalar_type() == at::kInt && mt->scalar_type() == at::kShort && ct->is_contiguous() &&
          mt->is_contiguous();
     if (ok) {
+      s->codes_t = *ct;
+      s->meta_t = *mt;
       s->codes = (const uint32_t*)ct->data_ptr();
       s->meta = (uint16_t*)mt->data_ptr();
       s->device = ct->get_device();
@@ -114,12 +118,14 @@ bool stream_of(int device, void** stream, PyObject** key) {  // key: new referen
   if (!*key || PyErr_Occurred()) { Py_XDECREF(*key); PyErr_Clear(); return false; }
   return true;
 }
-// the stream's workspace where it is large enough (the wrapper makes or grows it)
-bool workspace_of(PyObject* key, size_t need, void** ws, size_t* bytes) {
+// the stream's workspace where it is large enough (the wrapper makes or grows
+// it), held in *hold: a thread that needs a larger one replaces it
+bool workspace_of(PyObject* key, size_t need, at::Tensor* hold, void** ws, size_t* bytes) {
   PyObject* w = PyDict_GetItemWithError(fn.workspaces, key);
   if (!w) { PyErr_Clear(); return false; }
   const at::Tensor* t = tensor_of(w);
   if (!t || size_t(t->numel()) < need) return false;
+  *hold = *t;
   *ws = t->data_ptr();
   *bytes = size_t(t->numel());
   return true;
@@ -144,12 +150,11 @@ bool dense_segment(PyObject* o, int64_t r0, int64_t n, int64_t B, int64_t H, int
   g->dense = (const char*)t->data_ptr() + r0 * g->s_t * 2;
   return true;
 }
-// tokens [t0, len) of a store
+// tokens [t0, len) of a store (its fields, and the hold on its tensors, in s)
 bool packed_segment(PyObject* o, int64_t t0, int64_t len, bool channel, int64_t B, int64_t* H, int64_t D,
-                    at::ScalarType dt, int device, iq_segment* g) {
+                    at::ScalarType dt, int device, Store& s, iq_segment* g) {
   g->n = 0;
   if (o == Py_None) return t0 == 0;
-  Store s;
   if (!store_of(o, &s)) return false;
   if (len < 0) len = s.length;
   if (s.channel != channel || s.B != B || s.D != D || s.dtype != dt || s.device != device || (*H >= 0 && s.H != *H) ||
@@ -206,9 +211,10 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t na) {
   const at::ScalarType dt = q->scalar_type();
   const int dev = q->get_device();
   iq_segment ks[3] = {}, vs[3] = {};
+  Store kst, vst;
   int64_t H = -1;
-  if (!packed_segment(a[3], v[1], v[2], true, B, &H, D, dt, dev, &ks[1]) ||
-      !packed_segment(a[11], v[6], v[7], false, B, &H, D, dt, dev, &vs[1]) || H <= 0 || Hq % H ||
+  if (!packed_segment(a[3], v[1], v[2], true, B, &H, D, dt, dev, kst, &ks[1]) ||
+      !packed_segment(a[11], v[6], v[7], false, B, &H, D, dt, dev, vst, &vs[1]) || H <= 0 || Hq % H ||
       !dense_segment(a[1], v[0], a[1] == Py_None ? 0 : -1, B, H, D, dt, dev, &ks[0]) ||
       !dense_segment(a[6], v[3], a[6] == Py_None ? 0 : v[4], B, H, D, dt, dev, &ks[2]) ||
       !dense_segment(a[9], v[5], a[9] == Py_None ? 0 : -1, B, H, D, dt, dev, &vs[0]) ||
@@ -229,9 +235,10 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t na) {
   }
   void *stream, *ws;
   size_t wsb;
+  at::Tensor hold;
   PyObject* key;
   if (!stream_of(dev, &stream, &key)) Py_RETURN_NONE;
-  const bool have = workspace_of(key, fn.decode_ws(int(B), int(Hq), int(T), int(D)), &ws, &wsb);
+  const bool have = workspace_of(key, fn.decode_ws(int(B), int(Hq), int(T), int(D)), &hold, &ws, &wsb);
   Py_DECREF(key);
   if (!have) Py_RETURN_NONE;
   at::Tensor out;
@@ -276,9 +283,10 @@ PyObject* qk(PyObject*, PyObject* const* a, Py_ssize_t na) {
   }
   void *stream, *ws;
   size_t wsb;
+  at::Tensor hold;
   PyObject* key;
   if (!stream_of(dev, &stream, &key)) Py_RETURN_NONE;
-  const bool have = workspace_of(key, fn.qk_ws(int(B), int(Hq), int(D)), &ws, &wsb);
+  const bool have = workspace_of(key, fn.qk_ws(int(B), int(Hq), int(D)), &hold, &ws, &wsb);
   Py_DECREF(key);
   if (!have) Py_RETURN_NONE;
   at::Tensor out;
@@ -321,9 +329,10 @@ PyObject* av(PyObject*, PyObject* const* a, Py_ssize_t na) {
   }
   void *stream, *ws;
   size_t wsb;
+  at::Tensor hold;
   PyObject* key;
   if (!stream_of(dev, &stream, &key)) Py_RETURN_NONE;
-  const bool have = workspace_of(key, fn.av_ws(int(B), int(Hq), int(T), int(s.D), int(s.group)), &ws, &wsb);
+  const bool have = workspace_of(key, fn.av_ws(int(B), int(Hq), int(T), int(s.D), int(s.group)), &hold, &ws, &wsb);
   Py_DECREF(key);
   if (!have) Py_RETURN_NONE;
   at::Tensor out;
@@ -346,6 +355,8 @@ PyObject* av(PyObject*, PyObject* const* a, Py_ssize_t na) {
 // one role of a window append: its iq_window, and the state after it
 struct Role {
   iq_window w{};
+  at::Tensor buf;  // the window's and the store's tensors, held through the launch
+  Store s;
   PyObject *win = nullptr, *store = nullptr;
   int64_t start, n, shadow, length, flush;
   bool deq;
@@ -363,9 +374,11 @@ bool role_of(PyObject* win, PyObject* x, PyObject* flush, PyObject* store, PyObj
   r->flush = PyLong_AsLongLong(flush);
   PyObject* bo = PyObject_GetAttr(win, S_buf);
   PyObject* dq = PyObject_GetAttr(win, S_deq_rows);
-  const at::Tensor* buf = bo ? tensor_of(bo) : nullptr;
+  const at::Tensor* bt = bo ? tensor_of(bo) : nullptr;
+  if (bt) r->buf = *bt;
+  const at::Tensor* buf = bt ? &r->buf : nullptr;
   r->deq = dq == Py_True;
-  Py_XDECREF(bo);  // the window keeps it
+  Py_XDECREF(bo);
   Py_XDECREF(dq);
   const at::Tensor* t = tensor_of(x);
   if (PyErr_Occurred()) { PyErr_Clear(); return false; }
@@ -386,7 +399,7 @@ bool role_of(PyObject* win, PyObject* x, PyObject* flush, PyObject* store, PyObj
   w.sx_b = t->stride(0); w.sx_h = t->stride(1); w.sx_t = t->stride(2);
   w.m = int(m); w.flush = int(r->flush);
   if (r->flush) {
-    Store s;
+    Store& s = r->s;
     if (store == Py_None || !store_of(store, &s) || s.dtype != t->scalar_type() || s.device != *dev || s.B != *B ||
         s.H != *H || s.D != *D || s.length + r->flush > s.t_cap || (!s.channel && r->flush % s.group))
       return false;

@@ -1,10 +1,12 @@
 """The native call front (csrc/iq_pyfast.cpp) against the general Python path over the forms it accepts and
 the ones it passes on: the same kernels with the same arguments, so the same bits, the same errors and
 the same state afterwards.  (Runs short enough that no wave order varies between calls.)"""
+import ctypes
+
 import pytest
 import torch
 
-from innerq_amd import ops
+from innerq_amd import _lib, ops
 from innerq_amd.cache import InnerqDynamicLayer
 from innerq_amd.presets import preset_config
 
@@ -176,3 +178,66 @@ def test_streams_and_capture(general):
         torch.cuda.synchronize()
         assert torch.equal(out, want)
         ops.decode_attention(q, None, ks, None, None, vs, None, 0.1)
+
+
+ENTRIES = ("iq_decode_workspace_bytes", "iq_decode_attention", "iq_qk_workspace_bytes", "iq_qk_gemv",
+           "iq_av_workspace_bytes", "iq_av_gemv", "iq_window_append")
+ENTRY = {"decode": ENTRIES[1], "qk": ENTRIES[3], "av": ENTRIES[5], "append": ENTRIES[6]}
+
+
+def entered_as(entry, stand_in, call):
+    """call() with the front's C entry point replaced by the Python function ``stand_in`` (its status)."""
+    name = ENTRY[entry]
+    fake = ctypes.CFUNCTYPE(ctypes.c_int, *[t if issubclass(t, ctypes._SimpleCData) else ctypes.c_void_p
+                                            for t in _lib.SIGNATURES[name][1]])(stand_in)
+    at = {n: ctypes.cast(getattr(_lib.lib(), n), ctypes.c_void_p).value for n in ENTRIES}
+    at[name] = ctypes.cast(fake, ctypes.c_void_p).value
+    try:
+        ops._native(torch.empty(0, device=DEV)).bind(tuple(at[n] for n in ENTRIES), ops._WS,
+                                                     torch._C._cuda_getCurrentRawStream)
+        return call()
+    finally:
+        ops._fast = None  # bound to the library again by the next call
+
+
+def four_calls():
+    """The four entries' calls over one pair of stores and windows."""
+    x, ks, vs = stores(torch.float16)
+    q = torch.randn(2, 8, 128, device=DEV).half()
+    p = torch.rand(2, 8, 256, device=DEV).half()
+    kwin, vwin = (ops.RecentWindow(x[:, :, :40]) for _ in range(2))
+    new = x[:, :, 40:41].contiguous()
+    ks.reserve(512)
+    vs.reserve(512)
+    return ks, vs, kwin, vwin, {
+        "decode": lambda: ops.decode_attention(q, None, ks, None, None, vs, None, 0.1),
+        "qk": lambda: ops.qk_gemv(q, ks, 0.1), "av": lambda: ops.av_gemv(p, vs),
+        "append": lambda: ops.window_append(kwin, new, 32, ks, None, vwin, new, 32, vs)}
+
+
+@pytest.mark.parametrize("entry", ["decode", "qk", "av", "append"])
+def test_tensors_are_held_while_other_threads_run(entry):
+    """The front lets other threads run while it enqueues kernels.  What one of them may do meanwhile (a
+    larger workspace for the stream, a store or a window that grows) frees none of the call's memory.  The
+    entry point is stood in for by a function that drops every reference Python has; no kernel runs."""
+    ks, vs, kwin, vwin, calls = four_calls()
+    if entry != "append":
+        calls[entry]()  # the stream's workspace
+        kwin.buf = vwin.buf = None
+    if entry in ("qk", "av"):  # the other role's store is not this call's
+        other = vs if entry == "qk" else ks
+        other.codes = other.meta = None
+    freed = []
+
+    def during(*_):
+        before = torch.cuda.memory_allocated()
+        if entry != "append":
+            del ops._WS[(0, torch.cuda.current_stream().cuda_stream)]
+        for t in (ks, vs):
+            t.codes = t.meta = None
+        kwin.buf = vwin.buf = None
+        freed.append(before - torch.cuda.memory_allocated())
+        return 0
+
+    entered_as(entry, during, calls[entry])
+    assert freed == [0]
