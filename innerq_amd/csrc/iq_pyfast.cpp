@@ -9,8 +9,12 @@
 // 72 (24).  Each function here
 // returns None when anything is out of the ordinary (a shape, type, stride or
 // state that the wrapper converts or refuses, a buffer that has to grow, an
-// error status): nothing has been launched or changed then, and the wrapper's
-// general path runs and decides, so results and errors are its own.
+// argument that the entry point refuses): no window or store has been changed
+// then, and the wrapper's general path runs and decides, so results and errors
+// are its own.  A failed launch (IQ_ERR_HIP, which an earlier call's error also
+// gives) is raised from here as the general path raises it: the kernel may have
+// run, and an append run twice would quantize the rows that it left in the
+// window in place of the tokens.
 //
 // A CPython extension over libtorch's tensors; the kernels are entered through
 // the C ABI's function addresses, handed in by bind().
@@ -179,6 +183,17 @@ bool norm_of(PyObject* o, int64_t numel, at::ScalarType dt, int device, const vo
   return true;
 }
 
+// what a call returns whose entry point returned status st (not IQ_OK)
+PyObject* not_ok(const char* name, int st) {
+  if (st != IQ_ERR_HIP) Py_RETURN_NONE;
+  PyObject* m = PyImport_ImportModule("innerq_amd._lib");
+  PyObject* e = m ? PyObject_CallMethod(m, "IQError", "si", name, st) : nullptr;
+  if (e) PyErr_SetObject((PyObject*)Py_TYPE(e), e);
+  Py_XDECREF(e);
+  Py_XDECREF(m);
+  return nullptr;
+}
+
 bool ints(PyObject* const* a, std::initializer_list<int> at, int64_t* v) {
   for (int i : at) {
     if (!PyLong_Check(a[i])) return false;
@@ -252,7 +267,7 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t na) {
   st = fn.decode(q->data_ptr(), q->stride(0), q->stride(1), norm, ks, vs, int(B), int(Hq), int(H), int(T), int(D),
                  float(scale), out.data_ptr(), out.stride(0), out.stride(1), ws, wsb, stream);
   Py_END_ALLOW_THREADS
-  if (st != IQ_OK) Py_RETURN_NONE;
+  if (st != IQ_OK) return not_ok("iq_decode_attention", st);
   if (given) { Py_INCREF(a[19]); return a[19]; }
   return THPVariable_Wrap(std::move(out));
 }
@@ -301,7 +316,7 @@ PyObject* qk(PyObject*, PyObject* const* a, Py_ssize_t na) {
              int(t0), int(T), int(D), int(s.group), int(s.bits), int(s.mode), float(scale), (float*)out.data_ptr(),
              out.stride(0), out.stride(1), ws, wsb, stream);
   Py_END_ALLOW_THREADS
-  if (st != IQ_OK) Py_RETURN_NONE;
+  if (st != IQ_OK) return not_ok("iq_qk_gemv", st);
   if (given) { Py_INCREF(a[6]); return a[6]; }
   return THPVariable_Wrap(std::move(out));
 }
@@ -347,7 +362,7 @@ PyObject* av(PyObject*, PyObject* const* a, Py_ssize_t na) {
              int(T), int(s.D), int(s.group), int(s.bits), int(s.mode), nullptr, out.data_ptr(), out.stride(0),
              out.stride(1), 0, ws, wsb, stream);
   Py_END_ALLOW_THREADS
-  if (st != IQ_OK) Py_RETURN_NONE;
+  if (st != IQ_OK) return not_ok("iq_av_gemv", st);
   if (given) { Py_INCREF(a[4]); return a[4]; }
   return THPVariable_Wrap(std::move(out));
 }
@@ -434,7 +449,7 @@ PyObject* window_append(PyObject*, PyObject* const* a, Py_ssize_t na) {
   Py_BEGIN_ALLOW_THREADS
   st = fn.append(&r[0].w, &r[1].w, int(B), int(H), int(D), stream);
   Py_END_ALLOW_THREADS
-  if (st != IQ_OK) Py_RETURN_NONE;
+  if (st != IQ_OK) return not_ok("iq_window_append", st);
   for (Role& x : r) {
     if (!set_int(x.win, S_start, x.start + x.flush) || !set_int(x.win, S_n, x.n + x.w.m - x.flush)) return nullptr;
     if (x.flush) {  // the flushed rows now hold their dequantized values (deq_rows)

@@ -241,3 +241,23 @@ def test_tensors_are_held_while_other_threads_run(entry):
 
     entered_as(entry, during, calls[entry])
     assert freed == [0]
+
+
+@pytest.mark.parametrize("entry", ["decode", "qk", "av", "append"])
+def test_a_failed_launch_is_raised_once(entry):
+    """A launch that reports an error is not tried again (it may have run, and an append is no call to run
+    twice); an argument that the entry point refuses is the general path's to refuse or to serve."""
+    ks, vs, kwin, vwin, calls = four_calls()
+    state = [t.clone() for t in (ks.codes, ks.meta, vs.codes, vs.meta, kwin.tensor, vwin.tensor)]
+    with pytest.raises(_lib.IQError) as e:
+        calls[entry]() if entry != "append" else None  # the stream's workspace
+        entered_as(entry, lambda *_: -9, calls[entry])
+    assert e.value.status == -9 and ENTRY[entry] in str(e.value)
+    assert (ks.length, vs.length, kwin.start, kwin.n, vwin.start, vwin.n) == (256, 256, 0, 40, 0, 40)
+    for a, b in zip(state, (ks.codes, ks.meta, vs.codes, vs.meta, kwin.tensor, vwin.tensor)):
+        assert torch.equal(a, b)
+    served = entered_as(entry, lambda *_: -5, calls[entry])
+    if entry == "append":
+        assert (ks.length, vs.length, kwin.start, kwin.n) == (288, 288, 32, 9)
+    else:
+        assert torch.equal(served, calls[entry]())
