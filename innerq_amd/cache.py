@@ -25,6 +25,7 @@ import copy
 from typing import Any, Optional, Sequence
 
 import torch
+from torch.autograd import forward_ad
 from transformers.cache_utils import Cache, CacheLayerMixin
 
 from . import ops
@@ -32,6 +33,11 @@ from .quant import QMode
 
 # attn_implementation name of the fused decode path (innerq_amd.attention)
 FUSED_ATTENTION = "innerq_fused"
+
+
+def _differentiated(x: torch.Tensor) -> bool:
+    """Whether autograd, backward or forward mode, follows what is computed from x."""
+    return (x.requires_grad and torch.is_grad_enabled()) or forward_ad.unpack_dual(x).tangent is not None
 
 
 class _Quantized:
@@ -388,8 +394,11 @@ class InnerqDynamicLayer(CacheLayerMixin):
         fp32 dequantized values, as the reference's cat + .to(dtype)."""
         ns, nq, nr = sink.shape[-2], (q.length if q is not None else 0), recent.shape[-2]
         B, H, _, D = recent.shape
+        # one launch, which reads sink and recent by their addresses: not where autograd follows
+        # them (their gradients go through the copies below)
         if (nq and dtype == q.store.dtype == sink.dtype == recent.dtype and D % 8 == 0
-                and sink.stride(-1) == 1 and recent.stride(-1) == 1):
+                and sink.stride(-1) == 1 and recent.stride(-1) == 1
+                and not _differentiated(sink) and not _differentiated(recent)):
             return ops.read_dense(sink, q.store, recent, norm)
         out = torch.empty(B, H, ns + nq + nr, D, dtype=dtype, device=self.device)
         if ns:

@@ -5,8 +5,11 @@ bit for bit: fp32(c * s + z), times the factor in fp32, one rounding to the outp
 import numpy as np
 import pytest
 import torch
+from torch.autograd import forward_ad
 
 from innerq_amd import ops
+from innerq_amd.cache import InnerqDynamicLayer
+from innerq_amd.presets import preset_config
 from oracle import quant_ref as Q
 
 pytestmark = pytest.mark.gpu
@@ -92,3 +95,32 @@ def test_large_reads_equal_small_ones(axis):
         whole = st.dequant(dtype=dtype)
         for t0 in range(0, T, 6656):
             assert torch.equal(whole[:, :, t0:t0 + 6656], st.dequant(t0, 6656, dtype=dtype))
+
+
+@pytest.mark.parametrize("preset", ["innerq_base", "innerq_hybrid"])
+@pytest.mark.parametrize("act", ["f16", "bf16"])
+def test_gradients_pass_through_dense_reads(preset, act):
+    """A dense read of a layer whose prompt carries gradients: those of the rows that are the prompt's own
+    (sinks and windows) are 1, backward and forward, and the quantized tokens' are 0; the values are the
+    ones without gradients."""
+    layer = InnerqDynamicLayer(preset_config(preset), 0)
+    T = 300
+    k, v = (torch.randn(2, 2, T, 128, device=DEV).to(TD[act]).requires_grad_() for _ in range(2))
+    layer.update(k, v)
+    read = layer.get_deq_tensors()
+    (read[0].float().sum() + read[1].float().sum()).backward()
+    with torch.no_grad():
+        plain = layer.get_deq_tensors()
+    for x, r, p, sink, q in zip((k, v), read, plain, (layer.keys_sink, layer.values_sink), (layer._kq, layer._vq)):
+        assert torch.equal(r, p) and not p.requires_grad
+        want = torch.ones_like(x)
+        ns = sink.shape[2]
+        want[:, :, ns:ns + q.length] = 0.0
+        assert torch.equal(x.grad, want)
+    with forward_ad.dual_level():
+        layer = InnerqDynamicLayer(preset_config(preset), 0)
+        layer.update(*(forward_ad.make_dual(x.detach(), torch.ones_like(x)) for x in (k, v)))
+        for r, sink, q in zip(layer.get_deq_tensors(), (layer.keys_sink, layer.values_sink), (layer._kq, layer._vq)):
+            t = forward_ad.unpack_dual(r).tangent
+            ns = sink.shape[2]
+            assert bool((t[:, :, :ns] == 1).all()) and bool((t[:, :, ns + q.length:] == 1).all())
