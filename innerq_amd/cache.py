@@ -395,9 +395,11 @@ class InnerqDynamicLayer(CacheLayerMixin):
         ns, nq, nr = sink.shape[-2], (q.length if q is not None else 0), recent.shape[-2]
         B, H, _, D = recent.shape
         # one launch, which reads sink and recent by their addresses: not where autograd follows
-        # them (their gradients go through the copies below)
+        # them (their gradients go through the copies below), nor past its 32-bit counts
         if (nq and dtype == q.store.dtype == sink.dtype == recent.dtype and D % 8 == 0
                 and sink.stride(-1) == 1 and recent.stride(-1) == 1
+                and sink.device == recent.device == q.store.codes.device
+                and ns + nq + nr < 2 ** 31 and B * H * (ns + nr) * (D // 8) < 2 ** 31
                 and not _differentiated(sink) and not _differentiated(recent)):
             return ops.read_dense(sink, q.store, recent, norm)
         out = torch.empty(B, H, ns + nq + nr, D, dtype=dtype, device=self.device)

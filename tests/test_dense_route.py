@@ -2,6 +2,7 @@
 the rule alone, on tensors without memory, with the launch and the dequantization recorded."""
 from types import SimpleNamespace
 
+import pytest
 import torch
 from torch.autograd import forward_ad
 
@@ -42,3 +43,15 @@ def test_reads_that_autograd_follows_take_the_copies(monkeypatch):
     with forward_ad.dual_level():
         x = forward_ad.make_dual(rows(32), rows(32))
         assert route(monkeypatch, x, rows(96))[0] == ["copies"]
+
+
+@pytest.mark.parametrize("ns,nr,nq,taken", [(0, 2 ** 27 - 1, 64, "launch"), (0, 2 ** 27, 64, "copies"),
+                                            (2 ** 26, 2 ** 26, 64, "copies")])
+def test_reads_past_the_launchs_counts_take_the_copies(monkeypatch, ns, nr, nq, taken):
+    assert route(monkeypatch, rows(ns), rows(nr), nq)[0] == [taken]
+
+
+def test_other_types_and_devices_take_the_copies(monkeypatch):
+    assert route(monkeypatch, rows(32), rows(96), dtype=torch.float32)[0] == ["copies"]
+    assert route(monkeypatch, rows(32, dtype=torch.bfloat16), rows(96))[0] == ["copies"]
+    assert route(monkeypatch, rows(32, device="cpu"), rows(96))[0] == ["copies"]
