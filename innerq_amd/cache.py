@@ -74,6 +74,9 @@ class _Quantized:
         return ops.unpack_store(self.store)
 
 
+_PREFILL_STEPS = ("initialize_keys_recent", "initialize_values_recent", "initialize_keys_q", "initialize_values_q")
+
+
 class InnerqDynamicLayer(CacheLayerMixin):
     """cache.py:60-419 with packed quantized storage."""
     is_sliding = False
@@ -205,6 +208,10 @@ class InnerqDynamicLayer(CacheLayerMixin):
         return value_states
 
     def initialize_keys_recent(self, key_states: torch.Tensor) -> torch.Tensor:
+        return self._split_keys_recent(key_states).contiguous()
+
+    def _split_keys_recent(self, key_states: torch.Tensor) -> torch.Tensor:
+        """initialize_keys_recent() with the tokens to quantize as a view of key_states."""
         if self.key_quantize:
             viable_recent_size_key = min(self.key_w_recent, key_states.shape[-2])
             if self.key_quantize_over_token:
@@ -217,6 +224,9 @@ class InnerqDynamicLayer(CacheLayerMixin):
         return key_states[:, :, :nq, :]
 
     def initialize_values_recent(self, value_states: torch.Tensor) -> torch.Tensor:
+        return self._split_values_recent(value_states).contiguous()
+
+    def _split_values_recent(self, value_states: torch.Tensor) -> torch.Tensor:
         if self.value_quantize:
             viable_recent_size_value = min(self.value_w_recent, value_states.shape[-2])
             if self.value_quantize_over_token:
@@ -265,8 +275,11 @@ class InnerqDynamicLayer(CacheLayerMixin):
         self.dtype, self.device = key_states.dtype, key_states.device
         key_states = self.initialize_keys_sink(key_states)
         value_states = self.initialize_values_sink(value_states)
-        key_states = self.initialize_keys_recent(key_states)
-        value_states = self.initialize_values_recent(value_states)
+        # this class's own steps quantize straight from the prompt; a subclass's see the contiguous
+        # copy that the reference's helpers return (cache.py:157-186), theirs to change
+        own = all(getattr(getattr(self, n), "__func__", None) is getattr(InnerqDynamicLayer, n) for n in _PREFILL_STEPS)
+        key_states = (self._split_keys_recent if own else self.initialize_keys_recent)(key_states)
+        value_states = (self._split_values_recent if own else self.initialize_values_recent)(value_states)
         self.initialize_keys_q(key_states)
         self.initialize_values_q(value_states)
         self._keep_dequantized_rows()
