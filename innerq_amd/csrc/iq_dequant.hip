@@ -242,6 +242,32 @@ struct VDeq {
   int64_t items;  // B * H * nch * dq
 };
 
+// nd <= 4 columns of one token: v to element `at`
+template <bool BF, bool NT>
+__device__ __forceinline__ void put_cols(const DeqOut& o, int64_t at, int nd, bool num, const float (&v)[4]) {
+  if (o.out16) {
+    uint32_t p0, p1;
+    if (num) { p0 = out_pair_num<BF>(v[0], v[1]); p1 = out_pair_num<BF>(v[2], v[3]); }
+    else { p0 = out_pair<BF>(v[0], v[1]); p1 = out_pair<BF>(v[2], v[3]); }
+    if (o.vec16) {
+      put<NT>(o.out16 + at, u2_t{p0, p1});
+    } else {
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if (c < nd) o.out16[at + c] = uint16_t((c < 2 ? p0 : p1) >> (16 * (c & 1)));
+    }
+  }
+  if (o.out32) {
+    if (o.vec32) {
+      put<NT>(o.out32 + at, f4_t{v[0], v[1], v[2], v[3]});
+    } else {
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if (c < nd) o.out32[at + c] = v[c];
+    }
+  }
+}
+
 template <int BITS, int G, bool BF, bool NT>
 __global__ __launch_bounds__(256) void dequant_v_kernel(VDeq a, DeqOut o, CopyRows cr) {
   constexpr int W = G * BITS / 32, CPG = G / 32;  // chunks per group
@@ -296,28 +322,66 @@ __global__ __launch_bounds__(256) void dequant_v_kernel(VDeq a, DeqOut o, CopyRo
       const h2_t c01 = pair_at(y01, BITS * i, M, b01), c23 = pair_at(y23, BITS * i, M, b23);
       const float v[4] = {__builtin_fmaf(float(c01.x), s[0], z[0]), __builtin_fmaf(float(c01.y), s[1], z[1]),
                           __builtin_fmaf(float(c23.x), s[2], z[2]), __builtin_fmaf(float(c23.y), s[3], z[3])};
-      const int64_t at_t = at + int64_t(t) * o.sot;
-      if (o.out16) {
-        uint32_t p0, p1;
-        if (num) { p0 = out_pair_num<BF>(v[0], v[1]); p1 = out_pair_num<BF>(v[2], v[3]); }
-        else { p0 = out_pair<BF>(v[0], v[1]); p1 = out_pair<BF>(v[2], v[3]); }
-        if (o.vec16) {
-          put<NT>(o.out16 + at_t, u2_t{p0, p1});
-        } else {
+      put_cols<BF, NT>(o, at + int64_t(t) * o.sot, nd, num, v);
+    }
+  }
+}
+
+// The same for launches of at most V_FEW of those threads: four threads per
+// chunk and four columns, 8 tokens each.  Such a launch does not fill the
+// device and is bound by a thread's chain (its words, then 32 rows of stores),
+// which this cuts to 8 rows with 32-bit indices; past the line the words read
+// four times over cost more.  2-bit hybrid / 3-bit sym / 4-bit asym values, G =
+// 32, D = 128, us a launch with a thread per group and column (the first form),
+// with 32 tokens per thread, with 8: 1024 threads of 32 tokens 3.9 / 3.9 / 4.1,
+// 4.9 / 4.7 / 5.1, 3.2 / 3.0 / 3.2; 16384 4.6 / 4.6 / 4.8, 6.0 / 5.6 / 6.2, 3.8 /
+// 3.7 / 3.7; 49152 6.4 / 6.4 / 6.6, 7.0 / 6.4 / 7.0, 6.3 / 6.1 / 6.3; 53248 7.1 /
+// 7.1 / 7.2, 7.0 / 6.5 / 7.4, 7.1 / 6.9 / 7.1; 131072 11.0 / 11.0 / 11.3, 9.8 /
+// 9.5 / 10.7, 12.0 / 11.2 / 12.4.
+constexpr int64_t V_FEW = 49152;
+template <int BITS, int G, bool BF>
+__global__ __launch_bounds__(256) void dequant_v_few_kernel(VDeq a, DeqOut o, CopyRows cr) {
+  constexpr int W = G * BITS / 32, CPG = G / 32;
+  if (int64_t(blockIdx.x) >= cr.blocks0) {
+    copy_rows(cr, o);
+    return;
+  }
+  const uint32_t e = blockIdx.x * 256u + threadIdx.x;  // 4 a.items <= 4 V_FEW of them
+  if (e >= 4u * uint32_t(a.items)) return;
+  const uint32_t rq = e / uint32_t(a.dq), r = rq >> 2, b = r / uint32_t(a.nch);
+  const int d = int(e - rq * uint32_t(a.dq)) * 4, q = int(rq & 3u), k = int(r - b * uint32_t(a.nch));
+  const int64_t bh = b;
+  const int nd = min(4, a.D - d);
+  // the 8 fields: 8 BITS bits at 8 BITS q of the column's BITS words
+  constexpr int FB = 8 * BITS;
+  const int wi = FB * q >> 5, sh = FB * q & 31;
+  uint32_t y[4];
+  float s[4], z[4];
+  int off[4];
+  bool num = true;
 #pragma unroll
-          for (int c = 0; c < 4; ++c)
-            if (c < nd) o.out16[at_t + c] = uint16_t((c < 2 ? p0 : p1) >> (16 * (c & 1)));
-        }
-      }
-      if (o.out32) {
-        if (o.vec32) {
-          put<NT>(o.out32 + at_t, f4_t{v[0], v[1], v[2], v[3]});
-        } else {
+  for (int c = 0; c < 4; ++c) {
+    const int64_t unit = (bh * a.cap_groups + a.g0 + k / CPG) * a.D + d + (c < nd ? c : 0);
+    const uint32_t* w = a.codes + unit * W + (k % CPG) * BITS;
+    y[c] = w[wi] >> sh;
+    if constexpr (BITS == 3)  // q = 1, 2: the rest is in the next word
+      y[c] |= w[min(wi + 1, BITS - 1)] << ((32 - sh) & 31) & (sh > 8 ? ~0u : 0u);
+    unit_params<BF>(a.meta, unit, a.mode, BITS, s[c], z[c], off[c]);
+    num = num && tame(s[c], z[c]);
+  }
+  const h2_t b01 = bias_of(off[0], off[1]), b23 = bias_of(off[2], off[3]);
+  const int64_t at = (bh / a.H) * o.sob + (bh % a.H) * o.soh + (int64_t(k) * 32 + 8 * q) * o.sot + d;
+  constexpr uint32_t M = ((1u << BITS) - 1u) * 0x10001u, M4 = (1u << (4 * BITS)) - 1u;
 #pragma unroll
-          for (int c = 0; c < 4; ++c)
-            if (c < nd) o.out32[at_t + c] = v[c];
-        }
-      }
+  for (int x = 0; x < 2; ++x) {  // four tokens of two columns in the halves of a dword
+    const uint32_t y01 = (y[0] >> (4 * BITS * x) & M4) | (y[1] >> (4 * BITS * x) & M4) << 16;
+    const uint32_t y23 = (y[2] >> (4 * BITS * x) & M4) | (y[3] >> (4 * BITS * x) & M4) << 16;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const h2_t c01 = pair_at(y01, BITS * i, M, b01), c23 = pair_at(y23, BITS * i, M, b23);
+      const float v[4] = {__builtin_fmaf(float(c01.x), s[0], z[0]), __builtin_fmaf(float(c01.y), s[1], z[1]),
+                          __builtin_fmaf(float(c23.x), s[2], z[2]), __builtin_fmaf(float(c23.y), s[3], z[3])};
+      put_cols<BF, false>(o, at + int64_t(4 * x + i) * o.sot, nd, num, v);
     }
   }
 }
@@ -347,11 +411,13 @@ int launch_v(const uint32_t* codes, const uint16_t* meta, int64_t t_cap, int B, 
              int bits, int mode, bool bf, const DeqOut& o, CopyRows cr, int64_t copy_blocks, hipStream_t st) {
   const int nch = T / 32, dq = (D + 3) / 4;
   const VDeq a{codes, meta, t_cap / group, H, t0 / group, D, mode, nch, dq, int64_t(B) * H * nch * dq};
-  cr.blocks0 = ceil_div(a.items, 256);
+  const bool few = a.items <= V_FEW;
+  cr.blocks0 = ceil_div(few ? 4 * a.items : a.items, 256);
   const bool nt = streams(B, H, T, D, o);
   const dim3 grid(unsigned(cr.blocks0 + copy_blocks));
   return dispatch_store_bits_group(bits, group, [&]<int BITS, int G>() {
-    auto* kern = bf   ? (nt ? dequant_v_kernel<BITS, G, true, true> : dequant_v_kernel<BITS, G, true, false>)
+    auto* kern = few ? (bf ? dequant_v_few_kernel<BITS, G, true> : dequant_v_few_kernel<BITS, G, false>)
+                 : bf ? (nt ? dequant_v_kernel<BITS, G, true, true> : dequant_v_kernel<BITS, G, true, false>)
                  : nt ? dequant_v_kernel<BITS, G, false, true>
                       : dequant_v_kernel<BITS, G, false, false>;
     kern<<<grid, 256, 0, st>>>(a, o, cr);

@@ -85,6 +85,25 @@ def test_read_dense(act, axis, D, ns, n, nr, layout):
     assert torch.equal(got, torch.cat([sink, st.dequant(norm=norm), recent], dim=2))
 
 
+@pytest.mark.parametrize("act", ["f16", "bf16"])
+@pytest.mark.parametrize("bits,mode,G", [(1, "asymmetric", 32), (2, "hybrid", 64), (3, "symmetric", 32),
+                                         (3, "hybrid", 128), (4, "asymmetric", 128)])
+@pytest.mark.parametrize("D,n,layout", [(128, 24576, "plain"), (33, 87296, "odd rows"), (96, 32768, "heads last")])
+def test_value_reads_past_the_few_thread_line(act, bits, mode, G, D, n, layout):
+    """A read of values by more than 49,152 threads of 32 tokens (the line between the two kernels: 2 heads x
+    n / 32 x ceil(D / 4)), and one at the line, equal the same tokens read in small pieces (which the
+    tests above check against the oracle)."""
+    st = ops.PackedStore("token", 1, 2, D, G, bits, mode, DEV, dtype=TD[act])
+    st.append(torch.randn(1, 2, n + 256, D, device=DEV).to(TD[act]))
+    for dtype in (TD[act], torch.float32):
+        for T in (n, n + 256):
+            out = view(1, 2, T, D, dtype, layout)
+            st.dequant(0, T, out=out)
+            for t0 in range(0, T, 8192):
+                m = min(8192, T - t0)
+                assert torch.equal(out[:, :, t0:t0 + m], st.dequant(t0, m, dtype=dtype))
+
+
 @pytest.mark.parametrize("axis", ["channel", "token"])
 def test_large_reads_equal_small_ones(axis):
     """A read past the size where the stores stream equals the same tokens read in pieces below it."""
