@@ -104,16 +104,25 @@ def test_value_reads_past_the_few_thread_line(act, bits, mode, G, D, n, layout):
                 assert torch.equal(out[:, :, t0:t0 + m], st.dequant(t0, m, dtype=dtype))
 
 
+@pytest.mark.parametrize("act", ["f16", "bf16"])
 @pytest.mark.parametrize("axis", ["channel", "token"])
-def test_large_reads_equal_small_ones(axis):
-    """A read past the size where the stores stream equals the same tokens read in pieces below it."""
-    B, H, T, D = 2, 8, 26624, 128  # 109 MB in fp16
-    st = ops.PackedStore(axis, B, H, D, 32, 3, "symmetric", DEV)
-    st.append(torch.randn(B, H, T, D, device=DEV).half())
-    for dtype in (torch.float16, torch.float32):
-        whole = st.dequant(dtype=dtype)
-        for t0 in range(0, T, 6656):
-            assert torch.equal(whole[:, :, t0:t0 + 6656], st.dequant(t0, 6656, dtype=dtype))
+def test_large_reads_equal_small_ones(axis, act):
+    """A read past 104 MB of output, where the stores stream (16-bit and fp32 outputs), equals the same
+    tokens read in pieces below it."""
+    B, H, T, D, step = 2, 8, 28672, 128, 7168
+    assert 2 * B * H * T * D > 104 << 20 > 4 * B * H * step * D
+    st = ops.PackedStore(axis, B, H, D, 32, 3, "symmetric", DEV, dtype=TD[act])
+    norm = torch.rand(B, H, 1, D, device=DEV).to(TD[act]) + 0.5 if axis == "channel" else None
+    st.append(torch.randn(B, H, T, D, device=DEV).to(TD[act]), norm=norm)
+    for dtype in (TD[act], torch.float32):
+        whole = st.dequant(dtype=dtype, norm=norm)
+        for t0 in range(0, T, step):
+            assert torch.equal(whole[:, :, t0:t0 + step], st.dequant(t0, step, dtype=dtype, norm=norm))
+    sink, recent = (torch.randn(B, H, n, D, device=DEV).to(TD[act]) for n in (32, 95))
+    got = ops.read_dense(sink, st, recent, norm)
+    assert torch.equal(got[:, :, :32], sink) and torch.equal(got[:, :, 32 + T:], recent)
+    for t0 in range(0, T, step):
+        assert torch.equal(got[:, :, 32 + t0:32 + t0 + step], st.dequant(t0, step, norm=norm))
 
 
 @pytest.mark.parametrize("preset", ["innerq_base", "innerq_hybrid"])
