@@ -130,24 +130,70 @@ def test_values(act, mode, widths, groups, D, G, off, layout):
         assert same_meta(gm, meta, act)
 
 
-@pytest.mark.parametrize("n,t0", [(1, 0), (65, 0), (30, 50), (64, 0)])
-@pytest.mark.parametrize("mode", ["asymmetric", "symmetric"])
-def test_appended_store_clears_its_last_block(mode, n, t0):
-    """A store that an append made or grew is not cleared as a whole: the append clears the rows of
-    its last 64-token block past the tokens, here over memory that held other values."""
+@pytest.fixture
+def stale(monkeypatch):
+    """torch.empty as memory that held other values gives it: every byte of the stores' integers set."""
+    empty = torch.empty
+
+    def poisoned(*a, **k):
+        t = empty(*a, **k)
+        return t.fill_(-1) if t.dtype in (torch.int32, torch.int16) else t
+
+    monkeypatch.setattr(torch, "empty", poisoned)
+
+
+def token_rows(st):
+    """(codes, meta) of a K store as [B H, token, ...]."""
+    bh, nb, ng = st.B * st.H, st.t_cap // 64, st.D // st.group
+    return [t.view(bh, nb, ng, 64, -1).transpose(2, 3).reshape(bh, nb * 64, -1) for t in (st.codes, st.meta)]
+
+
+@pytest.mark.parametrize("n,t0", [(1, 0), (65, 0), (30, 50), (64, 0), (192, 64), (57, 200), (7, 250), (120, 250),
+                                  (300, 255), (64, 256), (400, 200)])
+@pytest.mark.parametrize("mode", ["asymmetric", "symmetric", "hybrid"])
+def test_appended_store_clears_its_last_block(stale, mode, n, t0):
+    """A store that an append made or grew (past 256 tokens here) is not cleared as a whole: the append
+    clears the rows of its last 64-token block past the tokens and the blocks after it, over memory that
+    held other values; the tokens of before stay."""
     B, H, D = 2, 3, 128
-    poison = [torch.full((1 << 20,), -1, dtype=torch.int32, device=DEV) for _ in range(8)]
-    del poison
     st = ops.PackedStore("channel", B, H, D, 32, 3, mode, DEV)
     x = torch.randn(B, H, t0 + n, D, device=DEV).half()
+    before = None
     if t0:
         st.append(x[:, :, :t0])
+        before = [t[:, :t0].clone() for t in token_rows(st)]
     st.append(x[:, :, t0:])
-    T, nb = t0 + n, st.t_cap // 64
-    codes = st.codes.view(B * H, nb, D // 32, 64, -1).transpose(2, 3).reshape(B * H, nb * 64, -1)
-    meta = st.meta.view(B * H, nb, D // 32, 64, -1).transpose(2, 3).reshape(B * H, nb * 64, -1)
-    assert int((codes[:, T:] != 0).sum()) == 0 and int((meta[:, T:] != 0).sum()) == 0
-    assert bool((meta[:, :T] != 0).any())
+    T, rows = t0 + n, token_rows(st)
+    assert all(int((t[:, T:] != 0).sum()) == 0 for t in rows)
+    if t0:
+        assert all(torch.equal(t[:, :t0], b) for t, b in zip(rows, before))
+    whole = ops.PackedStore("channel", B, H, D, 32, 3, mode, DEV)
+    whole.reserve(T)
+    whole.append(x)
+    assert all(torch.equal(t[:, :T], w[:, :T]) for t, w in zip(rows, token_rows(whole)))
+
+
+@pytest.mark.parametrize("axis,t0,n", [("channel", 0, 70), ("channel", 250, 70), ("token", 0, 64), ("token", 128, 32)])
+def test_a_failed_append_leaves_cleared_units(stale, monkeypatch, axis, t0, n):
+    """An append that grew the store and then raised leaves the new units as a cleared store has them."""
+    st = ops.PackedStore(axis, 2, 3, 128, 32, 2, "asymmetric", DEV)
+    x = torch.randn(2, 3, t0 + n, 128, device=DEV).half()
+    if t0:
+        st.append(x[:, :, :t0])
+    cap = st.t_cap
+    cut = -(-t0 // st.unit)
+    old = [t.view(6, cap // st.unit, -1)[:, :cut].clone() for t in (st.codes, st.meta)] if t0 else []
+
+    def fail(*a):
+        raise RuntimeError("launch")
+
+    monkeypatch.setattr(st, "_quantize", fail)
+    with pytest.raises(RuntimeError, match="launch"):
+        st.append(x[:, :, t0:])
+    assert st.t_cap > cap and st.length == t0
+    now = [t.view(6, st.t_cap // st.unit, -1) for t in (st.codes, st.meta)]
+    assert all(int((t[:, cut:] != 0).sum()) == 0 for t in now)
+    assert all(torch.equal(t[:, :cut], b) for t, b in zip(now, old))
 
 
 @pytest.mark.parametrize("act", ["f16", "bf16"])
