@@ -1,11 +1,9 @@
-"""The two K quantizers agree bit for bit: one lane per value (quant_k_lane_kernel
-and the window append's group items, used for calls of at most 65,536 groups:
-a decode step's tokens) and one thread per group (quant_k_kernel, larger calls:
-a prompt).  Same tokens quantized in one large call and in small calls, on
-inputs with the groups where the two could part: signed zeros at the minimum,
-constant groups (scale 0, NaN codes), NaN and infinity, exact rounding ties,
-fp16 subnormals.  The small calls are also checked against the oracle in
-test_gpu_kernels (random data)."""
+"""The K quantizers agree bit for bit: the prompt's (quant_k_kernel: a thread per eight values, packed
+arithmetic, a reciprocal for the division) in one large call and in many small ones, and the window
+append's (a lane per value, the reference's own arithmetic), on inputs with the groups where they could
+part: signed zeros at the minimum, constant groups (scale 0, NaN codes), NaN and infinity, exact rounding
+ties, fp16 subnormals.  Small calls are also checked against the oracle in test_gpu_kernels (random
+data) and test_gpu_quantize_edges."""
 import numpy as np
 import pytest
 import torch
@@ -14,8 +12,8 @@ from innerq_amd import ops
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
-N_TOK = 4160  # 8 heads x 4160 tokens: > 65,536 groups of 32 and of 64 -> one thread per group
-CHUNK = 64    # 8 x 64 x (128 / G) groups -> one lane per value
+N_TOK = 4160  # the large call: 2080 workgroups of quant_k_kernel
+CHUNK = 64    # the small ones: 32 workgroups, or a window append's flush
 
 
 def adversarial(H, T, D, seed):
@@ -55,10 +53,15 @@ def test_lane_and_thread_quantizers_agree(mode, bits, G, norm):
     small = ops.PackedStore("channel", 1, H, D, G, bits, mode, DEV)
     for t in range(0, N_TOK, CHUNK):
         small.append(x[:, :, t:t + CHUNK], norm=nf)
+    lanes = ops.PackedStore("channel", 1, H, D, G, bits, mode, DEV)
+    win = ops.RecentWindow(x[:, :, :0])
+    for t in range(0, N_TOK, CHUNK):
+        ops.window_append(win, x[:, :, t:t + CHUNK], CHUNK, lanes, nf, None, None, 0, None)
     bc, bm = store_bytes(big)
-    sc, sm = store_bytes(small)
-    np.testing.assert_array_equal(sc, bc)
-    np.testing.assert_array_equal(sm, bm)
+    for other in (small, lanes):
+        oc, om = store_bytes(other)
+        np.testing.assert_array_equal(oc, bc)
+        np.testing.assert_array_equal(om, bm)
 
 
 @pytest.mark.parametrize("mode", ["asymmetric", "symmetric"])
