@@ -609,14 +609,22 @@ __global__ __launch_bounds__(MERGE ? 256 * NS : 256) void dense_attn_kernel(Dens
   if constexpr (MERGE) {
     // ---- merge: the sections' states and the fused runs' partials ----
     __shared__ float mh[NH][NREP], lh[NH][NREP];
-    __shared__ float2 rml[MERGE_RUNS_MAX][NREP];  // the runs' statistics
-    static_assert(MERGE_RUNS_MAX * 4 <= NTH && MERGE_PRE * 8 <= NTH, "one thread per run and head");
-    float po2[EPT][MERGE_PRE];
-    if (nr > MERGE_PRE) {
+    // the runs' statistics (past the last run those of an empty one).  An
+    // instance of at most MERGE_PRE runs holds no code for more and reads all
+    // of them at once: as loops over up to 16, B = 10, 8 KV heads, 967 tokens,
+    // a 151-token window, bf16, kernel / call in us: 2 query heads per KV head
+    // 14.1 / 21.3, 4 heads 15.0 / 22.9; so 13.8 / 21.1 and 14.4 / 22.5.
+    constexpr int RM = merge_runs_max(BF, NREP);
+    __shared__ float2 rml[RM][NREP];
+    static_assert(RM * NREP <= NTH, "one thread per run and head");
+    float po2[RM > MERGE_PRE ? EPT : 1][MERGE_PRE];
+    if constexpr (RM > MERGE_PRE) {
+      if (nr > MERGE_PRE) {
 #pragma unroll
-      for (int e = 0; e < EPT; ++e) load_runs(e, MERGE_PRE, po2[e]);
+        for (int e = 0; e < EPT; ++e) load_runs(e, MERGE_PRE, po2[e]);
+      }
     }
-    if (int(threadIdx.x) < nr * NREP) rml[int(threadIdx.x) / NREP][int(threadIdx.x) % NREP] = rst;
+    if (int(threadIdx.x) < RM * NREP) rml[int(threadIdx.x) / NREP][int(threadIdx.x) % NREP] = rst;
     __shared__ float oh[BF ? NH : 1][BF ? NREP : 1][BF ? D : 1];  // BF: the sections' outputs
 #pragma unroll
     for (int hh = 0; hh < HPW; ++hh) {
@@ -646,7 +654,12 @@ __global__ __launch_bounds__(MERGE ? 256 * NS : 256) void dense_attn_kernel(Dens
       float M = -INFINITY;
 #pragma unroll
       for (int hf = 0; hf < NH; ++hf) M = fmaxf(M, mh[hf][h]);
-      for (int sp = 0; sp < nr; ++sp) M = fmaxf(M, rml[sp][h].x);
+      if constexpr (RM == MERGE_PRE) {
+#pragma unroll
+        for (int sp = 0; sp < RM; ++sp) M = fmaxf(M, rml[sp][h].x);
+      } else {
+        for (int sp = 0; sp < nr; ++sp) M = fmaxf(M, rml[sp][h].x);
+      }
       float L = 0.f, acc = 0.f;
       auto add_run = [&](float2 s, float pv) {  // the runs in slot order, then the sections
         const float w = s.x == -INFINITY ? 0.f : __expf(s.x - M);
@@ -656,11 +669,13 @@ __global__ __launch_bounds__(MERGE ? 256 * NS : 256) void dense_attn_kernel(Dens
 #pragma unroll
       for (int sp = 0; sp < MERGE_PRE; ++sp)
         if (sp < nr) add_run(rml[sp][h], po[e][sp]);
-      for (int s0 = MERGE_PRE; s0 < nr; s0 += MERGE_PRE) {
-        if (s0 > MERGE_PRE) load_runs(e, s0, po2[e]);
+      if constexpr (RM > MERGE_PRE) {
+        for (int s0 = MERGE_PRE; s0 < nr; s0 += MERGE_PRE) {
+          if (s0 > MERGE_PRE) load_runs(e, s0, po2[e]);
 #pragma unroll
-        for (int sp = 0; sp < MERGE_PRE; ++sp)
-          if (s0 + sp < nr) add_run(rml[s0 + sp][h], po2[e][sp]);
+          for (int sp = 0; sp < MERGE_PRE; ++sp)
+            if (s0 + sp < nr) add_run(rml[s0 + sp][h], po2[e][sp]);
+        }
       }
 #pragma unroll
       for (int hf = 0; hf < NH; ++hf) {
