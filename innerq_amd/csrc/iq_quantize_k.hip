@@ -316,16 +316,25 @@ __device__ __forceinline__ void quant_k8(uint32_t (&w)[4], int j, const QuantOut
 }
 
 // One lane per 8 consecutive values of a row: a wave loads whole rows (16 B
-// per lane), four such loads in flight per lane.  A lane's columns are the
-// same in all four where a row's lanes divide the workgroup, so a
+// per lane), KU such loads in flight per lane.  A lane's columns are the
+// same in all of them where a row's lanes divide the workgroup, so a
 // normalization factor's reciprocals are made once.
 // A thread per group, the form before, read 64 B per lane at a 64 B stride and
-// spent ~25 instructions a value.  PackedStore.append of 8 x 8 heads x 32768
-// tokens, 4-bit asym G = 32 (537 MB read, 168 MB written): 180 -> 161 us a
-// call (kernel 184 -> 134 us, 5.3 TB/s), 136 once it no longer clears the
-// whole new store first.
-constexpr int KU = 4;  // loads in flight per lane
-template <int BITS, int G, int MODE, bool BF>
+// spent ~25 instructions a value.  8 x 8 heads x 32768 tokens, 4-bit asym G =
+// 32 (537 MB read, 168 MB written), both traced on one box: kernel 174 -> 137
+// us (5.2 TB/s).  PackedStore.append of them, untraced: 180 -> 161 us a call,
+// 134 once it no longer clears the whole new store first.
+//
+// Four rows per lane, or one up to K_FEW lanes, where the device is not full
+// and a call is one lane's chain.  8 heads x 128-d tokens, fp16, us a launch in
+// a graph with one / four rows (before this kernel: a lane per value, later a
+// thread per group): 128 tokens 4-bit asym 2.4 / 4.3 (3.4), with a factor 2.9 /
+// 5.3 (3.6), 2-bit hybrid 2.7 / 5.4 (8.2); 4096 tokens (K_FEW) 4.4 / 5.1, 6.1 /
+// 6.2, 5.9 / 6.9; 8192 tokens 6.5 / 7.0, 9.7 / 9.0, 9.2 / 10.1; 32768 tokens
+// 19.4 / 19.4, 31.8 / 25.5, 30.1 / 30.0.  bf16 lies alike.
+constexpr int KROWS = 4;
+constexpr int64_t K_FEW = 1 << 19;
+template <int BITS, int G, int MODE, bool BF, int KU>
 __global__ __launch_bounds__(256) void quant_k_kernel(KArgs a, QuantOut o) {
   constexpr int LPG = G / 8;
   const int64_t bh = int64_t(blockIdx.x) / a.tiles, tile = int64_t(blockIdx.x) % a.tiles;
@@ -372,8 +381,12 @@ __global__ __launch_bounds__(256) void quant_k_kernel(KArgs a, QuantOut o) {
 }
 
 template <int BITS, int G, int MODE, bool BF>
-int launch_k(const KArgs& a, const QuantOut& o, int64_t blocks, hipStream_t st) {
-  quant_k_kernel<BITS, G, MODE, BF><<<dim3(unsigned(blocks)), 256, 0, st>>>(a, o);
+int launch_k(KArgs a, const QuantOut& o, int64_t heads, hipStream_t st) {
+  const int64_t lanes = int64_t(a.n_pad) * a.lpr;
+  const bool few = heads * lanes <= K_FEW;
+  a.tiles = ceil_div(lanes, 256 * (few ? 1 : KROWS));
+  auto* kern = few ? quant_k_kernel<BITS, G, MODE, BF, 1> : quant_k_kernel<BITS, G, MODE, BF, KROWS>;
+  kern<<<dim3(unsigned(heads * a.tiles)), 256, 0, st>>>(a, o);
   return launch_status();
 }
 }  // namespace
@@ -408,11 +421,10 @@ int iq_quantize_k(const void* x, int64_t sx_b, int64_t sx_h, int64_t sx_t, const
   const bool pow2 = (lpr & (lpr - 1)) == 0 && lpr <= 256;
   const int pad = zero_tail && k_codes ? int((TOKEN_BLOCK - (t_off + n) % TOKEN_BLOCK) % TOKEN_BLOCK) : 0;
   KArgs a{(const uint16_t*)x, sx_b, sx_h, sx_t, (const uint16_t*)norm, H, n, D, n + pad, lpr,
-          pow2 ? __builtin_ctz(unsigned(lpr)) : -1, ceil_div(int64_t(n + pad) * lpr, 256 * KU)};
+          pow2 ? __builtin_ctz(unsigned(lpr)) : -1, 0};
   return dispatch_format(bits, group, mode, [&]<int BITS, int G, int MODE>() {
-    const int64_t blocks = int64_t(B) * H * a.tiles;
-    return bf ? launch_k<BITS, G, MODE, true>(a, o, blocks, (hipStream_t)stream)
-              : launch_k<BITS, G, MODE, false>(a, o, blocks, (hipStream_t)stream);
+    return bf ? launch_k<BITS, G, MODE, true>(a, o, int64_t(B) * H, (hipStream_t)stream)
+              : launch_k<BITS, G, MODE, false>(a, o, int64_t(B) * H, (hipStream_t)stream);
   });
 }
 

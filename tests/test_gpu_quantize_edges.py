@@ -130,6 +130,25 @@ def test_values(act, mode, widths, groups, D, G, off, layout):
         assert same_meta(gm, meta, act)
 
 
+@pytest.mark.parametrize("act", ["f16", "bf16"])
+@pytest.mark.parametrize("bits,mode,D,G,norm", [(4, "asymmetric", 128, 32, False), (3, "symmetric", 96, 32, True),
+                                                (2, "hybrid", 64, 64, True), (1, "asymmetric", 384, 128, False)])
+@pytest.mark.parametrize("rows", [0, 37])
+def test_long_key_calls_equal_short_ones(act, bits, mode, D, G, norm, rows):
+    """A call of at most 2^19 lanes of 8 values takes one row per lane, a longer one four: calls at the line
+    and a ragged number of rows past it hold the bytes of calls of 100 tokens."""
+    B, H = 2, 4
+    n = (1 << 19) // (B * H * D // 8) + rows
+    x = torch.cat([planted(B, H, 64, D, bits, act), torch.randn(B, H, n - 64, D).to(TD[act])], dim=2).to(DEV)
+    nf = (torch.rand(B, H, 1, D, device=DEV) + 0.5).to(TD[act]) if norm else None
+    whole, parts = (ops.PackedStore("channel", B, H, D, G, bits, mode, DEV, dtype=TD[act]) for _ in range(2))
+    whole.append(x, norm=nf)
+    for t in range(0, n, 100):
+        parts.append(x[:, :, t:t + 100], norm=nf)
+    for a, b in zip(token_rows(whole), token_rows(parts)):
+        assert torch.equal(a[:, :n], b[:, :n]) and int((a[:, n:] != 0).sum()) == 0
+
+
 @pytest.fixture
 def stale(monkeypatch):
     """torch.empty as memory that held other values gives it: every byte of the stores' integers set."""
