@@ -6,6 +6,7 @@
 #include "iq_common.h"
 #include "iq_device.h"
 #include "iq_qcodes.h"
+#include "iq_quantize_v.h"
 
 using namespace iq;
 
@@ -163,6 +164,32 @@ __device__ __forceinline__ int32_t quant_group_lanes(float v, int i, int bits, i
     }
   }
   return c;
+}
+
+// Values quantized by a lane per value (iq_quantize_v.hip says where).
+template <int G>
+__global__ __launch_bounds__(256) void quant_v_lanes_kernel(detail::VArgs a, QuantOut o, int64_t groups, int bits,
+                                                            int mode, int bf) {
+  const int64_t e = int64_t(blockIdx.x) * 256 + threadIdx.x, gid = e / G;
+  const int i = int(e % G);
+  if (gid >= groups) return;  // whole G-lane segments
+  const int ngn = a.n / G;
+  const int64_t r = gid / a.D;  // bh * ngn + gi
+  const int d = int(gid - r * a.D);
+  const int64_t bh = r / ngn;
+  const int t = int(r - bh * ngn) * G + i;
+  const int64_t unit = (bh * o.cap_units + (o.t_off + t) / G) * a.D + d;
+  const float v = act2f(a.x[(bh / a.H) * a.sxb + (bh % a.H) * a.sxh + t * a.sxt + d], bf != 0);
+  float sg, s, z;
+  const int32_t c = quant_group_lanes<G>(v, i, bits, mode, bf != 0, o.codes != nullptr,
+                                         o.codes ? o.codes + unit * ((G * bits) >> 5) : nullptr, o.meta, unit, sg, s, z);
+  const int64_t el = (bh * a.n + t) * a.D + d, red = r * a.D + d;
+  if (o.codes_i32) o.codes_i32[el] = c;
+  if (o.signs16) o.signs16[el] = f2act(sg, bf != 0);
+  if (i == 0) {
+    if (o.scale16) o.scale16[red] = f2act(s, bf != 0);
+    if (o.zero16) o.zero16[red] = f2act(z, bf != 0);
+  }
 }
 
 // One group by one thread (groups of 128), with the bit width, mode and activation dtype known at run time: v[] holds the
@@ -511,6 +538,14 @@ __global__ __launch_bounds__(256) void window_append_kernel(AppendArgs a) {
 }
 
 }  // namespace
+
+int iq::detail::quantize_v_lanes(const VArgs& a, const QuantOut& o, int64_t heads, int group, int bits, int mode,
+                                 bool bf, hipStream_t st) {
+  const int64_t groups = heads * (a.n / group) * a.D;
+  auto* kern = group == 64 ? quant_v_lanes_kernel<64> : quant_v_lanes_kernel<32>;
+  kern<<<dim3(unsigned(ceil_div(groups * group, 256))), 256, 0, st>>>(a, o, groups, bits, mode, bf ? 1 : 0);
+  return launch_status();
+}
 
 // =============================================================================
 // C ABI

@@ -17,6 +17,9 @@ struct VArgs {
 };
 int quantize_v_f16(const VArgs& a, const QuantOut& o, int group, int bits, int mode, bool dense, hipStream_t st);
 int quantize_v_bf16(const VArgs& a, const QuantOut& o, int group, int bits, int mode, bool dense, hipStream_t st);
+// the same by a lane per value (iq_quant.hip): groups of 32 or 64, asym or sym
+int quantize_v_lanes(const VArgs& a, const QuantOut& o, int64_t heads, int group, int bits, int mode, bool bf,
+                     hipStream_t st);
 
 }  // namespace iq::detail
 
@@ -269,11 +272,14 @@ __device__ __forceinline__ void chunk32(const uint32_t (&v)[32], const GroupQ (&
 // are whole row pieces (256 B), every fp16 op covers both columns, a column's
 // words leave in one store.  Groups of 32 and 64 tokens stay in registers
 // (one or two chunks of 32); a group of 128 is read again chunk by chunk once
-// its extremes are known (and, hybrid, its errors), from L2.  DENSE: quant.py's
-// outputs as well.  A bf16 prompt's prefill (innerq_base, 4 x 8 heads x 8190
+// its extremes are known (and, hybrid, its errors), from L2.  DENSE 1: quant.py's
+// outputs as well, those that are asked for; 2: all of them, the signs of a
+// column pair as one dword, with no branch per store (8 heads x 512 tokens,
+// 3-bit sym fp16: 7.0 -> 5.4 us a launch, a thread per column before 5.5;
+// 32768 tokens 45 us, 47 before).  A bf16 prompt's prefill (innerq_base, 4 x 8 heads x 8190
 // tokens, K and V): 558 -> 166 us with this kernel and quant_k_kernel; one
 // lane or one thread per value or group took 239 (K) and 214 us (V) of it.
-template <int BITS, int G, int MODE, bool BF, bool DENSE>
+template <int BITS, int G, int MODE, bool BF, int DENSE>
 __global__ __launch_bounds__(256) void quant_v_kernel(VArgs a, QuantOut o) {
   constexpr int W = G * BITS / 32, NCH = G / 32;
   constexpr bool HELD = NCH <= 2;
@@ -335,18 +341,24 @@ __global__ __launch_bounds__(256) void quant_v_kernel(VArgs a, QuantOut o) {
 
   bool pick[2] = {MODE == IQ_MODE_SYM, MODE == IQ_MODE_SYM};
   double ea[2] = {0.0, 0.0}, es[2] = {0.0, 0.0};
+  const int next = two ? 1 : 0;  // a single last column is a pair of itself: the same value twice, and no branch per store
   auto dense = [&](int k, int i, int32_t c0, int32_t c1) {
     if constexpr (DENSE) {
       const int64_t at = el + int64_t(32 * k + i) * a.D;
       const uint32_t w = v[HELD ? k : 0][i];
       if constexpr (MODE == IQ_MODE_SYM) { c0 = abs(c0); c1 = abs(c1); }
-      if (o.codes_i32) {  // a constant group's codes: 0 / 0
+      if (DENSE == 2 || o.codes_i32) {  // a constant group's codes: 0 / 0
         o.codes_i32[at] = (MODE == IQ_MODE_SYM ? g[0].ss : g[0].s) == 0.f ? I32_MIN : c0;
-        if (two) o.codes_i32[at + 1] = (MODE == IQ_MODE_SYM ? g[1].ss : g[1].s) == 0.f ? I32_MIN : c1;
+        o.codes_i32[at + next] = (MODE == IQ_MODE_SYM ? g[1].ss : g[1].s) == 0.f ? I32_MIN : c1;
       }
-      if (o.signs16) {
-        o.signs16[at] = f2act(sign_of(lo16(w, BF)), BF);
-        if (two) o.signs16[at + 1] = f2act(sign_of(hi16(w, BF)), BF);
+      if (MODE != IQ_MODE_ASYM && (DENSE == 2 || o.signs16)) {
+        const uint32_t s0 = f2act(sign_of(lo16(w, BF)), BF), s1 = f2act(sign_of(hi16(w, BF)), BF);
+        if constexpr (DENSE == 2) {
+          *reinterpret_cast<uint32_t*>(o.signs16 + at) = s0 | (s1 << 16);
+        } else {
+          o.signs16[at] = uint16_t(s0);
+          o.signs16[at + next] = uint16_t(s1);
+        }
       }
     }
   };
@@ -435,11 +447,14 @@ int launch_quant_v(const VArgs& a, const QuantOut& o, int group, int bits, int m
   return dispatch_format(bits, group, mode, [&]<int BITS, int G, int MODE>() {
     if constexpr (MODE != IQ_MODE_HYBRID) {
       if (dense) {
-        quant_v_kernel<BITS, G, MODE, BF, true><<<grid, 256, 0, st>>>(a, o);
+        const bool pairs = o.signs16 && a.D % 2 == 0 && aligned(o.signs16, 4);
+        auto* kern = o.codes_i32 && (MODE == IQ_MODE_ASYM || pairs) ? quant_v_kernel<BITS, G, MODE, BF, 2>
+                                                                    : quant_v_kernel<BITS, G, MODE, BF, 1>;
+        kern<<<grid, 256, 0, st>>>(a, o);
         return launch_status();
       }
     }
-    quant_v_kernel<BITS, G, MODE, BF, false><<<grid, 256, 0, st>>>(a, o);
+    quant_v_kernel<BITS, G, MODE, BF, 0><<<grid, 256, 0, st>>>(a, o);
     return launch_status();
   });
 }

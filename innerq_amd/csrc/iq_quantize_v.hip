@@ -6,6 +6,21 @@ int iq::detail::quantize_v_f16(const VArgs& a, const QuantOut& o, int group, int
   return launch_quant_v<false>(a, o, group, bits, mode, dense, st);
 }
 
+namespace {
+
+// Values up to which a call goes by a lane per value (groups of 32 or 64, asym
+// or sym): a thread's chain over its 32 tokens and two columns bounds a short
+// call, whose lanes are few.  8 heads x 128 columns, us a launch in a graph,
+// lanes / threads: 128 tokens (2^17) bf16 to a store 3.3 / 3.9 (G = 32 asym), 3.2
+// / 3.5 (sym), 3.9 / 5.2 (G = 64), fp16 3.2 / 3.2, 3.1 / 3.3, 3.8 / 4.0; 256
+// tokens bf16 4.1 / 4.0, 3.9 / 3.6, 4.8 / 5.3, fp16 3.9 / 3.3, 3.8 / 3.3, 4.6 /
+// 4.0.  With quant.py's outputs the threads store more: 256 tokens bf16 4.4 /
+// 4.7, 4.7 / 5.9, 5.6 / 6.8, fp16 4.2 / 4.5, 4.7 / 5.2, 5.5 / 6.4; 512 tokens
+// 6.3 / 4.9, 6.7 / 6.0, 8.1 / 6.9, fp16 6.0 / 4.6, 6.4 / 5.4, 7.9 / 6.5.
+int64_t lane_values(int group, bool bf, bool dense) { return dense || (bf && group == 64) ? 1 << 18 : 1 << 17; }
+
+}  // namespace
+
 extern "C" {
 
 int iq_quantize_v(const void* x, int64_t sx_b, int64_t sx_h, int64_t sx_t, int B, int H, int n, int D,
@@ -35,6 +50,8 @@ int iq_quantize_v(const void* x, int64_t sx_b, int64_t sx_h, int64_t sx_t, int B
   const detail::VArgs a{(const uint16_t*)x, sx_b, sx_h, sx_t, H, n, D, dp,
           D % 2 == 0 && aligned(x, 4) && sx_b % 2 == 0 && sx_h % 2 == 0 && sx_t % 2 == 0,
           int64_t(B) * H * (n / group) * dp};
+  if (group <= 64 && mode != IQ_MODE_HYBRID && int64_t(B) * H * n * D <= lane_values(group, bf, dense))
+    return detail::quantize_v_lanes(a, o, int64_t(B) * H, group, bits, mode, bf, (hipStream_t)stream);
   return bf ? detail::quantize_v_bf16(a, o, group, bits, mode, dense, (hipStream_t)stream)
             : detail::quantize_v_f16(a, o, group, bits, mode, dense, (hipStream_t)stream);
 }

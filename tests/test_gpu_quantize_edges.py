@@ -130,6 +130,10 @@ def test_values(act, mode, widths, groups, D, G, off, layout):
         assert same_meta(gm, meta, act)
 
 
+def same_bits(a, b):
+    return torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))
+
+
 @pytest.mark.parametrize("act", ["f16", "bf16"])
 @pytest.mark.parametrize("bits,mode,D,G,norm", [(4, "asymmetric", 128, 32, False), (3, "symmetric", 96, 32, True),
                                                 (2, "hybrid", 64, 64, True), (1, "asymmetric", 384, 128, False)])
@@ -147,6 +151,29 @@ def test_long_key_calls_equal_short_ones(act, bits, mode, D, G, norm, rows):
         parts.append(x[:, :, t:t + 100], norm=nf)
     for a, b in zip(token_rows(whole), token_rows(parts)):
         assert torch.equal(a[:, :n], b[:, :n]) and int((a[:, n:] != 0).sum()) == 0
+
+
+@pytest.mark.parametrize("act", ["f16", "bf16"])
+@pytest.mark.parametrize("bits,mode", [(4, "asymmetric"), (2, "asymmetric"), (3, "symmetric")])
+@pytest.mark.parametrize("D,G,groups", [(130, 32, 12), (33, 32, 42), (128, 64, 6), (33, 64, 21), (128, 32, 6), (128, 64, 3),
+                                        (128, 32, 11)])
+def test_long_value_calls_equal_short_ones(act, bits, mode, D, G, groups):
+    """Short calls go by a lane per value (up to 2^17 or 2^18 values), longer ones by a thread per token group
+    and column pair: calls on either side of the lines hold the bytes of calls of one group, stores and
+    quant.py's outputs."""
+    B, H, n = 2, 3, groups * G
+    x = planted(B, H, n, D, bits, act).to(DEV)
+    whole, parts = (ops.PackedStore("token", B, H, D, G, bits, mode, DEV, dtype=TD[act]) for _ in range(2))
+    whole.append(x)
+    dense = []
+    for t in range(0, n, G):
+        parts.append(x[:, :, t:t + G])
+        dense.append(ops.quantize_dense(x[:, :, t:t + G].contiguous(), G, bits, mode, "token"))
+    for a, b in ((whole.codes, parts.codes), (whole.meta, parts.meta)):
+        m = whole.t_cap // G, parts.t_cap // G
+        assert torch.equal(a.view(B * H, m[0], -1)[:, :groups], b.view(B * H, m[1], -1)[:, :groups])
+    for a, b in zip(ops.quantize_dense(x, G, bits, mode, "token"), zip(*dense)):
+        assert same_bits(a, torch.cat(b, dim=2))
 
 
 @pytest.fixture
