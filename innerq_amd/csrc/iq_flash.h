@@ -849,7 +849,7 @@ int fused_launch_mixed(const FusedArgs& a, int vbits, int group, int D, int nrep
       const int nt = norm ? FusedShape<G, R, true>::NT : FusedShape<G, R, false>::NT;
       static detail::OccCache occ[2];
       const int pc = detail::blocks_per_cu(kern, nt, occ[norm ? 1 : 0]);
-      const int grid = int(std::min<int64_t>(a.nitems, int64_t(pc) * detail::num_cus()));
+      const int grid = detail::fused_workgroups(pc, a.nitems, nt / 64, FusedShape<G, R, true>::WTOK * DD * (KB + VB) / 8);
       if (grid_out) *grid_out = grid;
       if (!launch) return int(IQ_OK);
       kern<<<dim3(grid), nt, 0, stream>>>(detail::fused_grid(a, grid));
@@ -882,10 +882,9 @@ int fused_launch_kb(const FusedArgs& a, int vbits, int group, int D, int nrep, b
     }
     const bool qs = BF || norm;
     const int nt = qs ? FusedShape<G, R, true>::NT : FusedShape<G, R, false>::NT;
-    // as many workgroups as fit at once on the device (per instance)
-    static detail::OccCache occ[6];
+    static detail::OccCache occ[6];  // workgroups per CU at once
     const int pc = detail::blocks_per_cu(kern, nt, occ[(qs ? 1 : 0) + 2 * sm]);
-    const int grid = int(std::min<int64_t>(a.nitems, int64_t(pc) * detail::num_cus()));
+    const int grid = detail::fused_workgroups(pc, a.nitems, nt / 64, FusedShape<G, R, true>::WTOK * DD * (KB + VB) / 8);
     if (grid_out) *grid_out = grid;
     if (!launch) return int(IQ_OK);
     kern<<<dim3(grid), nt, 0, stream>>>(detail::fused_grid(a, grid));

@@ -98,4 +98,25 @@ int flash_fused_launch(const void* q, int64_t sq_b, int64_t sq_h, const void* no
   }
 }
 
+// One workgroup per CU, also where registers would let two on it: two halve a
+// workgroup's share and double a head's runs, which the combine or the merging
+// window kernel read.  (The register counts lie around the line of 128, so a
+// rule by occupancy alone changes sides with any edit: 4-bit K and V, one query
+// head per KV head, 133 -> 127 registers: B = 4, 4000 tokens 10.3 -> 11.8 us a
+// call, B = 8, 32768 tokens 58.3 -> 63.3.)  Two where a workgroup alone has too
+// few bytes in flight for the memory's latency and the shares are long: up to
+// 32 KB from 20 splits per CU on, one / two (8 KV heads, B = 8, 24000 tokens): 2-bit
+// K and V, one head 31.1 / 28.9, at D = 64 23.2 / 21.5 (at 16 splits per CU 23.6 /
+// 23.2, 17.9 / 17.6, and with a window 27.0 / 28.9, 20.8 / 22.0); 40-64 KB 36.2 / 34.9
+// to 34.6 / 34.7 and, at 32768 tokens, 58.0 / 63.3.  Workgroups of one wave per
+// SIMD (groups of 128), whose waves nothing else covers: up to 48 KB from 6
+// splits per CU on: 2-bit, eight heads, 8000 tokens 22.6 / 21.7, 32768 56.9 / 50.1;
+// 2-bit K and 4-bit V 27.4 / 26.0, 70.5 / 68.4; 4-bit K and V (64 KB), four heads, 32768
+// 87.0 / 92.9.
+int fused_workgroups(int pc, int64_t nitems, int waves, int block_bytes) {
+  const bool thin = waves <= 4;  // one wave per SIMD
+  const bool two = waves * block_bytes <= (thin ? 48 : 32) * 1024 && nitems >= int64_t(thin ? 6 : 20) * num_cus();
+  return int(std::min<int64_t>(nitems, int64_t(two ? pc : 1) * num_cus()));
+}
+
 }  // namespace iq::detail

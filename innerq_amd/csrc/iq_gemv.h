@@ -617,6 +617,10 @@ size_t av_part_bytes(int B, int Hq, int T, int D, int group);
 constexpr int MAX_DEVICES = 64;
 int device_index();
 int num_cus();
+// Workgroups of a fused launch over nitems splits, by a kernel that fits pc
+// times on a CU, in workgroups of `waves` that each have a wave block of
+// block_bytes of codes in flight (iq_flash.hip)
+int fused_workgroups(int pc, int64_t nitems, int waves, int block_bytes);
 // workgroups of `kern` (nt threads) resident per CU at once on the current
 // device, queried once per device and kernel (`cache`: one per kernel)
 struct OccCache {
