@@ -33,15 +33,24 @@ constexpr int NSD_MAX = 4;    // split slots of the dense tokens, at most
 constexpr int DSLICE = 32;    // dense tokens per split slot, at least
 // Fused runs per (batch, KV head) that the merging dense kernel takes: the
 // first MERGE_PRE of them are loaded with the window's rows, the next beside
-// the sections' last barrier, the rest MERGE_PRE at a time.  Up to four query
-// heads per KV head, fp16: 16 runs (4-bit, 8 KV heads of 4 query heads, 8192
-// tokens and a 128-token window, a call: B = 4, 8 runs, 21.2 us with the dense
-// slices and the combine, 19.4 merged; B = 2, 16 runs, 18.4 and 18.1; past 16
-// they measure the same).  Eight query heads per KV head and bf16 layers, whose
-// window takes longer in two sections than in four slices: 4 runs (8 runs of
-// eight bf16 query heads: 24.7 us with the slices, 27.9 merged).
-constexpr int MERGE_RUNS_MAX = 16, MERGE_PRE = 4;
-constexpr int merge_runs_max(bool bf, int nrep) { return bf || nrep > 4 ? MERGE_PRE : MERGE_RUNS_MAX; }
+// the sections' last barrier, the rest MERGE_PRE at a time.  MERGE_RUNS_MAX in
+// fp16 with up to four query heads per KV head, where the window is one chunk
+// per section (one head, whose slices are short: two chunks in all); else
+// MERGE_PRE.  Us a call in a graph, slices and combine / merged, 8 KV heads,
+// 4-bit K and V of 16000 tokens: a 128-token window, B = 4 (8 runs) four heads 26.4
+// / 24.4, two 25.6 / 24.0, one 23.7 / 22.5; B = 3 (11 runs) 23.9 / 22.4, 22.7 / 21.9,
+// 20.6 / 19.8; B = 2 (16 runs) over 4000 tokens 3-bit / 2-bit, four heads 15.3 /
+// 16.3, two 14.5 / 15.2.  250 tokens, two chunks: B = 4 26.5 / 28.0, 25.9 / 27.3;
+// 185 tokens, one head, B = 3 21.3 / 21.5.  Eight heads and bf16 layers, whose
+// window takes longer in two sections than in four slices: 8 runs of eight
+// bf16 query heads 24.7 / 27.9.
+constexpr int MERGE_RUNS_MAX = 12, MERGE_PRE = 4;
+constexpr int merge_runs_max(bool pk, bool bf, int nrep) {  // of an instance
+  return pk || bf || nrep > 4 ? MERGE_PRE : MERGE_RUNS_MAX;
+}
+constexpr int merge_runs(bool pk, bool bf, int nrep, int n_dense) {  // of a call
+  return n_dense <= (nrep == 1 ? 2 : 3) * DT ? merge_runs_max(pk, bf, nrep) : MERGE_PRE;
+}
 // 256-thread sections of the merging dense kernel: three where the window
 // holds packed rows (32 sinks, a 96-token recent window and the <= 31 packed
 // keys short of a V group, 129-159 tokens that two sections take in two
@@ -613,8 +622,8 @@ __global__ __launch_bounds__(MERGE ? 256 * NS : 256) void dense_attn_kernel(Dens
     // instance of at most MERGE_PRE runs holds no code for more and reads all
     // of them at once: as loops over up to 16, B = 10, 8 KV heads, 967 tokens,
     // a 151-token window, bf16, kernel / call in us: 2 query heads per KV head
-    // 14.1 / 21.3, 4 heads 15.0 / 22.9; so 13.8 / 21.1 and 14.4 / 22.5.
-    constexpr int RM = merge_runs_max(BF, NREP);
+    // 14.1 / 21.3, 4 heads 15.0 / 22.9; now 13.8 / 21.1 and 14.4 / 22.5.
+    constexpr int RM = merge_runs_max(PK, BF, NREP);
     __shared__ float2 rml[RM][NREP];
     static_assert(RM * NREP <= NTH, "one thread per run and head");
     float po2[RM > MERGE_PRE ? EPT : 1][MERGE_PRE];
@@ -1081,7 +1090,8 @@ int launch_splits(const void* q, int64_t sq_b, int64_t sq_h, const void* norm, c
     bool merge_dense = merge_cand;
     if (merge_cand) {
       const detail::ShareMap sm = detail::ShareMap::make(grid, int(bhs), nsf, plan->pair_e0);
-      for (int h = 0; h < int(bhs) && merge_dense; ++h) merge_dense = sm.nruns(h) <= merge_runs_max(bf, Hq / Hkv);
+      const int runs_max = merge_runs(pk, bf, Hq / Hkv, n_dense);
+      for (int h = 0; h < int(bhs) && merge_dense; ++h) merge_dense = sm.nruns(h) <= runs_max;
       if (!merge_dense)
         if (int e = launch_slices()) return e;
     }

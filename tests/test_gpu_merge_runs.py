@@ -1,6 +1,6 @@
 """Decode steps whose window is merged with 1 to 20 fused runs per KV head: the merging dense kernel takes
-up to 16 (4 for eight query heads per KV head and bf16 layers), the slices and the combine the rest;
-counts around its rounds of four.  Against the float64 oracle within the decode's 1e-3 of max|ref|."""
+up to 12 (4 for eight query heads per KV head, bf16 layers, windows past 192 tokens (one head: 128) and
+windows with packed rows), the slices and the combine the rest; counts around its rounds of four.  Against the float64 oracle within the decode's 1e-3 of max|ref|."""
 import pytest
 import torch
 
@@ -16,6 +16,21 @@ pytestmark = pytest.mark.gpu
 def test_runs_per_head(runs, nrep, D):
     seg = (0, 256 * runs, 70)
     assert _decode_case(1, 2, nrep, D, seg, seg, (4, 32, "asymmetric"), (4, 32, "asymmetric"), seed=runs) < TOL
+
+
+@pytest.mark.parametrize("runs", [4, 5, 12, 13])
+@pytest.mark.parametrize("nrep,win", [(2, 1), (2, 192), (2, 193), (2, 256), (2, 257), (1, 128), (1, 129)])
+def test_window_lengths(runs, nrep, win):
+    """Windows of one chunk per section, of two, and past what is merged."""
+    seg = (0, 256 * runs, win)
+    assert _decode_case(1, 2, nrep, 128, seg, seg, (4, 32, "asymmetric"), (4, 32, "asymmetric"), seed=win) < TOL
+
+
+@pytest.mark.parametrize("runs", [4, 5, 12])
+def test_windows_with_packed_rows(runs):
+    """K packed 32 tokens further than V: those rows are read packed in the window."""
+    k, v = (0, 256 * runs + 32, 70), (0, 256 * runs, 102)
+    assert _decode_case(1, 2, 4, 128, k, v, (4, 32, "asymmetric"), (4, 32, "asymmetric"), seed=runs) < TOL
 
 
 @pytest.mark.parametrize("runs", [4, 5, 9])
