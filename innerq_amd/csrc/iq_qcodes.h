@@ -2,9 +2,9 @@
 // every op of the reference is an fp32 op rounded to the activation dtype
 // (fp16, or bf16 with bf), the clamp keeps NaN, the rounding is half-to-even
 // and a NaN code is INT32_MIN in dense outputs, 0 (asym) or the offset (sym)
-// in packed fields.  The prompt quantizers (iq_quantize.hip) use these forms
-// for groups that hold NaN or infinity, the window append (iq_quant.hip) for
-// every group.
+// in packed fields.  The prompt quantizers (iq_quantize.h) use these forms for
+// groups that hold NaN or infinity, the lane-per-value quantizers of
+// iq_quant.hip (the window append, short calls of values) for every group.
 #pragma once
 #include "iq_common.h"
 #include "iq_device.h"

@@ -1,8 +1,10 @@
-// A decode step's window append, dense dequantization and unpacking (gfx950).
+// A decode step's window append, short calls of the value quantizer, dense
+// dequantization and unpacking (gfx950).
 //
 // The append quantizes a few hundred groups per step with the reference's own
-// per-value arithmetic (iq_qcodes.h); prompts go through iq_quantize_k.hip and
-// iq_quantize_v.h, whose results are the same bits.
+// per-value arithmetic (iq_qcodes.h), as short calls of values are; prompts go
+// through iq_quantize_k.hip and iq_quantize_v.h, whose results are the same
+// bits.
 #include "iq_common.h"
 #include "iq_device.h"
 #include "iq_qcodes.h"
